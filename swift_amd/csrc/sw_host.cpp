@@ -485,6 +485,14 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     // at most pos per cell, so a pair with any larger cell has one in
     // [2048 - pos, 2047] whose key is exact.
     uint32_t h_limit = (uint32_t)std::min(32767 - (4 * pos + 3) - 4, 4 * (2048 - pos));
+    // The lean sweeps: with their lower limit the same holds for keys 32H + 31
+    // + 32 * match below 0x7C00 (match <= 30).  Taken where no pair within
+    // maxq reaches it (larger scores would be re-run in int32 lanes); 32-bit
+    // lanes have no such limit.
+    const bool lean32 = lean_scoring(sc);
+    const uint32_t lean_limit = 4u * (uint32_t)(kLeanScoreLimit - 2 * pos);
+    const bool lean16 = lean32 && (int64_t)io.maxq * pos * 4 < (int64_t)lean_limit;
+    if (lean16) h_limit = lean_limit;
 
     // one launch zeroes the results (they start at "score 0": a pair no
     // kernel reaches never walks), the error flag, the flagged count, the
@@ -577,7 +585,7 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     BatchArgs ba{io.qseq, io.qoff, io.qlen, io.rseq, io.roff, io.rlen, w.order.as<int32_t>(),
                  w.tasks.as<Task>(), nullptr, nullptr, nullptr, w.trace.as<uint32_t>(),
                  w.res.as<PairResult>(), w.ptr.as<PairTrace>(), kc16, h_limit,
-                 io.score, io.start, io.end, io.alen, io.qcons, io.rcons, io.cons_off,
+                 io.score, io.start, io.end, io.alen, io.qcons, io.rcons, io.cons_off, 0,
                  tuning().walk_deferred, cnt + kCntFlagged};
     // One persistent kernel per (class, R) segment, each reading its task
     // range from the device (empty segments exit at once), spread over the
@@ -643,6 +651,7 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
             b.task_hi = t.seg_task0 + seg + 1;
             b.next_task = cnt + kCntQueues + pass * kQueuesPerPass + seg;
             b.kc = cls == 0 ? kc16 : kc32;
+            b.lean = cls == 0 ? lean16 : lean32;
             hipStream_t s2 = nside ? w.side[lane_of[seg]] : st;
             const int wpc = w.waves_per_cu >= 0 ? w.waves_per_cu : tuning().waves_per_cu;
             const bool wseg = t.wide && seg == 0;

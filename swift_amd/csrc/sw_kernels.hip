@@ -296,6 +296,189 @@ struct Sweep {
 };
 
 // ---------------------------------------------------------------------------
+// The lean sweep, for the scorings of lean_scoring: the same staggered
+// recurrence, keys and trace codes as Sweep in fewer and cheaper
+// instructions.
+//
+// What bounds a sweep is VALU issue.  Measured issue cost a wave (cycles per
+// SIMD): and/or/xor/add/sub and mov 2.3-2.5, everything else used here (packed
+// 16-bit, 3-operand, v_perm, shifts, max) 4.2-4.5.  A row of two packed cells
+// costs Sweep 15 instructions and about 57 cycles, this one 12.3 and 47:
+//  * A cell's key is one v_pk_maximum3_f16 (v_max3_u32 in 32-bit lanes) of its
+//    three candidates.  Every candidate is kept >= 0 by saturating subtracts,
+//    which makes the zero candidate implicit, and non-negative keys below
+//    0x7C00 order as half-precision bit patterns exactly as integers do.
+//  * Exits are key - penalty[direction], the penalty a byte picked by
+//    v_perm_b32 with the direction code itself as selector: the selector's
+//    zero bytes pick entry 0, which is 0 (a start's key is 0, so what is
+//    subtracted from it does not matter).
+//  * The match test's v_perm_b32 yields the mismatch penalty (0 or pm), so the
+//    diagonal candidate is one saturating subtract from x = 4H + 4*match + 3.
+//  * The best cell is kept per lane, not per row: each step's maximum over
+//    the rows of 32H + row code (smaller rows larger codes), and the first
+//    step at which it rose.  That is the lane's first maximum in row-major
+//    order, in 2 registers instead of 2R, which also lets another wave of the
+//    larger classes onto a SIMD.
+//  * Four steps a loop turn: their columns read together, their trace words
+//    stored 16 bytes a lane.
+// Sweep kernels before and after: 1.0M pairs of 150 x 300 (R = 10) 11.8 ->
+// 9.4 ms, 439k of 100 x 300 (R = 7) 3.89 -> 3.05 ms, 64 pairs up to 300 x 480
+// in the wide form 137 -> 79 us.
+// No step is masked: cells left of column 1 keep H = 0; cells right of a
+// pair's last column and rows below its query never match (padding
+// selectors, bit 7 of a padding row's table), so they score strictly below
+// the pair's best cell.
+// ---------------------------------------------------------------------------
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+
+template <bool PK> __device__ __forceinline__ uint32_t vmax3(uint32_t a, uint32_t b, uint32_t c) {
+    if constexpr (PK) {
+        const v2h x = __builtin_bit_cast(v2h, a), y = __builtin_bit_cast(v2h, b),
+                  z = __builtin_bit_cast(v2h, c);
+        return __builtin_bit_cast(
+            uint32_t, __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, y), z));
+    } else {
+        return max(max(a, b), c);
+    }
+}
+template <bool PK> __device__ __forceinline__ uint32_t vsub_sat(uint32_t a, uint32_t b) {
+    if constexpr (PK) return as_u(__builtin_elementwise_sub_sat(as_us(a), as_us(b)));
+    else return __builtin_elementwise_sub_sat(a, b);
+}
+
+// 32-bit lanes compare bytes in dual-rail code: bits 14..21 the byte, bits
+// 22..29 its complement on the query side, swapped on the reference side, so
+// q & r is zero exactly where the bytes are equal; N has neither (the
+// wildcard).  Bit 30: set in every query row and in padding columns; bit 31:
+// set in padding rows and in every column.  A non-zero q & r is >= 2^14,
+// above every mismatch penalty.
+__device__ __forceinline__ uint32_t rail_query(uint32_t c, bool pad_row) {
+    const uint32_t rails = c == 'N' ? 0u : c | (~c & 0xFFu) << 8;
+    return (rails << 14) | (1u << 30) | (pad_row ? 1u << 31 : 0u);
+}
+__device__ __forceinline__ uint32_t rail_ref(uint32_t c, bool pad_col) {
+    const uint32_t u = (uint32_t)upper_byte((int)c) & 0xFFu;
+    const uint32_t rails = u == 'N' ? 0u : (~u & 0xFFu) | u << 8;
+    return (rails << 14) | (1u << 31) | (pad_col ? 1u << 30 : 0u);
+}
+// Packed lanes: a row's match table (a byte per class A C G T: 0 where the
+// query byte matches, else the mismatch penalty; 0xFF throughout in padding
+// rows) and a column's selector, low byte: its class; N the sign of table
+// byte 1, 0xFF in padding rows and 0 else; padding and other bytes 0xFF.  The
+// high byte selects 0.
+__device__ __forceinline__ uint32_t lean_table(uint32_t c, bool pad_row, uint32_t pm) {
+    if (pad_row) return 0xFFFFFFFFu;
+    return ~query_table(query_mask_bf((unsigned char)c)) & (pm * 0x01010101u);
+}
+__device__ __forceinline__ uint32_t lean_selector(uint32_t cls, int half) {
+    const uint32_t s = cls < 4 ? cls + 4u * (uint32_t)half : cls == 4 ? 8u + 2u * (uint32_t)half : 13u;
+    return s | 0x0C00u;
+}
+
+template <int G, int R, bool PK>
+struct Lean {
+    static constexpr int KPW = PK ? 8 : 16;          // rows per trace word
+    static constexpr int W = (R + KPW - 1) / KPW;     // trace words per step
+    static constexpr uint32_t CMASK = PK ? 0x00030003u : 3u;
+    static constexpr int CTRL = G == 16 ? kRowShr1 : kWaveShr1;
+    // row r = block * B + k: codes 3 - block (2 bits), B - 1 - k (3 bits)
+    static constexpr int B = (R + 3) / 4;
+    static_assert(B <= 8, "row codes");
+
+    uint32_t q[R];             // PK: match tables of half 0; else dual-rail bytes
+    uint32_t q2[PK ? R : 1];   // PK: match tables of half 1
+    uint32_t x[R];             // 4H + 4*match + 3 of (row, j-1)
+    uint32_t el[R];            // left exit of (row, j-1)
+    uint32_t x_top, eu_last;
+    uint32_t best, tbest;      // best key and the step of its first cell
+    uint32_t c_x, c_sign, tab_u, tab_l, pm;
+
+    __device__ __forceinline__ void init(const KeyConsts &k) {
+        c_x = splat<PK>(k.x);
+        c_sign = splat<PK>(k.sign);
+        tab_u = k.tab_u;
+        tab_l = k.tab_l;
+        pm = (uint32_t)k.pm;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            x[r] = c_x;  // column 0: H = 0, start
+            el[r] = 0;
+        }
+        x_top = c_x;
+        eu_last = 0;
+        best = 8u * (c_x - splat<PK>(3)) + splat<PK>(31);  // H = 0 at any row
+        tbest = 0;
+    }
+
+    // One step on the reference code(s) rr of column t - g; tcode: t in every
+    // element.
+    __device__ __forceinline__ void step(uint32_t rr, uint32_t tcode, uint32_t *acc) {
+        // from the lane above (0 into a group's first lane, whose matrix row 0
+        // has H = 0: x = c_x, no up exit)
+        const uint32_t eu_in =
+            (uint32_t)__builtin_amdgcn_update_dpp(0, (int)eu_last, CTRL, 0xF, 0xF, true);
+        const uint32_t x_in = max(
+            (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x[R - 1], CTRL, 0xF, 0xF, true), c_x);
+        uint32_t diag[R];
+#pragma unroll
+        for (int r = R - 1; r >= 0; --r) {
+            const uint32_t pen = PK ? __builtin_amdgcn_perm(q2[PK ? r : 0], q[r], rr)
+                                    : min(q[r] & rr, pm);
+            diag[r] = vsub_sat<PK>(r ? x[r - 1] : x_top, pen);
+        }
+        x_top = x_in;
+        uint32_t eu = eu_in;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t K = vmax3<PK>(diag[r], el[r], eu);
+            const uint32_t c = K & CMASK;
+            acc[r / KPW] |= c << (2 * (r % KPW));
+            eu = vsub_sat<PK>(K, __builtin_amdgcn_perm(tab_u, tab_u, c));
+            el[r] = vsub_sat<PK>(K, __builtin_amdgcn_perm(tab_l, tab_l, c));
+            x[r] = (K & ~CMASK) + c_x;  // no half carries into the other
+        }
+        eu_last = eu;
+        // the step's best key: rows of one k by block, then over k
+        uint32_t kb[B];
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            uint32_t v[4];
+            int n = 0;
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                if (b * B + k < R) v[n++] = x[b * B + k] - splat<PK>(b);
+            uint32_t m = v[0];
+            if (n == 2) m = vmax<PK>(m, v[1]);
+            if (n >= 3) m = vmax3<PK>(m, v[1], v[2]);
+            if (n == 4) m = vmax<PK>(m, v[3]);
+            if constexpr (PK) kb[k] = vmad<true>(m, splat<true>(8), splat<true>(B - 1 - k));
+            else kb[k] = (m << 3) + (uint32_t)(B - 1 - k);
+        }
+        uint32_t m = kb[0];
+#pragma unroll
+        for (int k = 1; k + 1 < B; k += 2) m = vmax3<PK>(m, kb[k], kb[k + 1]);
+        if constexpr (B % 2 == 0) m = vmax<PK>(m, kb[B - 1]);
+        if constexpr (PK) {
+            const uint32_t up = as_u(as_s(vsub<true>(best, m)) >> as_s(c_sign));
+            tbest = (up & tcode) | (~up & tbest);
+            best = vmax<true>(best, m);
+        } else {
+            tbest = m > best ? tcode : tbest;
+            best = max(best, m);
+        }
+    }
+
+    // best cell of the lane: H, its row within the lane (0-based), its step
+    __device__ __forceinline__ void result(int half, uint32_t &h, int &r, int &t) const {
+        const uint32_t s = 16u * (uint32_t)half, m = PK ? 0xFFFFu : ~0u;
+        const uint32_t k = ((best >> s) & m) - 8u * (((c_x >> s) & m) - 3u);
+        h = k >> 5;
+        r = (int)(3u - ((k >> 3) & 3u)) * B + B - 1 - (int)(k & 7u);
+        t = (int)((tbest >> s) & m);
+    }
+};
+
+// ---------------------------------------------------------------------------
 // Result of a lane group: per lane, best (H, row, col) over its valid rows,
 // then a group-wide max of (H desc, row asc) -- the reference's first strict
 // maximum in row-major order.  Every lane of the group receives the result.
@@ -583,25 +766,27 @@ sw_plain_kernel(const char *__restrict__ qseq, const char *__restrict__ rseq, in
 // ---------------------------------------------------------------------------
 // Batched persistent kernels.
 // ---------------------------------------------------------------------------
-// LDS words per lane group of G lanes: G zero columns before column 0, the
-// reference columns, and G columns of tail
-template <int G>
-constexpr int group_lds_words() { return G + kBatchCols + G; }
+// LDS words per wave: each of the 64 / G groups has its reference columns and
+// a tail of G + 2 padding columns (the lanes run up to G - 1 columns past the
+// last, and steps are rounded up to whole granules of 4); the G columns before
+// a group's column 0 are the end of the tail before it, or the wave's first G
+// words; 4 words past the end are read ahead.  31.2 KB a workgroup of the
+// 16-lane kernels: five of them fit a CU.
+template <int G> constexpr int group_lds_stride() { return kBatchCols + G + 2; }
+template <int G> constexpr int wave_lds_words() { return G + 64 / G * group_lds_stride<G>() + 4; }
 
 // One wave task: 64 / G groups of G lanes (G = 16: 4 groups; G = 64, the
 // wide form: one); PK -> 2 pairs per group (halves).
-template <int G, int R, bool PK, int POL>
+template <int G, int R, bool PK, bool LEAN>
 __device__ __forceinline__ void run_task(const BatchArgs &a, const Task &tk, uint32_t *lds) {
-    using S = Sweep<G, R, PK, POL>;
+    using S = std::conditional_t<LEAN, Lean<G, R, PK>, Sweep<G, R, PK, PK ? kOneHot : kBytes>>;
     constexpr int PPG = PK ? 2 : 1;  // pairs per group
     constexpr int NG = 64 / G;       // groups per wave
-    constexpr int PAD = G;           // zero columns before column 0
-    constexpr int GL = group_lds_words<G>();
+    constexpr int TAIL = G + 2;      // padding columns after the last
     const int lane = threadIdx.x & 63;
     const int grp = lane / G, g = lane % G;
-    // reference codes at [PAD + j]; the PAD leading entries and the tail
-    // are read by lanes outside the pair's columns (their results unused)
-    uint32_t *rr_lds = lds + grp * GL;
+    // reference codes at [j], -G <= j < columns + TAIL
+    uint32_t *rr_lds = lds + G + grp * group_lds_stride<G>();
 
     // the group's pairs.  The loads are unconditional (a slot past the
     // task's pairs reads its first pair and is then cleared; byte loads are
@@ -655,7 +840,13 @@ __device__ __forceinline__ void run_task(const BatchArgs &a, const Task &tk, uin
     const int ncols = tk.steps - (G - 1);
     constexpr int NB = 8;
     uint32_t exotic = 0;  // bit h: the pair's reference holds a byte outside ACGTNacgtn
-    for (int j0 = g; j0 < ncols + G; j0 += NB * G) {
+    auto ref_word = [](uint32_t cls_or_byte, bool pad, int half) -> uint32_t {
+        if constexpr (!PK) return LEAN ? rail_ref(cls_or_byte, pad) : pad ? 0u : byte_rcode((unsigned char)cls_or_byte);
+        else return LEAN ? lean_selector(cls_or_byte, half) : column_selector(cls_or_byte, half);
+    };
+    const uint32_t pad_word = PK ? ref_word(kRefPad, true, 0) | ref_word(kRefPad, true, 1) << 16
+                                 : ref_word(0, true, 0);
+    for (int j0 = g; j0 < ncols + TAIL; j0 += NB * G) {
         unsigned char cb[NB][PPG];
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
@@ -667,19 +858,19 @@ __device__ __forceinline__ void run_task(const BatchArgs &a, const Task &tk, uin
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
             const int j = j0 + i * G;
-            if (j < ncols + G) {
+            if (j < ncols + TAIL) {
                 uint32_t v = 0;
 #pragma unroll
                 for (int h = 0; h < PPG; ++h) {
-                    uint32_t code = PK ? kRefPad : 0u;
-                    if (j < rl[h]) {
-                        code = PK ? ref_index_bf(cb[i][h]) : byte_rcode(cb[i][h]);
-                        if (PK && code == kRefOther) exotic |= 1u << h;
+                    const bool pad = j >= rl[h];
+                    uint32_t code = cb[i][h];
+                    if constexpr (PK) {
+                        code = pad ? kRefPad : ref_index_bf(cb[i][h]);
+                        if (code == kRefOther) exotic |= 1u << h;
                     }
-                    if constexpr (PK) code = column_selector(code, h);
-                    v |= code << (16 * h);
+                    v |= ref_word(code, pad, h) << (16 * h);
                 }
-                rr_lds[PAD + j] = v;
+                rr_lds[j] = v;
             }
         }
     }
@@ -687,15 +878,20 @@ __device__ __forceinline__ void run_task(const BatchArgs &a, const Task &tk, uin
 #pragma unroll
         for (int s2 = G / 2; s2 >= 1; s2 >>= 1) exotic |= __shfl_xor(exotic, s2, G);
     }
-    if (g < PAD)
-        rr_lds[g] = PK ? column_selector(kRefPad, 0) | column_selector(kRefPad, 1) << 16 : 0u;
+    // the G columns before column 0: the wave's first words, and the end of
+    // each group's tail
+    if (grp == 0) rr_lds[g - G] = pad_word;
+    rr_lds[kBatchCols + 2 + g] = pad_word;
     sw.init(a.kc);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         // 256: a row past the query (no match anywhere)
-        auto conv = [](uint32_t c) -> uint32_t {
-            return c > 255u ? 0u : PK ? query_table(query_mask_bf((unsigned char)c))
-                                      : byte_qcode((unsigned char)c);
+        auto conv = [&](uint32_t c) -> uint32_t {
+            if constexpr (LEAN)
+                return PK ? lean_table(c, c > 255u, (uint32_t)a.kc.pm) : rail_query(c & 255u, c > 255u);
+            else
+                return c > 255u ? 0u : PK ? query_table(query_mask_bf((unsigned char)c))
+                                          : byte_qcode((unsigned char)c);
         };
         sw.q[r] = conv(sw.q[r]);
         if constexpr (PK) sw.q2[r] = conv(sw.q2[r]);
@@ -704,62 +900,101 @@ __device__ __forceinline__ void run_task(const BatchArgs &a, const Task &tk, uin
     __builtin_amdgcn_s_waitcnt(0);  // LDS writes of this wave visible to its lanes
     __builtin_amdgcn_wave_barrier();
 
-    uint32_t *tr = a.trace + tk.trace_base;
-    uint32_t rr_next = rr_lds[PAD - g];  // column of step 0
-    auto run = [&](auto masked, int t) {
-        int j = t - g;
-        uint32_t rr = rr_next;
-        // prefetch the next step's column (clamped: steps past the last
-        // granule boundary read a stale word whose results are unused)
-        rr_next = rr_lds[min(PAD + 1 + j, GL - 1)];
-        uint32_t vmask = 0;
-        if constexpr (decltype(masked)::value) {
-#pragma unroll
-            for (int h = 0; h < PPG; ++h)
-                if (j >= 0 && j < rl[h]) vmask |= (PK ? 0xFFFFu : 0xFFFFFFFFu) << (16 * h);
-        }
-        uint32_t a1[S::W];
-#pragma unroll
-        for (int w = 0; w < S::W; ++w) a1[w] = 0;
-        sw.template step<decltype(masked)::value>(rr, j, vmask, splat<PK>(15 - (t & 15)), a1);
-#pragma unroll
-        for (int w = 0; w < S::W; ++w) tr[trace_word<S::W>(t, w, lane)] = a1[w];
-    };
-    // int32: masked steps keep the cells outside a pair's columns out of its
-    // row maxima.  Packed: no step is masked (see Sweep).
     const int T = tk.steps;
-    if constexpr (PK) {
-        for (int t = 0; t < T; ++t) {
-            run(std::false_type{}, t);
-            if ((t & 15) == 15 || t == T - 1) sw.block_end(splat<true>((t >> 4) << 5));
+    if constexpr (LEAN) {
+        // granules of 4 steps: their columns are read during the granule
+        // before, their trace words stored 16 bytes a lane and word.  (Global
+        // stores: a 16-byte buffer store with its offset in a scalar register
+        // was seen to lose data to a 2-cycle instruction overwriting its
+        // source right after it; the compiler keeps only the other forms of
+        // wide stores apart from such writes.)
+        typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+        v4u *tr = reinterpret_cast<v4u *>(a.trace + tk.trace_base);
+        const uint32_t *col = rr_lds - g;
+        uint32_t nx[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) nx[u] = col[u];
+        for (int t = 0; t < T; t += 4) {
+            uint32_t cur[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                cur[u] = nx[u];
+                nx[u] = col[t + 4 + u];
+            }
+            uint32_t acc[4][S::W];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+#pragma unroll
+                for (int w = 0; w < S::W; ++w) acc[u][w] = 0;
+                sw.step(cur[u], splat<PK>(t + u), acc[u]);
+            }
+#pragma unroll
+            for (int w = 0; w < S::W; ++w)
+                tr[w * 64 + lane] = (v4u){acc[0][w], acc[1][w], acc[2][w], acc[3][w]};
+            tr += S::W * 64;
         }
     } else {
-        const int lo = min(G - 1, T), hi = max(lo, tk.min_rlen);
-        sweep_steps(T, lo, hi, run);
+        uint32_t *tr = a.trace + tk.trace_base;
+        uint32_t rr_next = rr_lds[-g];  // column of step 0
+        auto run = [&](auto masked, int t) {
+            int j = t - g;
+            uint32_t rr = rr_next;
+            rr_next = rr_lds[1 + j];  // prefetch the next step's column
+            uint32_t vmask = 0;
+            if constexpr (decltype(masked)::value) {
+#pragma unroll
+                for (int h = 0; h < PPG; ++h)
+                    if (j >= 0 && j < rl[h]) vmask |= (PK ? 0xFFFFu : 0xFFFFFFFFu) << (16 * h);
+            }
+            uint32_t a1[S::W];
+#pragma unroll
+            for (int w = 0; w < S::W; ++w) a1[w] = 0;
+            sw.template step<decltype(masked)::value>(rr, j, vmask, splat<PK>(15 - (t & 15)), a1);
+#pragma unroll
+            for (int w = 0; w < S::W; ++w) tr[trace_word<S::W>(t, w, lane)] = a1[w];
+        };
+        // int32: masked steps keep the cells outside a pair's columns out of
+        // its row maxima.  Packed: no step is masked (see Sweep).
+        if constexpr (PK) {
+            for (int t = 0; t < T; ++t) {
+                run(std::false_type{}, t);
+                if ((t & 15) == 15 || t == T - 1) sw.block_end(splat<true>((t >> 4) << 5));
+            }
+        } else {
+            const int lo = min(G - 1, T), hi = max(lo, tk.min_rlen);
+            sweep_steps(T, lo, hi, run);
+        }
     }
 
-    // per half: lane best over valid rows, then group max
+    // per half: the lane's best cell, then the group's
     GroupResult gres[PPG];
 #pragma unroll
     for (int h = 0; h < PPG; ++h) {
         uint32_t bh = 0, brow = 0, bcol = 0;
+        if constexpr (LEAN) {
+            int row, t;
+            sw.result(h, bh, row, t);
+            brow = (uint32_t)(g * R + row + 1);
+            bcol = (uint32_t)(t - g + 1);
+        } else {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            int row = g * R + r;
-            uint32_t hv, cv;
-            if constexpr (PK) {
-                // block << 5 | (15 - t%16) -> step t -> column t - g (+1)
-                const uint32_t bc = (sw.bcol[r] >> (16 * h)) & 0xFFFFu;
-                hv = ((sw.best[r] >> (16 * h)) & 0xFFFFu) >> 5;
-                cv = ((bc >> 5) << 4) + 15u - (bc & 15u) - (uint32_t)g + 1;
-            } else {
-                hv = sw.best[r] >> kColBits;
-                cv = kMaxCols - (sw.best[r] & kMaxCols) + 1;
-            }
-            if (row < ql[h] && hv > bh) {
-                bh = hv;
-                brow = row + 1;
-                bcol = cv;
+            for (int r = 0; r < R; ++r) {
+                int row = g * R + r;
+                uint32_t hv, cv;
+                if constexpr (PK) {
+                    // block << 5 | (15 - t%16) -> step t -> column t - g (+1)
+                    const uint32_t bc = (sw.bcol[r] >> (16 * h)) & 0xFFFFu;
+                    hv = ((sw.best[r] >> (16 * h)) & 0xFFFFu) >> 5;
+                    cv = ((bc >> 5) << 4) + 15u - (bc & 15u) - (uint32_t)g + 1;
+                } else {
+                    hv = sw.best[r] >> kColBits;
+                    cv = kMaxCols - (sw.best[r] & kMaxCols) + 1;
+                }
+                if (row < ql[h] && hv > bh) {
+                    bh = hv;
+                    brow = row + 1;
+                    bcol = cv;
+                }
             }
         }
         gres[h] = group_best<G>(bh, brow, bcol, R, PK, a.h_limit, (exotic >> h) & 1);
@@ -1234,15 +1469,17 @@ __global__ void __launch_bounds__(64) sw_plain_expand_kernel(const char *qseq, c
 
 // Occupancy floor per row class (waves per SIMD), set where the natural
 // register count sits just above an occupancy step.
-__host__ __device__ constexpr int batch_waves_per_eu(int R, bool pk) {
-    return pk ? (R <= 7 ? 5 : R <= 12 ? 4 : R <= 16 ? 3 : 2) : (R <= 10 ? 5 : R <= 16 ? 4 : 3);
+__host__ __device__ constexpr int batch_waves_per_eu(int R, bool pk, bool lean) {
+    return lean ? (R <= 6 ? 5 : R <= 12 ? 4 : 3)
+           : pk ? (R <= 7 ? 5 : R <= 12 ? 4 : R <= 16 ? 3 : 2)
+                : (R <= 10 ? 5 : R <= 16 ? 4 : 3);
 }
 
-template <int R, bool PK, int POL>
+template <int R, bool PK, bool LEAN>
 __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(batch_waves_per_eu(R, PK))))
+__attribute__((amdgpu_waves_per_eu(batch_waves_per_eu(R, PK, LEAN))))
 sw_batch_kernel(BatchArgs a) {
-    __shared__ uint32_t lds[4][4 * group_lds_words<kBatchG>()];
+    __shared__ uint32_t lds[4][wave_lds_words<kBatchG>()];
     const int wave = threadIdx.x >> 6;
     const int lo = *a.task_lo, hi = *a.task_hi;
     if (lo >= hi) return;
@@ -1252,7 +1489,7 @@ sw_batch_kernel(BatchArgs a) {
         tid = __builtin_amdgcn_readfirstlane(__shfl(tid, 0, 64)) + lo;
         if (tid >= hi) break;
         const Task tk = a.tasks[tid];
-        run_task<kBatchG, R, PK, POL>(a, tk, lds[wave]);
+        run_task<kBatchG, R, PK, LEAN>(a, tk, lds[wave]);
     }
 }
 
@@ -1261,9 +1498,9 @@ sw_batch_kernel(BatchArgs a) {
 // pairs per task.  A 16-lane group sweeps R = 20 rows per lane over rlen + 15
 // steps; a 64-lane group 5 rows over rlen + 63, so one task's latency, which
 // is all a small batch waits for, drops about 3.5x for the same total work.
-template <int R>
+template <int R, bool LEAN>
 __global__ void __launch_bounds__(256) sw_batch_wide_kernel(BatchArgs a) {
-    __shared__ uint32_t lds[4][group_lds_words<kWideG>()];
+    __shared__ uint32_t lds[4][wave_lds_words<kWideG>()];
     const int wave = threadIdx.x >> 6;
     const int lo = *a.task_lo, hi = *a.task_hi;
     if (lo >= hi) return;
@@ -1273,7 +1510,7 @@ __global__ void __launch_bounds__(256) sw_batch_wide_kernel(BatchArgs a) {
         tid = __builtin_amdgcn_readfirstlane(__shfl(tid, 0, 64)) + lo;
         if (tid >= hi) break;
         const Task tk = a.tasks[tid];
-        run_task<kWideG, R, true, kOneHot>(a, tk, lds[wave]);
+        run_task<kWideG, R, true, LEAN>(a, tk, lds[wave]);
     }
 }
 
@@ -1757,9 +1994,8 @@ hipError_t launch_plain(const char *q, const char *r, int qlen, int rlen_max, co
 
 // Persistent grid of one row-class kernel: as many 256-thread blocks as fit
 // on every CU at once (cached per kernel); `waves_per_cu` > 0 caps it.
-template <int RR, bool PK, class K>
-static int full_grid(K kernel, int cu_count, int waves_per_cu, int max_tasks) {
-    static int cached = -1;  // one per row class and lane width
+template <class K>
+static int full_grid(K kernel, int &cached, int cu_count, int waves_per_cu, int max_tasks) {
     if (cached < 0) {
         int blocks = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, 256, 0) != hipSuccess ||
@@ -1776,49 +2012,59 @@ static int full_grid(K kernel, int cu_count, int waves_per_cu, int max_tasks) {
     return b * cu_count;
 }
 
-hipError_t launch_batch_wide(const BatchArgs &ba, int cu_count, int max_tasks, hipStream_t st) {
-    auto k = sw_batch_wide_kernel<kWideRows>;
+template <bool LEAN>
+static void launch_wide(const BatchArgs &ba, int cu_count, int max_tasks, hipStream_t st) {
     static int blocks = -1;  // per CU, at full occupancy
-    if (blocks < 0) {
-        int b = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k, 256, 0) != hipSuccess || b < 1)
-            b = 2;
-        blocks = b;
-    }
-    int grid = blocks * cu_count;
-    if (max_tasks > 0) grid = min(grid, (max_tasks + 3) / 4);
-    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, ba);
+    auto k = sw_batch_wide_kernel<kWideRows, LEAN>;
+    hipLaunchKernelGGL(k, dim3(full_grid(k, blocks, cu_count, 0, max_tasks)), dim3(256), 0, st, ba);
+}
+
+hipError_t launch_batch_wide(const BatchArgs &ba, int cu_count, int max_tasks, hipStream_t st) {
+    if (ba.lean) launch_wide<true>(ba, cu_count, max_tasks, st);
+    else launch_wide<false>(ba, cu_count, max_tasks, st);
     return hipGetLastError();
 }
 
-hipError_t launch_batch(const BatchArgs &ba, bool int16, int rows, int cu_count, int waves_per_cu,
-                        int max_tasks, hipStream_t st) {
+template <int R, bool PK, bool LEAN>
+static void launch_class(const BatchArgs &ba, int cu_count, int waves_per_cu, int max_tasks,
+                         hipStream_t st) {
+    static int blocks = -1;  // one per row class, lane width and form
+    auto k = sw_batch_kernel<R, PK, LEAN>;
+    hipLaunchKernelGGL(k, dim3(full_grid(k, blocks, cu_count, waves_per_cu, max_tasks)), dim3(256),
+                       0, st, ba);
+}
+
+template <bool LEAN>
+static hipError_t launch_rows(const BatchArgs &ba, bool int16, int rows, int cu_count,
+                              int waves_per_cu, int max_tasks, hipStream_t st) {
     if (int16) {
         switch (rows) {
-#define SWIFT_L16(RR)                                                                      \
-    case RR: {                                                                             \
-        auto k = sw_batch_kernel<RR, true, kOneHot>;                                       \
-        hipLaunchKernelGGL(k, dim3(full_grid<RR, true>(k, cu_count, waves_per_cu, max_tasks)), dim3(256), 0, st, ba); \
-        break;                                                                             \
-    }
+#define SWIFT_L16(RR)                                                        \
+    case RR:                                                                 \
+        launch_class<RR, true, LEAN>(ba, cu_count, waves_per_cu, max_tasks, st); \
+        break;
             SWIFT_R16_CASES(SWIFT_L16)
 #undef SWIFT_L16
         default: return hipErrorInvalidValue;
         }
     } else {
         switch (rows) {
-#define SWIFT_L32(RR)                                                                      \
-    case RR: {                                                                             \
-        auto k = sw_batch_kernel<RR, false, kBytes>;                                       \
-        hipLaunchKernelGGL(k, dim3(full_grid<RR, false>(k, cu_count, waves_per_cu, max_tasks)), dim3(256), 0, st, ba); \
-        break;                                                                             \
-    }
+#define SWIFT_L32(RR)                                                         \
+    case RR:                                                                  \
+        launch_class<RR, false, LEAN>(ba, cu_count, waves_per_cu, max_tasks, st); \
+        break;
             SWIFT_R32_CASES(SWIFT_L32)
 #undef SWIFT_L32
         default: return hipErrorInvalidValue;
         }
     }
     return hipGetLastError();
+}
+
+hipError_t launch_batch(const BatchArgs &ba, bool int16, int rows, int cu_count, int waves_per_cu,
+                        int max_tasks, hipStream_t st) {
+    return ba.lean ? launch_rows<true>(ba, int16, rows, cu_count, waves_per_cu, max_tasks, st)
+                   : launch_rows<false>(ba, int16, rows, cu_count, waves_per_cu, max_tasks, st);
 }
 
 hipError_t launch_walk(const BatchArgs &ba, const int32_t *order, const int32_t *first,

@@ -17,6 +17,11 @@ struct KeyConsts {
     // no sign-splat to turn a masked merge of packed halves into per-half
     // compares and selects
     int sign;
+    // lean sweeps (see Lean): the diagonal-ready addend 4*match + 3, the
+    // mismatch penalty 4*(match - mismatch), and the exits' penalties by the
+    // cell's direction code, one byte each
+    int x, pm;
+    uint32_t tab_u, tab_l;
 };
 
 // ONEHOT: flag = match,    dr = 4*mismatch + 3, dsub = 4*(match - mismatch)
@@ -36,8 +41,29 @@ inline KeyConsts make_consts(const Scoring &s, int policy) {
     k.eo1 = 4 * s.gap_open + 1;
     k.de = 4 * (s.gap_ext - s.gap_open);
     k.sign = 15;
+    k.x = 4 * s.match + 3;
+    k.pm = 4 * (s.match - s.mismatch);
+    // exit = key - penalty: 4*(H + gap) + 2 (up) or + 1 (left) from 4*H + d;
+    // d = 0 (a start, key 0) saturates whatever is subtracted
+    k.tab_u = k.tab_l = 0;
+    for (int d = 1; d <= 3; ++d) {
+        k.tab_u |= (uint32_t)((d - 2 - 4 * (d == 2 ? s.gap_ext : s.gap_open)) & 0xFF) << (8 * d);
+        k.tab_l |= (uint32_t)((d - 1 - 4 * (d == 1 ? s.gap_ext : s.gap_open)) & 0xFF) << (8 * d);
+    }
     return k;
 }
+
+// Scorings of the lean sweeps: mismatch and gap moves all lose score (their
+// steps run unmasked), the exits' penalties fit a byte, and the mismatch
+// penalty 7 bits (bit 7 of a match table marks padding rows).
+inline bool lean_scoring(const Scoring &s) {
+    return s.match >= 1 && s.mismatch < 0 && s.match - s.mismatch <= 31 && s.gap_open <= -1 &&
+           s.gap_open >= -63 && s.gap_ext <= -1 && s.gap_ext >= -63;
+}
+// ... and the packed ones' best-cell keys 32*H + row code must stay below the
+// half-precision infinity's bit pattern, 0x7C00 (their maxima are taken as
+// half-precision numbers): scores below this limit
+constexpr int kLeanScoreLimit = 960;
 
 constexpr int kColBits = 12;                   // int32 best key: H << 12 | (4095 - j)
 constexpr int kMaxCols = (1 << kColBits) - 1;  // longest reference window (plain kernel)
@@ -88,6 +114,7 @@ struct BatchArgs {
     int32_t *score_out, *start_out, *end_out, *alen_out;
     char *qcons, *rcons;
     const int64_t *coff;
+    int lean;                 // 1: the lean sweeps (lean_scoring)
     int walk_deferred;        // 1: record PairTrace descriptors, walk in sw_walk_kernel
     int32_t *nflagged;        // counts the pairs flagged for the int32 re-run
 };
