@@ -82,22 +82,22 @@ int swift_align_sequences_noalloc(char *querySeq_d, char *refSeq_d, int querySeq
     bool f32;
     if ((rc = validate_scoring(sc, qlen, rlen, &f32))) return rc;
     if (npairs == 0) return kOk;
-    // words per pair: the trace, the best cell and the walk's moves
-    const int64_t wpp = plain_scratch_words(qlen, rlen);
-    if (wpp > kNoAllocWords) {
+    const PlainPlan pl = plain_plan(sc, qlen, rlen, npairs);
+    int chunk, waves;
+    plain_chunk(pl, npairs, kNoAllocWords, &chunk, &waves);
+    if (plain_words(pl, 1, 1) > kNoAllocWords) {
         set_error("one pair's traceback needs %lld words, beyond the %lld-word scratch",
-                  (long long)wpp, (long long)kNoAllocWords);
+                  (long long)plain_words(pl, 1, 1), (long long)kNoAllocWords);
         return kErrCapacity;
     }
     uint32_t *trace = nullptr;
     if ((rc = scratch_words(&trace))) return rc;
-    const int chunk = (int)std::min<int64_t>(npairs, kNoAllocWords / wpp);
     hipStream_t st = (hipStream_t)stream;
     for (int c0 = 0; c0 < npairs; c0 += chunk) {
         const int cn = std::min(chunk, npairs - c0);
         PlainOut out{score_d, alignStart_d, alignEnd_d, alignLength_d, queryConsensus_d,
                      refConsensus_d, (int64_t)qlen + rlen + 2};
-        SWIFT_HIP_TRY(launch_plain(querySeq_d, refSeq_d, qlen, rlen, sc, cn, c0, trace, out, st));
+        SWIFT_HIP_TRY(launch_plain(pl, querySeq_d, refSeq_d, sc, cn, c0, trace, waves, out, st));
     }
     return kOk;
 }

@@ -262,10 +262,11 @@ int align_sequences_status(char *q_d, char *r_d, int qlen, int rlen, float match
     bool f32;
     if ((rc = validate_scoring(sc, qlen, rlen, &f32))) return rc;
     Workspace &w = ws();
-    const int64_t wpp = plain_scratch_words(qlen, rlen);
-    int chunk = (int)std::min<int64_t>(npairs, std::max<int64_t>(1, g_plain_budget_words / wpp));
+    const PlainPlan pl = plain_plan(sc, qlen, rlen, npairs);
+    int chunk, waves;
+    plain_chunk(pl, npairs, (int64_t)g_plain_budget_words, &chunk, &waves);
     if (g_plain_chunk_pairs > 0) chunk = std::min(chunk, g_plain_chunk_pairs);
-    const size_t need = (size_t)chunk * wpp * 4;
+    const size_t need = (size_t)plain_words(pl, chunk, waves) * 4;
     if (!w.p_done) SWIFT_HIP_TRY(hipEventCreateWithFlags(&w.p_done, hipEventDisableTiming));
     if (w.p_pending) {
         // a larger trace replaces the buffer the last call's kernels may
@@ -283,8 +284,8 @@ int align_sequences_status(char *q_d, char *r_d, int qlen, int rlen, float match
     const PlainOut out{score_d, start_d, end_d, alen_d, qcons_d, rcons_d, (int64_t)qlen + rlen + 2};
     for (int c0 = 0; c0 < npairs; c0 += chunk) {
         const int cn = std::min(chunk, npairs - c0);
-        SWIFT_HIP_TRY(launch_plain(q_d, r_d, qlen, rlen, sc, cn, c0, w.p_trace.as<uint32_t>(),
-                                   out, st));
+        SWIFT_HIP_TRY(launch_plain(pl, q_d, r_d, sc, cn, c0, w.p_trace.as<uint32_t>(), waves, out,
+                                   st));
     }
     SWIFT_HIP_TRY(hipEventRecord(w.p_done, st));
     w.p_pending = true;

@@ -11,17 +11,28 @@ struct BatchArgs;
 struct BinArgs;
 struct TaskArgs;
 
-// launch helpers implemented in sw_kernels.hip
+// The plain path's route for a call, and its sizes in 32-bit words
+// (sw_plain.hip)
+struct PlainPlan {
+    enum Route { kGeneral, kPacked, kWave } route;
+    int qlen, rlen, move_words;
+    int wave_rows, packed_rows;   // rows a lane of the whole-wave and the packed sweeps
+    int64_t wave_words;           // trace of a pair swept by a whole wave
+    int64_t task_words;           // trace of eight packed pairs
+};
 struct PlainOut;
-// Plain path over pairs [pair0, pair0 + npairs) of the caller's arrays:
-// sweep, walk and consensus expansion.  scratch holds
-// npairs * plain_scratch_words(qlen, rlen_max) words.
-hipError_t launch_plain(const char *q, const char *r, int qlen, int rlen_max, const Scoring &sc,
-                        int npairs, int pair0, uint32_t *scratch, const PlainOut &out,
+PlainPlan plain_plan(const Scoring &sc, int qlen, int rlen, int npairs);
+// the largest chunk of at most npairs pairs that fits `budget` words of
+// scratch (one pair at least), with its waves of the wave kernel
+void plain_chunk(const PlainPlan &pl, int npairs, int64_t budget, int *chunk, int *waves);
+int64_t plain_words(const PlainPlan &pl, int npairs, int waves);
+// Plain path over pairs [pair0, pair0 + npairs) of the caller's arrays: sweep,
+// walk and consensus expansion.  scratch holds plain_words(pl, npairs, waves)
+// words, 16-byte aligned.
+hipError_t launch_plain(const PlainPlan &pl, const char *q, const char *r, const Scoring &sc,
+                        int npairs, int pair0, uint32_t *scratch, int waves, const PlainOut &out,
                         hipStream_t st);
 int plain_rows_for(int qlen);
-int plain_trace_words(int R);
-int64_t plain_scratch_words(int qlen, int rlen);  // device words per pair
 void set_plain_chunk_pairs(int pairs);             // 0: chunks by the scratch budget alone
 hipError_t launch_fill(int32_t *p, int n, int32_t v, hipStream_t st);
 // up to four int32 arrays zeroed by one kernel launch
