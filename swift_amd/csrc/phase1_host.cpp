@@ -492,6 +492,7 @@ int align_enqueue(const MapArgs &m, const PairsDev &p, Workspace *sws, int nread
     io.rcons = rec.ref_cons;
     io.cons_off = p.coff;
     io.refs_plain = m.ix.plain_bases;
+    io.sparse = 1;
     if (sync)
         rc = sws ? sw_batch_run_in(sws, io, sc, st) : sw_batch_run(io, sc, st, true);
     else

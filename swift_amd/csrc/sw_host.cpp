@@ -91,7 +91,9 @@ struct Workspace {
         int64_t steps[2 * kRBins];
         int32_t seg[2 * kRBins + 1];
         int32_t cnt[16];
+        int32_t small[kSmallFlags];  // written by the one-launch form
     } *stage = nullptr;
+    int32_t reruns_seen = 0;  // the one-launch form's counter after the last call that read it
     int cu_count = 0;
     BatchStats stats{};
     // Side streams the row-class kernels are spread over (fork/join by
@@ -325,6 +327,11 @@ static int64_t worst_trace_words(int npairs, int maxq, int maxr) {
         int64_t w32t = (r32_class(kRBins) + 15) / 16;
         words = std::max(words, tw * wsteps * 64 + 2 * t32 * w32t * steps * 64);
     }
+    // the one-launch form's waves
+    if (small_call(npairs, maxq, true)) {
+        const int waves = npairs <= kSmallSingles ? npairs : std::min((npairs + 7) / 2, kSmallWaves);
+        words = std::max(words, waves * small_wave_words(maxr));
+    }
     return words;
 }
 
@@ -346,7 +353,10 @@ static int reserve_common(Workspace &w, int npairs) {
     if ((rc = w.scan_sums.ensure(((size_t)mt / 2048 + 2) * 8))) return rc;
     if ((rc = w.bins.ensure((size_t)4 * kNumBins * 4))) return rc;
     if ((rc = w.segs.ensure((size_t)2 * 3 * (2 * kRBins + 1) * 4))) return rc;
-    if ((rc = w.counters.ensure(256 * 4))) return rc;
+    if (!w.counters.ptr) {
+        if ((rc = w.counters.ensure(256 * 4))) return rc;
+        SWIFT_HIP_TRY(hipMemset(w.counters.ptr, 0, 256 * 4));
+    }
     if ((rc = w.totals.ensure((size_t)(kTotSteps + 2 * 2 * kRBins) * 8))) return rc;
     if (!w.stage) {
         void *p = nullptr;
@@ -386,6 +396,7 @@ int reserve_batch_in(Workspace *w, int npairs, int maxq, int maxr) {
 constexpr int kCntError = 8;
 constexpr int kCntFlagged = 9;
 constexpr int kCntQueues = 16;
+constexpr int kCntReruns = 200;  // never zeroed (sw_small.hip)
 constexpr int kQueuesPerPass = 2 * kRBins;
 // sync_sizes: the sizes of each pass are read back (synchronising); then
 // final_sync also waits for the pass's last kernels before returning
@@ -417,6 +428,70 @@ int sw_batch_check_in(Workspace *w, hipStream_t st) {
         set_error("pair lengths beyond the batched limits (%d/%d)", kMaxBatchQ, kMaxBatchR);
         return kErrCapacity;
     }
+    return kOk;
+}
+
+// A small call as one kernel (sw_small.hip).  *done: 0 when a pair was longer
+// than the call said and the general path has to run.
+static int batch_run_small(Workspace &w, const BatchIO &io, const KeyConsts &kc, uint32_t h_limit,
+                           hipStream_t st, bool final_sync, int *done) {
+    const int n = io.npairs;
+    SmallArgs a{};
+    a.qseq = io.qseq;
+    a.qoff = io.qoff;
+    a.qlen = io.qlen;
+    a.rseq = io.rseq;
+    a.roff = io.roff;
+    a.rlen = io.rlen;
+    a.npairs = n;
+    a.ppw = n <= kSmallSingles ? 1 : 2;
+    a.maxq = std::max(io.maxq, 1);
+    a.maxr = std::max(io.maxr, 1);
+    a.kc = kc;
+    a.h_limit = h_limit;
+    a.wave_words = small_wave_words(a.maxr);
+    // workgroups of four waves where several of them share a SIMD anyway
+    a.wpb = n >= kWideShortPairs && a.maxq <= kBatchG * kCoarseRowsSmall ? 4 : 1;
+    const int blocks = std::min((n + a.ppw * a.wpb - 1) / (a.ppw * a.wpb), kSmallWaves / a.wpb);
+    const int waves = blocks * a.wpb;
+    int rc;
+    if ((rc = w.trace.ensure((size_t)waves * a.wave_words * 4))) return rc;
+    a.trace = w.trace.as<uint32_t>();
+    a.score_out = io.score;
+    a.start_out = io.start;
+    a.end_out = io.end;
+    a.alen_out = io.alen;
+    a.qcons = io.qcons;
+    a.rcons = io.rcons;
+    a.coff = io.cons_off;
+    a.flags = w.stage->small;
+    a.reruns = w.counters.as<int32_t>() + kCntReruns;
+    volatile int32_t *flags = w.stage->small;
+    for (int i = 0; i < kSmallFlags; ++i) flags[i] = 0;
+    for (int i = 0; i < 2; ++i) SWIFT_HIP_TRY(mark(i, st, w.timed));
+    SWIFT_HIP_TRY(launch_small(a, blocks, st));
+    for (int i = 2; i < 5; ++i) SWIFT_HIP_TRY(mark(i, st, w.timed));
+    w.stats.ntasks16 = (n + a.ppw * a.wpb - 1) / (a.ppw * a.wpb);
+    w.stats.trace_words = (int64_t)waves * a.wave_words;
+    *done = 1;
+    if (!final_sync) return kOk;
+    SWIFT_HIP_TRY(hipStreamSynchronize(st));
+    if (flags[kSmallError]) {
+        set_error("pair lengths beyond maxq/maxr or the batched limits (%d/%d)", kMaxBatchQ,
+                  kMaxBatchR);
+        return kErrCapacity;
+    }
+    if (flags[kSmallLonger]) *done = 0;
+    if (flags[kSmallRerun]) {
+        int32_t now = 0;
+        SWIFT_HIP_TRY(hipMemcpyAsync(&now, a.reruns, 4, hipMemcpyDeviceToHost, st));
+        SWIFT_HIP_TRY(hipStreamSynchronize(st));
+        w.stats.nrerun = w.stats.ntasks32 = now - w.reruns_seen;
+        w.reruns_seen = now;
+    }
+    if (g_timing.on && w.timed)
+        for (int i = 0; i < 4; ++i)
+            SWIFT_HIP_TRY(hipEventElapsedTime(&g_timing.ms[i], g_timing.ev[i], g_timing.ev[i + 1]));
     return kOk;
 }
 
@@ -465,8 +540,9 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
                : n >= kCoarseTinyPairs || (n >= kWideShortPairs && short_q) ? kCoarseRowsSmall
                                                                            : kRBins)
             : 0;
-    // a single class (the smallest batches) runs the wide form: its few
-    // tasks are each one wave, and a wave's sweep is the batch's latency
+    // a single class (the smallest batches, other scorings than the
+    // one-launch form's) runs the wide form: its few tasks are each one wave,
+    // and a wave's sweep is the batch's latency
     const int wide = coarse == kRBins ? 1 : 0;
     auto pass_args = [&](int pass, const PairResult *prev, int f32, BinArgs &b, TaskArgs &t) {
         b = BinArgs{io.rseq, io.roff, io.qlen, io.rlen, prev, n, f32, w.bin_of.as<int32_t>(),
@@ -494,6 +570,17 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     const uint32_t lean_limit = 4u * (uint32_t)(kLeanScoreLimit - 2 * pos);
     const bool lean16 = lean32 && (int64_t)io.maxq * pos * 4 < (int64_t)lean_limit;
     if (lean16) h_limit = lean_limit;
+
+    // a small call in one launch, unless row classes are asked for (coarse
+    // ones below kCoarseTinyPairs are this form)
+    if (lean16 && !force32 && (cmode < 0 || (cmode == 1 && n < kCoarseTinyPairs)) &&
+        small_call(n, io.maxq, io.sparse)) {
+        int done = 0;
+        if ((rc = batch_run_small(w, io, kc16, h_limit, st, sync_sizes && final_sync, &done)) ||
+            done)
+            return rc;
+        w.stats = BatchStats{};
+    }
 
     // one launch zeroes the results (they start at "score 0": a pair no
     // kernel reaches never walks), the error flag, the flagged count, the
@@ -652,10 +739,10 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
             b.task_hi = t.seg_task0 + seg + 1;
             b.next_task = cnt + kCntQueues + pass * kQueuesPerPass + seg;
             b.kc = cls == 0 ? kc16 : kc32;
-            b.lean = cls == 0 ? lean16 : lean32;
             hipStream_t s2 = nside ? w.side[lane_of[seg]] : st;
             const int wpc = w.waves_per_cu >= 0 ? w.waves_per_cu : tuning().waves_per_cu;
             const bool wseg = t.wide && seg == 0;
+            b.lean = cls == 0 ? lean16 && !wseg : lean32;
             const int ntk = seg_host ? seg_host[seg + 1] - seg_host[seg] : 0;
             if (wseg)
                 SWIFT_HIP_TRY(launch_batch_wide(b, w.cu_count, ntk, s2));

@@ -83,6 +83,9 @@ struct BatchIO {
     // the pipeline does from its index); with scores that cannot reach the
     // int16 limit either, no pair can take the int32 re-run
     int refs_plain = 0;
+    // 1: npairs is a capacity and pairs may be missing (length 0), as in the
+    // pipeline
+    int sparse = 0;
 };
 
 int validate_scoring(const Scoring &s, int maxq, int maxr, bool *force32);
@@ -142,6 +145,25 @@ constexpr int kCoarseTinyPairs = 4096;    // ... and to one class (R = kRBins) b
 // ... but from this many pairs only when some query needs more than
 // kCoarseRowsSmall rows per 16-lane group
 constexpr int kWideShortPairs = 2048;
+// One-launch form (sw_small.hip): a pair a wave up to kSmallSingles pairs (one
+// wave a SIMD), then two.
+constexpr int kSmallSingles = 1024;
+constexpr int kSmallWaves = 4096;   // each keeps a trace area
+// Its waves take pairs unsorted, 64 lanes of ceil(maxq / 64) rows each, against
+// the general path's binning, readback and 16-lane groups: taken up to
+// kSmallWork = pairs x rows a lane.  Queries of 50-300 and of 100 bases, us a
+// call, general -> one launch:
+//   50-300: 512 172 -> 104, 4,000 240 -> 172, 8,000 408 -> 286, 16,000 568 ->
+//   526, 20,000 618 -> 621, 24,000 637 -> 752
+//   100: 512 143 -> 55, 4,500 208 -> 100, 24,000 478 -> 391, 40,000 659 -> 623
+// A pipeline's capacity counts slots of which a half or fewer hold records, so
+// twice that: 5,000 reads of 300 bases (capacity 30,000) 1,052 -> 816 us,
+// 13,000 of 100 1,039 -> 995.
+constexpr int kSmallWork = 80000;
+inline bool small_call(int npairs, int maxq, bool sparse) {
+    const int64_t rows = maxq > 64 ? (maxq + 63) / 64 : 1;
+    return npairs * rows <= (sparse ? 2 : 1) * (int64_t)kSmallWork;
+}
 Tuning &tuning();
 
 }  // namespace swift

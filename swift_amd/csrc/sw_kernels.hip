@@ -432,12 +432,13 @@ sw_batch_kernel(BatchArgs a) {
     }
 }
 
-// The wide form for batches too small to fill the chip: one 64-lane group
+// The wide form for batches too small to fill the chip (scorings outside
+// lean_scoring; the others take sw_small.hip's kernel): one 64-lane group
 // per wave (the lane shift a wave_shr), kWideRows rows per lane, two packed
 // pairs per task.  A 16-lane group sweeps R = 20 rows per lane over rlen + 15
 // steps; a 64-lane group 5 rows over rlen + 63, so one task's latency, which
 // is all a small batch waits for, drops about 3.5x for the same total work.
-template <int R, bool LEAN>
+template <int R>
 __global__ void __launch_bounds__(256) sw_batch_wide_kernel(BatchArgs a) {
     __shared__ uint32_t lds[4][wave_lds_words<kWideG>()];
     const int wave = threadIdx.x >> 6;
@@ -449,7 +450,7 @@ __global__ void __launch_bounds__(256) sw_batch_wide_kernel(BatchArgs a) {
         tid = __builtin_amdgcn_readfirstlane(__shfl(tid, 0, 64)) + lo;
         if (tid >= hi) break;
         const Task tk = a.tasks[tid];
-        run_task<kWideG, R, true, LEAN>(a, tk, lds[wave]);
+        run_task<kWideG, R, true, false>(a, tk, lds[wave]);
     }
 }
 
@@ -846,16 +847,10 @@ static int full_grid(K kernel, int &cached, int cu_count, int waves_per_cu, int 
     return b * cu_count;
 }
 
-template <bool LEAN>
-static void launch_wide(const BatchArgs &ba, int cu_count, int max_tasks, hipStream_t st) {
-    static int blocks = -1;  // per CU, at full occupancy
-    auto k = sw_batch_wide_kernel<kWideRows, LEAN>;
-    hipLaunchKernelGGL(k, dim3(full_grid(k, blocks, cu_count, 0, max_tasks)), dim3(256), 0, st, ba);
-}
-
 hipError_t launch_batch_wide(const BatchArgs &ba, int cu_count, int max_tasks, hipStream_t st) {
-    if (ba.lean) launch_wide<true>(ba, cu_count, max_tasks, st);
-    else launch_wide<false>(ba, cu_count, max_tasks, st);
+    static int blocks = -1;  // per CU, at full occupancy
+    auto k = sw_batch_wide_kernel<kWideRows>;
+    hipLaunchKernelGGL(k, dim3(full_grid(k, blocks, cu_count, 0, max_tasks)), dim3(256), 0, st, ba);
     return hipGetLastError();
 }
 

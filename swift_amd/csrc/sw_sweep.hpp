@@ -828,6 +828,12 @@ __device__ __forceinline__ WalkOut walk_wave(const uint4 *tr, int R, int W, int 
     return WalkOut{start, start + nrb, tick};
 }
 
+// A flag in mapped host memory, read by the host after it has waited for the
+// kernel.
+__device__ __forceinline__ void host_flag(int32_t *f) {
+    __hip_atomic_store(f, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // One pair's consensus expansion, by one row of L lanes of a wave (lane sl of

@@ -119,6 +119,31 @@ struct BatchArgs {
     int32_t *nflagged;        // counts the pairs flagged for the int32 re-run
 };
 
+// One-launch form of a small batched call (sw_small.hip).  flags: mapped host
+// words, zeroed by the host before the launch.
+enum SmallFlag { kSmallError = 0, kSmallLonger = 1, kSmallRerun = 2, kSmallFlags = 3 };
+struct SmallArgs {
+    const char *qseq;
+    const int64_t *qoff;
+    const int32_t *qlen;
+    const char *rseq;
+    const int64_t *roff;
+    const int32_t *rlen;
+    int npairs, ppw, wpb;     // pairs, pairs a wave (1 or 2), waves a workgroup (<= 4)
+    int maxq, maxr;
+    KeyConsts kc;
+    uint32_t h_limit;         // 4*H at or above this: swept again in 32-bit lanes
+    uint32_t *trace;          // wave_words for each wave of the grid
+    int64_t wave_words;
+    int32_t *score_out, *start_out, *end_out, *alen_out;
+    char *qcons, *rcons;
+    const int64_t *coff;
+    int32_t *flags;
+    int32_t *reruns;          // device: pairs swept again, counted on from call to call
+};
+int64_t small_wave_words(int maxr);
+hipError_t launch_small(const SmallArgs &a, int blocks, hipStream_t st);
+
 // outputs of the plain (alignSequences) kernel: reference layout
 struct PlainOut {
     float *score;

@@ -1,5 +1,5 @@
-"""The plain path's one-launch and packed routes against the oracle, at the
-sizes where they change."""
+"""The one-launch forms of small calls (batched and plain) and the plain path's
+packed route against the oracle, at the sizes where they change."""
 import random
 
 import numpy as np
@@ -14,6 +14,34 @@ pytestmark = pytest.mark.gpu
 def A():
     from swift_amd import align
     return align
+
+
+# pairs: one; the last with a pair a wave, the first with two (an odd count);
+# past one turn of the persistent waves; queries: each rows-per-lane count
+@pytest.mark.parametrize("n,qmax,rmax", [(1, 320, 480), (1024, 64, 300), (1025, 65, 97),
+                                         (2049, 160, 250), (300, 192, 480), (77, 320, 30),
+                                         (9001, 128, 200)])
+def test_small_batch(A, orc, n, qmax, rmax):
+    rnd = random.Random(n)
+    qs, rs = edge_pairs(rnd, n, qmax, rmax)
+    if n > 10:  # empty sequences: no strings, an empty alignment
+        qs[3], rs[5] = b"", b""
+    got = A.sw_batch(qs, rs)
+    if n > 100:
+        assert A.batch_stats()["nrerun"] > 0  # references with R, Y or k
+    if n > 10:
+        assert got.end[3] == got.end[5] == -1 and got.length[3] == got.length[5] == 0
+    check(got, orc.sw_batch(qs, rs, nthreads=8))
+
+
+def test_small_batch_longer_than_said(A, orc):
+    """maxq and maxr below the pairs' own lengths: the call still aligns them."""
+    rnd = random.Random(5)
+    qs, rs = edge_pairs(rnd, 200, 300, 400)
+    b = A.PairBatch(qs, rs)
+    b.maxq, b.maxr = 90, 120
+    b.run()
+    check(b.results(), orc.sw_batch(qs, rs, nthreads=8))
 
 
 # the wave route (any lengths) and the packed one from 4,096 pairs: rows 1, a
