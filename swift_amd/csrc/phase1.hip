@@ -31,13 +31,10 @@ namespace swift {
 
 __device__ __forceinline__ uint32_t kcode(unsigned char c) {
     // preprocessCreate (src/preprocess.cu:30-48): A/a 0, C/c 1, G/g 2,
-    // T/t 3, every other byte 0
-    switch (c) {
-    case 'C': case 'c': return 1;
-    case 'G': case 'g': return 2;
-    case 'T': case 't': return 3;
-    default: return 0;
-    }
+    // T/t 3, every other byte 0.  Selects, not a switch: a switch over bytes
+    // costs more scalar branch work than the whole hash
+    const uint32_t u = c & 0xDFu;
+    return u == 'C' ? 1u : u == 'G' ? 2u : u == 'T' ? 3u : 0u;
 }
 
 __device__ __forceinline__ unsigned char rc_byte(unsigned char c) {
@@ -66,6 +63,34 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
         if (lane >= d) v += o;
     }
     return v;
+}
+
+// The same scan, and reductions, through data-parallel primitives: row shifts
+// within 16 lanes, then row broadcasts (no LDS round trips).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_or(uint32_t old, uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, ROWS, 0xF, false);
+}
+template <class Op>
+__device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v, uint32_t identity, Op op) {
+    v = op(v, dpp_or<0x111, 0xF>(identity, v));  // row_shr 1, 2, 4, 8
+    v = op(v, dpp_or<0x112, 0xF>(identity, v));
+    v = op(v, dpp_or<0x114, 0xF>(identity, v));
+    v = op(v, dpp_or<0x118, 0xF>(identity, v));
+    v = op(v, dpp_or<0x142, 0xA>(identity, v));  // lane 15 of rows 0, 2 to rows 1, 3
+    v = op(v, dpp_or<0x143, 0xC>(identity, v));  // lane 31 to rows 2, 3
+    return v;
+}
+__device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
+    return wave_scan_dpp(v, 0u, [](uint32_t x, uint32_t y) { return x + y; });
+}
+__device__ __forceinline__ uint32_t wave_all_min(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_readlane(
+        (int)wave_scan_dpp(v, ~0u, [](uint32_t x, uint32_t y) { return min(x, y); }), 63);
+}
+__device__ __forceinline__ uint32_t wave_all_max(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_readlane(
+        (int)wave_scan_dpp(v, 0u, [](uint32_t x, uint32_t y) { return max(x, y); }), 63);
 }
 
 // Bitonic sort of n2 (a power of two) keys by threads tid, tid + nthr, ...;
@@ -121,46 +146,65 @@ __global__ void __launch_bounds__(256) idx_count(IndexDev ix, int64_t ntup) {
 
 __device__ __forceinline__ int kept(int c, int thr) { return (c > 0 && c <= thr) ? c : 0; }
 
-// per-chunk sums of the kept counts and the largest kept count
+// per chunk of kScanChunk hashes: the kept counts' sum, the largest of them and
+// the number of non-empty buckets (a word each: one address for every chunk's
+// atomics costs 10 ns a chunk)
 __global__ void __launch_bounds__(1024) idx_scan_blocks(IndexDev ix, IndexBuildScratch s) {
-    __shared__ int64_t red[1024];
-    __shared__ int32_t redm[1024];
+    __shared__ int64_t red[16];
+    __shared__ int32_t redm[16], redf[16];
     const int64_t base = (int64_t)blockIdx.x * kScanChunk;
+    uint32_t mx = 0, filled = 0;
     int64_t sum = 0;
-    int32_t mx = 0;
     for (int i = threadIdx.x; i < kScanChunk; i += 1024) {
         int64_t h = base + i;
         if (h < ix.nhash) {
-            int c = kept(ix.count[h], ix.thr);
+            const int c = kept(ix.count[h], ix.thr);
             sum += c;
-            mx = max(mx, c);
+            mx = max(mx, (uint32_t)c);
+            filled += c > 0;
         }
     }
-    red[threadIdx.x] = sum;
-    redm[threadIdx.x] = mx;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    mx = wave_all_max(mx);
+    const uint32_t wf = wave_scan_add(filled);
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 63) {
+        red[w] = sum;
+        redm[w] = (int32_t)mx;
+        redf[w] = (int32_t)wf;
+    }
     __syncthreads();
-    for (int off = 512; off > 0; off >>= 1) {
-        if (threadIdx.x < off) {
-            red[threadIdx.x] += red[threadIdx.x + off];
-            redm[threadIdx.x] = max(redm[threadIdx.x], redm[threadIdx.x + off]);
-        }
-        __syncthreads();
-    }
     if (threadIdx.x == 0) {
-        s.block_sum[blockIdx.x] = red[0];
-        atomicMax(s.max_actual, redm[0]);
+        int64_t t = 0;
+        int32_t m = 0, f = 0;
+        for (int i = 0; i < 16; ++i) {
+            t += red[i];
+            m = max(m, redm[i]);
+            f += redf[i];
+        }
+        s.block_sum[blockIdx.x] = t;
+        s.block_stat[blockIdx.x] = make_int2(m, f);
     }
 }
 
-// exclusive scan of the chunk sums (one workgroup); the total into *total
+// exclusive scan of the chunk sums (one workgroup); the total, the largest
+// kept count and the number of non-empty buckets beside it
 __global__ void __launch_bounds__(1024) idx_scan_sums(IndexBuildScratch s, int nblocks) {
     __shared__ int64_t part[1024];
     const int per = (nblocks + 1023) / 1024;
     int64_t sum = 0;
+    int32_t mx = 0, filled = 0;
     for (int i = 0; i < per; ++i) {
         int b = threadIdx.x * per + i;
-        if (b < nblocks) sum += s.block_sum[b];
+        if (b < nblocks) {
+            sum += s.block_sum[b];
+            mx = max(mx, s.block_stat[b].x);
+            filled += s.block_stat[b].y;
+        }
     }
+    if (mx) atomicMax(s.max_actual, mx);
+    if (filled) atomicAdd(s.filled, filled);
     part[threadIdx.x] = sum;
     __syncthreads();
     for (int off = 1; off < 1024; off <<= 1) {
@@ -216,6 +260,15 @@ __global__ void __launch_bounds__(1024) idx_scan_apply(IndexDev ix, IndexBuildSc
         }
         run += loc[i];
     }
+    // this thread's `per` hashes of the non-empty buckets' bitmap, 32 to a word
+    static_assert(per == 4, "eight threads to a word");
+    uint32_t w = 0;
+#pragma unroll
+    for (int i = 0; i < per; ++i) w |= loc[i] > 0 ? 1u << i : 0u;
+    w <<= 4 * (threadIdx.x & 7);
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) w |= (uint32_t)__shfl_xor((int)w, d, 8);
+    if ((threadIdx.x & 7) == 0 && base < ix.nhash) ix.present_w[base >> 5] = w;
 }
 
 // scatter every kept tuple into its bucket (order fixed by the sort below)
@@ -518,6 +571,239 @@ __global__ void __launch_bounds__(64) map_strands(MapArgs a) {
     __syncthreads();
     bitonic<false>(keys, n2, lane, 64, [] { __syncthreads(); });
     emit_best(a, sidx, keys, total);
+}
+
+// ---------------------------------------------------------------------------
+// Flat tier: map_strands' work for reads of at most 64 * NR k-mers on an index
+// with 32-bit cluster ids, one wave per strand, no sort.
+//
+// What bounds the tier above on a sparse index (50 Mbp: 89 k-mers and 39 hits a
+// strand) is instruction issue, the scalar unit first (2,325 scalar and 1,027
+// vector instructions a strand: byte switches and per-stage loop control), then
+// a 128-byte line for each of the strand's bucket lookups, four in five of them
+// to empty buckets.  Here:
+//  * the strand's bases become 2-bit codes through two ballots per 64 bases,
+//    interleaved into words in LDS; a k-mer's hash is two words and one
+//    v_alignbit_b32;
+//  * a bitmap of the non-empty buckets (2 MB for k = 12: it stays in each
+//    XCD's L2) filters the lookups;
+//  * hits are listed in LDS (entry index, query offset) and their entries
+//    loaded one per lane, all at once;
+//  * clusters are counted in an LDS table by cluster id (count in the high
+//    half, by atomic add; smallest query offset in the low half): every
+//    cluster of the biggest count M has one hit whose insertion returned M,
+//    and the first max_hits of those by cluster id are wave minima.  Where M
+//    is 1 every hit is its cluster.
+// The waves are persistent and load their next strand's bases during the
+// current one.  105,000 reads of 100 bases on 50 Mbp: the kernel
+// 0.90 -> 0.35 ms.
+// ---------------------------------------------------------------------------
+constexpr int kFlatSlots = 512;  // at most kMapCap clusters: half full
+static_assert(kFlatSlots >= 2 * kMapCap, "every insertion finds its slot");
+
+// bits 0..15 of x to the even bits of the result
+__device__ __forceinline__ uint32_t spread16(uint32_t x) {
+    x = (x | (x << 8)) & 0x00FF00FFu;
+    x = (x | (x << 4)) & 0x0F0F0F0Fu;
+    x = (x | (x << 2)) & 0x33333333u;
+    return (x | (x << 1)) & 0x55555555u;
+}
+
+template <int NR>
+__global__ void __launch_bounds__(64) map_strands_flat(MapArgs a) {
+    constexpr int NB = NR + 1;                 // rounds of 64 bases (k <= 15)
+    constexpr int HPT = kMapCap / 64;          // hits per lane
+    constexpr uint32_t kEmpty = 0xFFFFFFFFu, kFresh = 0x0000FFFFu;
+    __shared__ uint32_t words[4 * NB + 2];
+    __shared__ uint32_t hidx[kMapCap];         // a hit's entry,
+    __shared__ uint16_t hoff[kMapCap];         // its query offset
+    __shared__ uint32_t tkey[kFlatSlots], tval[kFlatSlots];
+    const int lane = threadIdx.x;
+    const int n = 2 * a.rd.nreads, G = gridDim.x;
+    const int k = a.ix.k;
+    const uint32_t hmask = (uint32_t)(a.ix.nhash - 1);
+    for (int i = lane; i < kFlatSlots; i += 64) {
+        tkey[i] = kEmpty;
+        tval[i] = kFresh;
+    }
+    if (lane < 2) words[4 * NB + lane] = 0;
+    // cluster-id base of sequence lane and 64 + lane (none: past every id)
+    const uint32_t c0 = lane < a.ix.nseq ? a.ix.cid0[lane] : kEmpty;
+    const uint32_t c1 = 64 + lane < a.ix.nseq ? a.ix.cid0[64 + lane] : kEmpty;
+    // base `64 * b + lane` of a strand, as the strand reads it
+    unsigned char nb[NB];
+    int nL = 0;
+    auto fetch = [&](int s) {
+        int len = a.rd.len[s >> 1];
+        if (len < 0 || len > a.max_len) {
+            if (lane == 0) atomicOr(a.error, 2);
+            len = 0;
+        }
+        const unsigned char *src = (const unsigned char *)a.rd.seq + a.rd.off[s >> 1];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int i = b * 64 + lane;
+            nb[b] = i < len ? src[(s & 1) ? len - 1 - i : i] : 0;
+        }
+        nL = len;
+    };
+    if ((int)blockIdx.x < n) fetch(blockIdx.x);
+    for (int s = blockIdx.x; s < n; s += G) {
+        const int L = nL, nq = L - k + 1;
+        // 2-bit codes of the strand's bases, 16 to a word
+        uint32_t w0 = 0, w1 = 0;
+        char *dst = a.strand_seq ? a.strand_seq + (int64_t)s * a.qstride : nullptr;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int i = b * 64 + lane;
+            const unsigned char v = (s & 1) ? rc_byte(nb[b]) : nb[b];
+            if (dst && i < L) dst[i] = (char)v;
+            const uint32_t c = i < L ? kcode(v) : 0u;
+            const uint64_t m0 = __ballot(c & 1u), m1 = __ballot(c & 2u);
+            if ((lane >> 2) == b) {  // lane 4b + j: bases 64b + 16j ..
+                w0 = (uint32_t)(m0 >> (16 * (lane & 3))) & 0xFFFFu;
+                w1 = (uint32_t)(m1 >> (16 * (lane & 3))) & 0xFFFFu;
+            }
+        }
+        if (lane < 4 * NB) words[lane] = spread16(w0) | spread16(w1) << 1;
+        wave_sync();
+        if (s + G < n) fetch(s + G);
+        // the buckets of the strand's k-mers
+        uint32_t h[NR];
+        int2 bk[NR];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const int i = r * 64 + lane, at = i >> 4;
+            h[r] = __builtin_amdgcn_alignbit(words[at + 1], words[at], 2 * (i & 15)) & hmask;
+        }
+        if (a.ix.present) {
+            uint32_t pw[NR];
+#pragma unroll
+            for (int r = 0; r < NR; ++r) pw[r] = r * 64 + lane < nq ? a.ix.present[h[r] >> 5] : 0u;
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                bk[r] = make_int2(0, 0);
+                if ((pw[r] >> (h[r] & 31)) & 1u) bk[r] = a.ix.bucket[h[r]];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                bk[r] = make_int2(0, 0);
+                if (r * 64 + lane < nq) bk[r] = a.ix.bucket[h[r]];
+            }
+        }
+        int at[NR], total = 0;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const int incl = (int)wave_scan_add((uint32_t)bk[r].y);
+            at[r] = total + incl - bk[r].y;
+            total += __builtin_amdgcn_readlane(incl, 63);
+        }
+        if (lane == 0) a.out.nhits[s] = total;
+        if (total == 0 || total > kMapCap) {
+            if (lane == 0) {
+                if (total) {
+                    a.ovl_list[atomicAdd(a.ovl_count, 1)] = s;
+                } else {
+                    a.out.nbest[s] = 0;
+                    a.out.nbig[s] = 0;
+                }
+            }
+            continue;
+        }
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+            for (int j = 0; j < bk[r].y; ++j) {
+                hidx[at[r] + j] = (uint32_t)(bk[r].x + j);
+                hoff[at[r] + j] = (uint16_t)(r * 64 + lane);
+            }
+        wave_sync();
+        // hit u of a lane (64 * u + lane < total): its cluster id, its offset,
+        // its slot and the count its insertion made
+        uint32_t cid[HPT], off[HPT], slot[HPT], cnt[HPT], best = 0;
+#pragma unroll
+        for (int u = 0; u < HPT; ++u) {
+            const int e = u * 64 + lane;
+            cid[u] = kEmpty;
+            off[u] = 0;
+            if (e < total) {
+                off[u] = hoff[e];
+                cid[u] = a.ix.gpos[hidx[e]];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < HPT; ++u) {
+            cnt[u] = 0;
+            slot[u] = 0;
+            if (u * 64 + lane < total) {
+                cid[u] = cid[u] - off[u] + (uint32_t)kShiftBias;
+                uint32_t q = (cid[u] * 2654435761u) >> (32 - __builtin_ctz(kFlatSlots));
+                for (;;) {
+                    const uint32_t old = atomicCAS(&tkey[q], kEmpty, cid[u]);
+                    if (old == kEmpty || old == cid[u]) break;
+                    q = (q + 1) & (kFlatSlots - 1);
+                }
+                slot[u] = q;
+                cnt[u] = (atomicAdd(&tval[q], 1u << 16) >> 16) + 1;
+                best = max(best, cnt[u]);
+            }
+        }
+        best = wave_all_max(best);
+        wave_sync();
+        if (best > 1) {
+            // smallest query offset of the biggest clusters (every update of
+            // such a slot carries the same count bits)
+#pragma unroll
+            for (int u = 0; u < HPT; ++u)
+                if (u * 64 + lane < total && (tval[slot[u]] >> 16) == best)
+                    atomicMin(&tval[slot[u]], best << 16 | off[u]);
+            wave_sync();
+        }
+        // one hit for each biggest cluster
+        int nbig = 0;
+        bool rep[HPT];
+#pragma unroll
+        for (int u = 0; u < HPT; ++u) {
+            rep[u] = cnt[u] == best;
+            nbig += (int)__popcll(__ballot(rep[u]));
+            if (rep[u] && best > 1) off[u] = tval[slot[u]] & 0xFFFFu;
+        }
+        const int take = min(nbig, a.max_hits);
+        const int64_t o = (int64_t)s * a.out.stride;
+        for (int r = 0; r < take; ++r) {
+            uint32_t m = kEmpty;
+#pragma unroll
+            for (int u = 0; u < HPT; ++u)
+                if (rep[u]) m = min(m, cid[u]);
+            const uint32_t lo = wave_all_min(m);
+            // the last sequence whose cluster ids start at or below it
+            const int ref = (int)__popcll(__ballot(c0 <= lo)) + (int)__popcll(__ballot(c1 <= lo)) - 1;
+            const uint32_t base = (uint32_t)__builtin_amdgcn_readlane(
+                (int)(ref < 64 ? c0 : c1), ref & 63);
+            const int sh = (int)((int64_t)(lo - base) - kShiftBias);
+#pragma unroll
+            for (int u = 0; u < HPT; ++u)
+                if (rep[u] && cid[u] == lo) {  // cluster ids are distinct
+                    a.out.ref[o + r] = (int8_t)ref;
+                    a.out.shift[o + r] = sh;
+                    a.out.pos[o + r] = sh + (int)off[u];
+                    rep[u] = false;
+                }
+        }
+        if (lane == 0) {
+            a.out.nbest[s] = take;
+            a.out.nbig[s] = nbig;
+        }
+        // clear the slots used (every read of the table is done)
+        wave_sync();
+#pragma unroll
+        for (int u = 0; u < HPT; ++u)
+            if (u * 64 + lane < total) {
+                tkey[slot[u]] = kEmpty;
+                tval[slot[u]] = kFresh;
+            }
+        wave_sync();
+    }
 }
 
 // Strands past one tier's capacity are sorted by a workgroup of THREADS
@@ -1629,7 +1915,16 @@ hipError_t launch_map(const MapArgs &a, hipStream_t st, int mid_blocks) {
     // workgroup would still clear its LDS tables)
     const int nstr = 2 * a.rd.nreads;
     auto grid = [nstr](int g) { return dim3((unsigned)std::max(1, std::min(g, nstr))); };
-    if (!hash_first) hipLaunchKernelGGL(map_strands, dim3(2 * a.rd.nreads), dim3(64), 0, st, a);
+    if (!hash_first) {
+        const int nq = a.max_len - a.ix.k + 1;
+        // seven waves a SIMD: what the flat tier's LDS lets a CU hold
+        if (a.ix.cid_ok && nq <= 128)
+            hipLaunchKernelGGL(map_strands_flat<2>, grid(28 * 256), dim3(64), 0, st, a);
+        else if (a.ix.cid_ok && nq <= 320)
+            hipLaunchKernelGGL(map_strands_flat<5>, grid(28 * 256), dim3(64), 0, st, a);
+        else
+            hipLaunchKernelGGL(map_strands, dim3(2 * a.rd.nreads), dim3(64), 0, st, a);
+    }
     if (mid_blocks > 0) {
         if (a.ix.cid_ok && hash_first && a.max_len <= kShortRead) {
             // short reads, every strand: first the half-size table (four

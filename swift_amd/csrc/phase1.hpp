@@ -30,6 +30,8 @@ constexpr int kLongFilterCap = 18432;  // short-read strands past kHashCap: the 
 constexpr int kSmallBucket = 32;       // buckets sorted by one thread
 constexpr int kWaveBucket = 1024;      // buckets sorted by one wave in LDS
 constexpr int kScanChunk = 4096;       // hashes per scan workgroup
+constexpr int64_t kPresentHashes = (int64_t)1 << 24;  // bucket bitmaps up to 2 MB: a lookup
+                                       // then hits its XCD's 4 MB of L2
 
 // Index arrays in HBM.  Sequences are stored as the index sees them (the
 // reference's line handling applied, see the FASTA reader), back to back.
@@ -55,6 +57,10 @@ struct IndexDev {
     // cluster id is this minus its query offset plus kShiftBias, so the hash
     // tier reads 4 bytes per hit instead of the 8-byte entry
     const uint32_t *gpos;
+    // bitmap of the non-empty buckets; null when it would not pay (present_w:
+    // the array itself, for the build)
+    const uint32_t *present;
+    uint32_t *present_w;
     // 1: every base of seq is one of ACGTNacgtn (so no window can send a pair
     // to the int32 re-run for its reference bytes)
     int plain_bases;
@@ -62,8 +68,10 @@ struct IndexDev {
 
 struct IndexBuildScratch {
     int64_t *block_sum;       // [nhash / kScanChunk + 1]
+    int2 *block_stat;         // [same] largest kept count, non-empty buckets
     int64_t *total;           // [1] kept tuples
     int32_t *max_actual;      // [1]
+    int32_t *filled;          // [1] non-empty buckets
     int32_t *mid_list, *mid_count;   // buckets for the wave sort
     int32_t *big_list, *big_count;   // buckets for the block sort
     uint64_t *big_scratch;    // [big_slots * big_cap]

@@ -203,19 +203,22 @@ static int index_build(const char *bases, const int64_t *off, const int64_t *len
     if ((rc = ix->actual.alloc(4 * nh))) return rc;
     if ((rc = ix->cursor.alloc(4 * nh))) return rc;
     if ((rc = ix->bucket.alloc(8 * nh))) return rc;
+    if ((rc = ix->present.alloc(nh / 8 + 4))) return rc;
     SWIFT_HIP_TRY(hipMemset(ix->count.ptr, 0, 4 * nh));
 
     const int nblocks = (int)((ix->nhash + kScanChunk - 1) / kScanChunk);
     DevArr block_sum, small, mid_list, big_list, big_scratch;
-    if ((rc = block_sum.alloc(8 * (size_t)nblocks))) return rc;
+    if ((rc = block_sum.alloc(16 * (size_t)nblocks))) return rc;
     if ((rc = small.alloc(64))) return rc;
     SWIFT_HIP_TRY(hipMemset(small.ptr, 0, 64));
     IndexBuildScratch sc{};
     sc.block_sum = block_sum.as<int64_t>();
+    sc.block_stat = reinterpret_cast<int2 *>(sc.block_sum + nblocks);
     sc.total = small.as<int64_t>();
     sc.max_actual = small.as<int32_t>() + 2;
     sc.mid_count = small.as<int32_t>() + 3;
     sc.big_count = small.as<int32_t>() + 4;
+    sc.filled = small.as<int32_t>() + 5;
     IndexDev d = ix->dev();
     SWIFT_HIP_TRY(launch_index_build(d, ix->ntup, sc, nullptr));
     int32_t head[6];
@@ -224,6 +227,8 @@ static int index_build(const char *bases, const int64_t *off, const int64_t *len
     memcpy(&total, head, 8);
     ix->total = total;
     ix->max_actual = head[2];
+    // with half the buckets empty the bitmap saves more lines than it reads
+    ix->use_present = ix->nhash <= kPresentHashes && 2 * (int64_t)head[5] <= ix->nhash;
     if (total >= INT32_MAX) {
         set_error("%lld kept tuples: bucket starts are 32-bit", (long long)total);
         return kErrCapacity;

@@ -37,8 +37,10 @@ struct DevArr {
 struct IndexObj {
     int k = 0, thr = 0, nseq = 0, max_actual = 0;
     int64_t nhash = 0, ntup = 0, total = 0;
-    DevArr seq, seq_off, seq_len, tup0, count, start, actual, cursor, bucket, entry, cid0, gpos;
+    DevArr seq, seq_off, seq_len, tup0, count, start, actual, cursor, bucket, entry, cid0, gpos,
+        present;
     int cid_ok = 0;
+    int use_present = 0;  // the bucket bitmap pays: few buckets hold tuples
     int plain_bases = 0;  // every base one of ACGTNacgtn
     std::vector<int64_t> h_off, h_len;
     std::vector<std::string> names;
@@ -63,6 +65,8 @@ struct IndexObj {
         d.cid_ok = cid_ok;
         d.plain_bases = plain_bases;
         d.gpos = gpos.as<const uint32_t>();
+        d.present_w = present.as<uint32_t>();
+        d.present = use_present ? d.present_w : nullptr;
         return d;
     }
 };
