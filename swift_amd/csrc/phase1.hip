@@ -121,6 +121,14 @@ __device__ __forceinline__ int next_pow2(int n) {
     return n2;
 }
 
+// bucket of a hash: (first entry, kept count), from two neighbours of the
+// prefix array (one 8-byte load)
+__device__ __forceinline__ int2 bucket_of(const IndexDev &ix, uint32_t h) {
+    typedef uint32_t pair __attribute__((ext_vector_type(2), aligned(4)));
+    const pair p = *reinterpret_cast<const pair *>(ix.first + h);
+    return make_int2((int)p.x, (int)(p.y - p.x));
+}
+
 // ---------------------------------------------------------------------------
 // Index build
 // ---------------------------------------------------------------------------
@@ -225,8 +233,8 @@ __global__ void __launch_bounds__(1024) idx_scan_sums(IndexBuildScratch s, int n
     if (threadIdx.x == 1023) *s.total = part[1023];
 }
 
-// start = 1 + exclusive prefix of the kept counts (0 for empty or dropped
-// hashes), actual = kept count (src/lookupTable5.cu:199-208)
+// first = 1 + exclusive prefix of the kept counts, which are its differences
+// (src/lookupTable5.cu:199-208), and the bitmap of the non-empty buckets
 __global__ void __launch_bounds__(1024) idx_scan_apply(IndexDev ix, IndexBuildScratch s) {
     __shared__ int64_t part[1024];
     constexpr int per = kScanChunk / 1024;
@@ -251,14 +259,9 @@ __global__ void __launch_bounds__(1024) idx_scan_apply(IndexDev ix, IndexBuildSc
 #pragma unroll
     for (int i = 0; i < per; ++i) {
         int64_t h = base + i;
-        if (h < ix.nhash) {
-            int32_t st = loc[i] ? (int32_t)(run + 1) : 0;
-            ix.start[h] = st;
-            ix.actual[h] = loc[i];
-            ix.bucket[h] = make_int2(st, loc[i]);
-            ix.cursor[h] = 0;
-        }
+        if (h < ix.nhash) ix.first_w[h] = (uint32_t)(run + 1);
         run += loc[i];
+        if (h == ix.nhash - 1) ix.first_w[h + 1] = (uint32_t)(run + 1);
     }
     // this thread's `per` hashes of the non-empty buckets' bitmap, 32 to a word
     static_assert(per == 4, "eight threads to a word");
@@ -271,61 +274,88 @@ __global__ void __launch_bounds__(1024) idx_scan_apply(IndexDev ix, IndexBuildSc
     if ((threadIdx.x & 7) == 0 && base < ix.nhash) ix.present_w[base >> 5] = w;
 }
 
-// scatter every kept tuple into its bucket (order fixed by the sort below)
-__global__ void __launch_bounds__(256) idx_fill(IndexDev ix, int64_t ntup) {
+// Scatter every kept tuple into its bucket (order fixed by the sort below), the
+// count of each kept hash counted down as the cursor: as its 4-byte global
+// position where cluster ids fit 32 bits, else as its 8-byte entry.
+__global__ void __launch_bounds__(256) idx_fill(IndexDev ix, int64_t ntup, uint32_t *gpos) {
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < ntup;
          t += (int64_t)gridDim.x * blockDim.x) {
         int s = seq_of_tuple(ix.tup0, ix.nseq, t);
         int64_t pos = (t - ix.tup0[s]) * ix.k;
         uint32_t h = kmer_hash((const unsigned char *)ix.seq + ix.seq_off[s] + pos, ix.k);
-        if (ix.actual[h] == 0) continue;
-        int slot = ix.start[h] + atomicAdd(&ix.cursor[h], 1);
-        ix.entry[slot] = ((uint64_t)(uint32_t)s << 32) | (uint32_t)pos;
+        const int2 b = bucket_of(ix, h);
+        if (b.y == 0) continue;
+        const int slot = b.x + atomicSub(&ix.count[h], 1) - 1;
+        if (gpos) gpos[slot] = ix.cid0[s] + (uint32_t)pos;
+        else ix.entry[slot] = ((uint64_t)(uint32_t)s << 32) | (uint32_t)pos;
     }
 }
 
 // Reverse file order within a bucket (src/lookupTable5.cu:219-229) is
-// descending (refIdx, refPos).  Buckets of <= kSmallBucket entries are sorted
-// by one thread in registers; larger ones are listed for the wave sort or
-// the workgroup sort.
-__global__ void __launch_bounds__(256) idx_sort_small(IndexDev ix, IndexBuildScratch s) {
-    int64_t h = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (h >= ix.nhash) return;
-    const int a = ix.actual[h];
-    if (a < 2) return;
-    if (a > kSmallBucket) {
-        if (a <= kWaveBucket) s.mid_list[atomicAdd(s.mid_count, 1)] = (int32_t)h;
-        else s.big_list[atomicAdd(s.big_count, 1)] = (int32_t)h;
-        return;
+// descending (refIdx, refPos), i.e. descending keys of either form.  Buckets of
+// <= kSmallBucket are sorted by one thread in registers, by an odd-even merge
+// network as large as the wave's largest bucket needs (most waves' is 2 to 4 on
+// a sparse index); larger ones are listed for the wave sort or the workgroup
+// sort.  50 Mbp, 4.2M tuples in 16.8M buckets: 1.28 ms (32-key insertion network
+// on 8-byte entries in every wave) -> 0.053; what bounds it now is the read of
+// the prefix array.
+template <int I, int J, class K> __device__ __forceinline__ void compare_desc(K *v) {
+    const K x = v[I], y = v[J];
+    v[I] = x > y ? x : y;
+    v[J] = x > y ? y : x;
+}
+template <int N, int P, int Q, int I, class K> __device__ __forceinline__ void merge_pass(K *v) {
+    // Batcher's odd-even merge: pass (P, Q), comparators (i, i + Q)
+    if constexpr (I + Q < N) {
+        if constexpr (I >= Q % P && (I - Q % P) % (2 * Q) < Q && I / (2 * P) == (I + Q) / (2 * P))
+            compare_desc<I, I + Q>(v);
+        merge_pass<N, P, Q, I + 1>(v);
     }
-    uint64_t *e = ix.entry + ix.start[h];
-    uint64_t v[kSmallBucket];
+}
+template <int N, int P, int Q, class K> __device__ __forceinline__ void merge_net(K *v) {
+    merge_pass<N, P, Q, 0>(v);
+    if constexpr (Q > 1) merge_net<N, P, Q / 2>(v);
+    else if constexpr (2 * P < N) merge_net<N, 2 * P, 2 * P>(v);
+}
+template <int N, class K> __device__ __forceinline__ void sort_bucket(K *e, int a) {
+    K v[N];
+    // padding zeros sort last; a real key equal to 0 is indistinguishable
 #pragma unroll
-    for (int i = 0; i < kSmallBucket; ++i) v[i] = i < a ? e[i] : 0;
-    // padding zeros sort last; a real entry equal to 0 is indistinguishable
+    for (int i = 0; i < N; ++i) v[i] = i < a ? e[i] : 0;
+    merge_net<N, 1, 1>(v);
 #pragma unroll
-    for (int i = 1; i < kSmallBucket; ++i) {
-#pragma unroll
-        for (int j = i; j > 0; --j) {
-            uint64_t x = v[j - 1], y = v[j];
-            bool sw = y > x;
-            v[j - 1] = sw ? y : x;
-            v[j] = sw ? x : y;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < kSmallBucket; ++i)
+    for (int i = 0; i < N; ++i)
         if (i < a) e[i] = v[i];
 }
 
+template <class K>
+__global__ void __launch_bounds__(256) idx_sort_small(IndexDev ix, IndexBuildScratch s, K *keys) {
+    const int64_t h = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    int2 b = h < ix.nhash ? bucket_of(ix, (uint32_t)h) : make_int2(0, 0);
+    if (b.y > kSmallBucket) {
+        if (b.y <= kWaveBucket) s.mid_list[atomicAdd(s.mid_count, 1)] = (int32_t)h;
+        else s.big_list[atomicAdd(s.big_count, 1)] = (int32_t)h;
+        b.y = 0;
+    }
+    const uint32_t most = wave_all_max((uint32_t)b.y);
+    K *e = keys + b.x;
+    if (most < 2) return;
+    if (most <= 2) sort_bucket<2>(e, b.y);
+    else if (most <= 4) sort_bucket<4>(e, b.y);
+    else if (most <= 8) sort_bucket<8>(e, b.y);
+    else if (most <= 16) sort_bucket<16>(e, b.y);
+    else sort_bucket<kSmallBucket>(e, b.y);
+}
+
 // one wave per listed bucket, keys in LDS
-__global__ void __launch_bounds__(64) idx_sort_mid(IndexDev ix, IndexBuildScratch s) {
-    __shared__ uint64_t key[kWaveBucket];
+template <class K>
+__global__ void __launch_bounds__(64) idx_sort_mid(IndexDev ix, IndexBuildScratch s, K *keys) {
+    __shared__ K key[kWaveBucket];
     const int n = *s.mid_count;
     for (int it = blockIdx.x; it < n; it += gridDim.x) {
-        const int h = s.mid_list[it];
-        const int a = ix.actual[h];
-        uint64_t *e = ix.entry + ix.start[h];
+        const int2 b = bucket_of(ix, (uint32_t)s.mid_list[it]);
+        const int a = b.y;
+        K *e = keys + b.x;
         const int n2 = next_pow2(a);
         for (int i = threadIdx.x; i < n2; i += 64) key[i] = i < a ? e[i] : 0;
         __syncthreads();
@@ -336,19 +366,43 @@ __global__ void __launch_bounds__(64) idx_sort_mid(IndexDev ix, IndexBuildScratc
 }
 
 // one workgroup per listed bucket, keys in a global scratch slot
-__global__ void __launch_bounds__(256) idx_sort_big(IndexDev ix, IndexBuildScratch s) {
+template <class K>
+__global__ void __launch_bounds__(256) idx_sort_big(IndexDev ix, IndexBuildScratch s, K *keys) {
     const int n = *s.big_count;
-    uint64_t *key = s.big_scratch + (int64_t)blockIdx.x * s.big_cap;
+    K *key = reinterpret_cast<K *>(s.big_scratch) + (int64_t)blockIdx.x * s.big_cap;
     for (int it = blockIdx.x; it < n; it += gridDim.x) {
-        const int h = s.big_list[it];
-        const int a = ix.actual[h];
-        uint64_t *e = ix.entry + ix.start[h];
+        const int2 b = bucket_of(ix, (uint32_t)s.big_list[it]);
+        const int a = b.y;
+        K *e = keys + b.x;
         const int n2 = next_pow2(a);
         for (int i = threadIdx.x; i < n2; i += 256) key[i] = i < a ? e[i] : 0;
         __syncthreads();
         bitonic<true>(key, n2, threadIdx.x, 256, [] { __syncthreads(); });
         for (int i = threadIdx.x; i < a; i += 256) e[i] = key[i];
         __syncthreads();
+    }
+}
+
+// entries from the sorted global positions: the last sequence whose cluster
+// ids start at or below one holds it
+__global__ void __launch_bounds__(256) idx_entries(IndexDev ix, int64_t total, uint32_t *gpos) {
+    __shared__ uint32_t c0[kMaxIndexSeqs];
+    for (int i = threadIdx.x; i < ix.nseq; i += 256) c0[i] = ix.cid0[i];
+    __syncthreads();
+    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i <= total; i += (int64_t)gridDim.x * 256) {
+        if (i == 0) {
+            gpos[0] = 0xFFFFFFFFu;
+            ix.entry[0] = ~0ull;  // sentinel (-1, -1)
+            continue;
+        }
+        const uint32_t g = gpos[i];
+        int lo = 0, hi = ix.nseq - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (c0[mid] <= g) lo = mid;
+            else hi = mid - 1;
+        }
+        ix.entry[i] = ((uint64_t)(uint32_t)lo << 32) | (g - c0[lo]);
     }
 }
 
@@ -414,7 +468,7 @@ __device__ int gather_hits(const IndexDev &ix, const unsigned char *qb, int nq, 
         const int i = b + lane;
         int cnt = 0, st = 0;
         if (i < nq) {
-            int2 bk = ix.bucket[kmer_hash(qb + i, ix.k)];
+            int2 bk = bucket_of(ix, kmer_hash(qb + i, ix.k));
             st = bk.x;
             cnt = bk.y;
         }
@@ -457,7 +511,7 @@ __device__ int gather_hits_flat(const IndexDev &ix, const unsigned char *qb, int
         cnt[r] = 0;
         st[r] = 0;
         if (i < nq) {
-            const int2 bk = ix.bucket[kmer_hash(qb + i, ix.k)];
+            const int2 bk = bucket_of(ix, kmer_hash(qb + i, ix.k));
             st[r] = bk.x;
             cnt[r] = bk.y;
         }
@@ -683,13 +737,13 @@ __global__ void __launch_bounds__(64) map_strands_flat(MapArgs a) {
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 bk[r] = make_int2(0, 0);
-                if ((pw[r] >> (h[r] & 31)) & 1u) bk[r] = a.ix.bucket[h[r]];
+                if ((pw[r] >> (h[r] & 31)) & 1u) bk[r] = bucket_of(a.ix, h[r]);
             }
         } else {
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 bk[r] = make_int2(0, 0);
-                if (r * 64 + lane < nq) bk[r] = a.ix.bucket[h[r]];
+                if (r * 64 + lane < nq) bk[r] = bucket_of(a.ix, h[r]);
             }
         }
         int at[NR], total = 0;
@@ -836,7 +890,7 @@ map_strands_wg(MapArgs a, const int32_t *list, const int32_t *list_count, int32_
             c[u] = 0;
             st[u] = 0;
             if (o < nq) {
-                const int2 b = a.ix.bucket[kmer_hash(qb + o, a.ix.k)];
+                const int2 b = bucket_of(a.ix, kmer_hash(qb + o, a.ix.k));
                 st[u] = b.x;
                 c[u] = b.y;
             }
@@ -1003,7 +1057,7 @@ map_strands_hash(MapArgs a, const int32_t *list, const int32_t *list_count, int3
             c[u] = 0;
             st[u] = 0;
             if (o < nq) {
-                const int2 b = a.ix.bucket[kmer_hash(qb + o, a.ix.k)];
+                const int2 b = bucket_of(a.ix, kmer_hash(qb + o, a.ix.k));
                 st[u] = b.x;
                 c[u] = b.y;
             }
@@ -1324,7 +1378,7 @@ map_strands_filter(MapArgs a, const int32_t *src, const int32_t *src_count, int3
             c[u] = 0;
             st[u] = 0;
             if (o < nq) {
-                const int2 b = a.ix.bucket[kmer_hash(qb + o, a.ix.k)];
+                const int2 b = bucket_of(a.ix, kmer_hash(qb + o, a.ix.k));
                 st[u] = b.x;
                 c[u] = b.y;
             }
@@ -1851,26 +1905,27 @@ hipError_t launch_index_build(const IndexDev &ix, int64_t ntup, const IndexBuild
     return hipGetLastError();
 }
 
-__global__ void __launch_bounds__(256) idx_gpos(IndexDev ix, int64_t total, uint32_t *gpos) {
-    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i <= total; i += (int64_t)gridDim.x * 256) {
-        const uint64_t e = ix.entry[i];
-        gpos[i] = i == 0 ? 0xFFFFFFFFu : ix.cid0[(int)(e >> 32)] + (uint32_t)e;
-    }
-}
-
-hipError_t launch_index_gpos(const IndexDev &ix, int64_t total, uint32_t *gpos, hipStream_t st) {
-    hipLaunchKernelGGL(idx_gpos, dim3(tuple_grid(total + 1)), dim3(256), 0, st, ix, total, gpos);
-    return hipGetLastError();
-}
-
-hipError_t launch_index_fill(const IndexDev &ix, int64_t ntup, const IndexBuildScratch &s,
-                             hipStream_t st) {
-    if (ntup > 0) hipLaunchKernelGGL(idx_fill, dim3(tuple_grid(ntup)), dim3(256), 0, st, ix, ntup);
-    hipLaunchKernelGGL(idx_sort_small, dim3((unsigned)((ix.nhash + 255) / 256)), dim3(256), 0, st,
-                       ix, s);
-    hipLaunchKernelGGL(idx_sort_mid, dim3(8192), dim3(64), 0, st, ix, s);
+template <class K>
+static void launch_index_sort(const IndexDev &ix, const IndexBuildScratch &s, K *keys,
+                              hipStream_t st) {
+    hipLaunchKernelGGL(idx_sort_small<K>, dim3((unsigned)((ix.nhash + 255) / 256)), dim3(256), 0,
+                       st, ix, s, keys);
+    hipLaunchKernelGGL(idx_sort_mid<K>, dim3(8192), dim3(64), 0, st, ix, s, keys);
     if (s.big_slots > 0)
-        hipLaunchKernelGGL(idx_sort_big, dim3(s.big_slots), dim3(256), 0, st, ix, s);
+        hipLaunchKernelGGL(idx_sort_big<K>, dim3(s.big_slots), dim3(256), 0, st, ix, s, keys);
+}
+
+hipError_t launch_index_fill(const IndexDev &ix, int64_t ntup, int64_t total, uint32_t *gpos,
+                             const IndexBuildScratch &s, hipStream_t st) {
+    if (ntup > 0)
+        hipLaunchKernelGGL(idx_fill, dim3(tuple_grid(ntup)), dim3(256), 0, st, ix, ntup, gpos);
+    if (gpos) {
+        launch_index_sort(ix, s, gpos, st);
+        hipLaunchKernelGGL(idx_entries, dim3(std::min(tuple_grid(total + 1), 4096)), dim3(256), 0,
+                           st, ix, total, gpos);
+    } else {
+        launch_index_sort(ix, s, ix.entry, st);
+    }
     return hipGetLastError();
 }
 

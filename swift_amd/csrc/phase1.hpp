@@ -42,11 +42,13 @@ struct IndexDev {
     const int64_t *tup0;      // [nseq] first tuple number of sequence s
     int nseq, k, thr;
     int64_t nhash;            // 4^k
-    int32_t *count;           // [nhash] occurrences (_numRepeatsPerTuple)
-    int32_t *start;           // [nhash] 1-based bucket start, 0 if empty/dropped
-    int32_t *actual;          // [nhash] kept occurrences (0 if count > thr)
-    int32_t *cursor;          // [nhash] fill cursor
-    int2 *bucket;             // [nhash] (start, actual) for the mapper
+    // [nhash] occurrences (_numRepeatsPerTuple) of the dropped hashes; the
+    // fill counts the kept ones' down to 0
+    int32_t *count;
+    // [nhash + 1] 1-based start of each hash's bucket; its kept count is the
+    // difference to the next (empty: 0).  first_w: the array itself
+    const uint32_t *first;
+    uint32_t *first_w;
     uint64_t *entry;          // [total + 1] refIdx << 32 | refPos, [0] sentinel
     // 32-bit cluster ids: cid = cid0[refIdx] + shift + kShiftBias, with
     // cid0[s] = sum over r < s of (len[r] + 2 * kShiftBias); increasing in
@@ -135,9 +137,9 @@ struct PairsDev {
 
 hipError_t launch_index_build(const IndexDev &ix, int64_t ntup, const IndexBuildScratch &s,
                               hipStream_t st);
-hipError_t launch_index_gpos(const IndexDev &ix, int64_t total, uint32_t *gpos, hipStream_t st);
-hipError_t launch_index_fill(const IndexDev &ix, int64_t ntup, const IndexBuildScratch &s,
-                             hipStream_t st);
+// gpos: filled and sorted with the entries when cluster ids fit 32 bits, else null
+hipError_t launch_index_fill(const IndexDev &ix, int64_t ntup, int64_t total, uint32_t *gpos,
+                             const IndexBuildScratch &s, hipStream_t st);
 // mid_blocks: persistent workgroups of map_strands_mid (0 when no strand can
 // pass kMapCap hits)
 hipError_t launch_map(const MapArgs &a, hipStream_t st, int mid_blocks);

@@ -161,10 +161,16 @@ static int index_build(const char *bases, const int64_t *off, const int64_t *len
     }
     ix->ntup = nt;
     if ((rc = ix->seq.alloc((size_t)nb + 64))) return rc;
-    for (int s = 0; s < nseq; ++s)
-        if (len[s] > 0)
-            SWIFT_HIP_TRY(hipMemcpy(ix->seq.as<char>() + ix->h_off[s], bases + off[s], (size_t)len[s],
+    // sequences that follow one another in the source go in one copy
+    for (int s = 0; s < nseq;) {
+        int e = s + 1;
+        int64_t n = len[s];
+        while (e < nseq && off[e] == off[s] + n) n += len[e++];
+        if (n > 0)
+            SWIFT_HIP_TRY(hipMemcpy(ix->seq.as<char>() + ix->h_off[s], bases + off[s], (size_t)n,
                                     hipMemcpyHostToDevice));
+        s = e;
+    }
     {
         // ACGTN bases only? (then no alignment window can need the int32
         // re-run for its reference bytes)
@@ -199,10 +205,7 @@ static int index_build(const char *bases, const int64_t *off, const int64_t *len
     }
     const size_t nh = (size_t)ix->nhash;
     if ((rc = ix->count.alloc(4 * nh))) return rc;
-    if ((rc = ix->start.alloc(4 * nh))) return rc;
-    if ((rc = ix->actual.alloc(4 * nh))) return rc;
-    if ((rc = ix->cursor.alloc(4 * nh))) return rc;
-    if ((rc = ix->bucket.alloc(8 * nh))) return rc;
+    if ((rc = ix->first.alloc(4 * (nh + 1)))) return rc;
     if ((rc = ix->present.alloc(nh / 8 + 4))) return rc;
     SWIFT_HIP_TRY(hipMemset(ix->count.ptr, 0, 4 * nh));
 
@@ -234,7 +237,12 @@ static int index_build(const char *bases, const int64_t *off, const int64_t *len
         return kErrCapacity;
     }
     if ((rc = ix->entry.alloc(8 * (size_t)(total + 1)))) return rc;
-    SWIFT_HIP_TRY(hipMemset(ix->entry.ptr, 0xFF, 8));  // sentinel (-1, -1)
+    if (ix->cid_ok) {
+        // the hash tiers' 4-byte form of the entries, which the build sorts
+        if ((rc = ix->gpos.alloc(4 * (size_t)(total + 1)))) return rc;
+    } else {
+        SWIFT_HIP_TRY(hipMemset(ix->entry.ptr, 0xFF, 8));  // sentinel (-1, -1)
+    }
     const int64_t nlist = total / (kSmallBucket + 1) + 1;
     if ((rc = mid_list.alloc(4 * (size_t)nlist))) return rc;
     if ((rc = big_list.alloc(4 * (size_t)nlist))) return rc;
@@ -248,12 +256,8 @@ static int index_build(const char *bases, const int64_t *off, const int64_t *len
         sc.big_scratch = big_scratch.as<uint64_t>();
     }
     d = ix->dev();
-    SWIFT_HIP_TRY(launch_index_fill(d, ix->ntup, sc, nullptr));
-    if (ix->cid_ok) {
-        // the hash tier's 4-byte form of the (now ordered) entries
-        if ((rc = ix->gpos.alloc(4 * (size_t)(total + 1)))) return rc;
-        SWIFT_HIP_TRY(launch_index_gpos(d, total, ix->gpos.as<uint32_t>(), nullptr));
-    }
+    SWIFT_HIP_TRY(launch_index_fill(d, ix->ntup, total,
+                                    ix->cid_ok ? ix->gpos.as<uint32_t>() : nullptr, sc, nullptr));
     SWIFT_HIP_TRY(hipDeviceSynchronize());
     return kOk;
 }
@@ -261,9 +265,17 @@ static int index_build(const char *bases, const int64_t *off, const int64_t *len
 static int index_export(const IndexObj &ix, int32_t *start, int32_t *count, int32_t *actual,
                         int8_t *ref_idx, int32_t *ref_pos) {
     const size_t nh = (size_t)ix.nhash;
-    if (start) SWIFT_HIP_TRY(hipMemcpy(start, ix.start.ptr, 4 * nh, hipMemcpyDeviceToHost));
-    if (count) SWIFT_HIP_TRY(hipMemcpy(count, ix.count.ptr, 4 * nh, hipMemcpyDeviceToHost));
-    if (actual) SWIFT_HIP_TRY(hipMemcpy(actual, ix.actual.ptr, 4 * nh, hipMemcpyDeviceToHost));
+    if (start || count || actual) {
+        std::vector<uint32_t> first(nh + 1);
+        SWIFT_HIP_TRY(hipMemcpy(first.data(), ix.first.ptr, 4 * (nh + 1), hipMemcpyDeviceToHost));
+        if (count) SWIFT_HIP_TRY(hipMemcpy(count, ix.count.ptr, 4 * nh, hipMemcpyDeviceToHost));
+        for (size_t h = 0; h < nh; ++h) {
+            const int32_t n = (int32_t)(first[h + 1] - first[h]);
+            if (start) start[h] = n ? (int32_t)first[h] : 0;
+            if (actual) actual[h] = n;
+            if (count && n) count[h] = n;
+        }
+    }
     if (ref_idx || ref_pos) {
         std::vector<uint64_t> e((size_t)ix.total + 1);
         SWIFT_HIP_TRY(hipMemcpy(e.data(), ix.entry.ptr, 8 * e.size(), hipMemcpyDeviceToHost));

@@ -37,8 +37,7 @@ struct DevArr {
 struct IndexObj {
     int k = 0, thr = 0, nseq = 0, max_actual = 0;
     int64_t nhash = 0, ntup = 0, total = 0;
-    DevArr seq, seq_off, seq_len, tup0, count, start, actual, cursor, bucket, entry, cid0, gpos,
-        present;
+    DevArr seq, seq_off, seq_len, tup0, count, first, entry, cid0, gpos, present;
     int cid_ok = 0;
     int use_present = 0;  // the bucket bitmap pays: few buckets hold tuples
     int plain_bases = 0;  // every base one of ACGTNacgtn
@@ -56,10 +55,7 @@ struct IndexObj {
         d.thr = thr;
         d.nhash = nhash;
         d.count = count.as<int32_t>();
-        d.start = start.as<int32_t>();
-        d.actual = actual.as<int32_t>();
-        d.cursor = cursor.as<int32_t>();
-        d.bucket = bucket.as<int2>();
+        d.first = d.first_w = first.as<uint32_t>();
         d.entry = entry.as<uint64_t>();
         d.cid0 = cid0.as<const uint32_t>();
         d.cid_ok = cid_ok;

@@ -62,3 +62,22 @@ def test_flat_hit_capacity(S, orc, copies):
     want = orc.Index(seqs, k, 1000)
     assert want.map_query(unit, 3, orc.TIE_FIRST)[2] >= 8 * copies
     check_strands(want, reads, got, 3, orc)
+
+
+def test_index_bucket_sizes(S, orc):
+    """Buckets of every size a sort network takes, and on both sides of the
+    one-thread, one-wave and workgroup sorts, spread over three sequences."""
+    rnd = random.Random(9)
+    k = 8
+    sizes = list(range(1, 41)) + [63, 64, 65, 1023, 1024, 1025, 2049]
+    kmers = rnd.sample(range(4 ** k), len(sizes))
+    grid = [m for m, n in zip(kmers, sizes) for _ in range(n)]
+    rnd.shuffle(grid)
+    text = ["".join("ACGT"[(m >> (2 * i)) & 3] for i in range(k)) for m in grid]
+    cut = len(text) // 3
+    seqs = ["".join(text[a:b]).encode() for a, b in ((0, cut), (cut, 2 * cut), (2 * cut, None))]
+    for thr in (5000, 33):
+        got = S.Index.from_sequences(seqs, k, thr).arrays()
+        want = orc.Index(seqs, k, thr).arrays()
+        for key in ("start", "count", "actual", "refIdx", "refPos"):
+            assert (got[key] == want[key]).all(), (thr, key)
