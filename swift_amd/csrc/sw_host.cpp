@@ -433,8 +433,8 @@ int sw_batch_check_in(Workspace *w, hipStream_t st) {
 
 // A small call as one kernel (sw_small.hip).  *done: 0 when a pair was longer
 // than the call said and the general path has to run.
-static int batch_run_small(Workspace &w, const BatchIO &io, const KeyConsts &kc, uint32_t h_limit,
-                           hipStream_t st, bool final_sync, int *done) {
+static int batch_run_small(Workspace &w, const BatchIO &io, SweepForm form, const KeyConsts &kc,
+                           uint32_t h_limit, hipStream_t st, bool final_sync, int *done) {
     const int n = io.npairs;
     SmallArgs a{};
     a.qseq = io.qseq;
@@ -447,6 +447,7 @@ static int batch_run_small(Workspace &w, const BatchIO &io, const KeyConsts &kc,
     a.ppw = n <= kSmallSingles ? 1 : 2;
     a.maxq = std::max(io.maxq, 1);
     a.maxr = std::max(io.maxr, 1);
+    a.form = form;
     a.kc = kc;
     a.h_limit = h_limit;
     a.wave_words = small_wave_words(a.maxr);
@@ -562,21 +563,17 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     // at most pos per cell, so a pair with any larger cell has one in
     // [2048 - pos, 2047] whose key is exact.
     uint32_t h_limit = (uint32_t)std::min(32767 - (4 * pos + 3) - 4, 4 * (2048 - pos));
-    // The lean sweeps: with their lower limit the same holds for keys 32H + 31
-    // + 32 * match below 0x7C00 (match <= 30).  Taken where no pair within
-    // maxq reaches it (larger scores would be re-run in int32 lanes); 32-bit
-    // lanes have no such limit.
-    const bool lean32 = lean_scoring(sc);
-    const uint32_t lean_limit = 4u * (uint32_t)(kLeanScoreLimit - 2 * pos);
-    const bool lean16 = lean32 && (int64_t)io.maxq * pos * 4 < (int64_t)lean_limit;
-    if (lean16) h_limit = lean_limit;
+    const bool lean32 = lean_scoring(sc);  // 32-bit lanes have no limit
+    const SweepForm form16 = packed_form(sc, io.maxq);
+    if (form16 != kGeneralForm) h_limit = 4u * (uint32_t)lean_limit(form16, sc.match);
 
     // a small call in one launch, unless row classes are asked for (coarse
     // ones below kCoarseTinyPairs are this form)
-    if (lean16 && !force32 && (cmode < 0 || (cmode == 1 && n < kCoarseTinyPairs)) &&
+    if (form16 != kGeneralForm && !force32 && (cmode < 0 || (cmode == 1 && n < kCoarseTinyPairs)) &&
         small_call(n, io.maxq, io.sparse)) {
         int done = 0;
-        if ((rc = batch_run_small(w, io, kc16, h_limit, st, sync_sizes && final_sync, &done)) ||
+        if ((rc = batch_run_small(w, io, form16, kc16, h_limit, st, sync_sizes && final_sync,
+                                  &done)) ||
             done)
             return rc;
         w.stats = BatchStats{};
@@ -742,7 +739,7 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
             hipStream_t s2 = nside ? w.side[lane_of[seg]] : st;
             const int wpc = w.waves_per_cu >= 0 ? w.waves_per_cu : tuning().waves_per_cu;
             const bool wseg = t.wide && seg == 0;
-            b.lean = cls == 0 ? lean16 && !wseg : lean32;
+            b.form = cls == 0 ? (wseg ? kGeneralForm : form16) : lean32 ? kLean : kGeneralForm;
             const int ntk = seg_host ? seg_host[seg + 1] - seg_host[seg] : 0;
             if (wseg)
                 SWIFT_HIP_TRY(launch_batch_wide(b, w.cu_count, ntk, s2));

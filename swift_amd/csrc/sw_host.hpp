@@ -16,6 +16,7 @@ struct TaskArgs;
 struct PlainPlan {
     enum Route { kGeneral, kPacked, kWave } route;
     int qlen, rlen, move_words;
+    int form;                     // of the packed sweep (SweepForm)
     int wave_rows, packed_rows;   // rows a lane of the whole-wave and the packed sweeps
     int64_t wave_words;           // trace of a pair swept by a whole wave
     int64_t task_words;           // trace of eight packed pairs

@@ -49,9 +49,11 @@ template <int G> constexpr int wave_lds_words() { return G + 64 / G * group_lds_
 
 // One wave task: 64 / G groups of G lanes (G = 16: 4 groups; G = 64, the
 // wide form: one); PK -> 2 pairs per group (halves).
-template <int G, int R, bool PK, bool LEAN>
+template <int G, int R, bool PK, int FORM>
 __device__ __forceinline__ void run_task(const BatchArgs &a, const Task &tk, uint32_t *lds) {
-    using S = std::conditional_t<LEAN, Lean<G, R, PK>, Sweep<G, R, PK, PK ? kOneHot : kBytes>>;
+    constexpr bool LEAN = FORM != kGeneralForm;
+    using S = std::conditional_t<LEAN, Lean<G, R, PK, FORM>,
+                                 Sweep<G, R, PK, PK ? kOneHot : kBytes>>;
     constexpr int PPG = PK ? 2 : 1;  // pairs per group
     constexpr int NG = 64 / G;       // groups per wave
     constexpr int TAIL = G + 2;      // padding columns after the last
@@ -414,9 +416,9 @@ __host__ __device__ constexpr int batch_waves_per_eu(int R, bool pk, bool lean) 
                 : (R <= 10 ? 5 : R <= 16 ? 4 : 3);
 }
 
-template <int R, bool PK, bool LEAN>
+template <int R, bool PK, int FORM>
 __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(batch_waves_per_eu(R, PK, LEAN))))
+__attribute__((amdgpu_waves_per_eu(batch_waves_per_eu(R, PK, FORM != kGeneralForm))))
 sw_batch_kernel(BatchArgs a) {
     __shared__ uint32_t lds[4][wave_lds_words<kBatchG>()];
     const int wave = threadIdx.x >> 6;
@@ -428,7 +430,7 @@ sw_batch_kernel(BatchArgs a) {
         tid = __builtin_amdgcn_readfirstlane(__shfl(tid, 0, 64)) + lo;
         if (tid >= hi) break;
         const Task tk = a.tasks[tid];
-        run_task<kBatchG, R, PK, LEAN>(a, tk, lds[wave]);
+        run_task<kBatchG, R, PK, FORM>(a, tk, lds[wave]);
     }
 }
 
@@ -450,7 +452,7 @@ __global__ void __launch_bounds__(256) sw_batch_wide_kernel(BatchArgs a) {
         tid = __builtin_amdgcn_readfirstlane(__shfl(tid, 0, 64)) + lo;
         if (tid >= hi) break;
         const Task tk = a.tasks[tid];
-        run_task<kWideG, R, true, false>(a, tk, lds[wave]);
+        run_task<kWideG, R, true, kGeneralForm>(a, tk, lds[wave]);
     }
 }
 
@@ -854,23 +856,23 @@ hipError_t launch_batch_wide(const BatchArgs &ba, int cu_count, int max_tasks, h
     return hipGetLastError();
 }
 
-template <int R, bool PK, bool LEAN>
+template <int R, bool PK, int FORM>
 static void launch_class(const BatchArgs &ba, int cu_count, int waves_per_cu, int max_tasks,
                          hipStream_t st) {
     static int blocks = -1;  // one per row class, lane width and form
-    auto k = sw_batch_kernel<R, PK, LEAN>;
+    auto k = sw_batch_kernel<R, PK, FORM>;
     hipLaunchKernelGGL(k, dim3(full_grid(k, blocks, cu_count, waves_per_cu, max_tasks)), dim3(256),
                        0, st, ba);
 }
 
-template <bool LEAN>
+template <int FORM>
 static hipError_t launch_rows(const BatchArgs &ba, bool int16, int rows, int cu_count,
                               int waves_per_cu, int max_tasks, hipStream_t st) {
     if (int16) {
         switch (rows) {
 #define SWIFT_L16(RR)                                                        \
     case RR:                                                                 \
-        launch_class<RR, true, LEAN>(ba, cu_count, waves_per_cu, max_tasks, st); \
+        launch_class<RR, true, FORM>(ba, cu_count, waves_per_cu, max_tasks, st); \
         break;
             SWIFT_R16_CASES(SWIFT_L16)
 #undef SWIFT_L16
@@ -880,7 +882,7 @@ static hipError_t launch_rows(const BatchArgs &ba, bool int16, int rows, int cu_
         switch (rows) {
 #define SWIFT_L32(RR)                                                         \
     case RR:                                                                  \
-        launch_class<RR, false, LEAN>(ba, cu_count, waves_per_cu, max_tasks, st); \
+        launch_class<RR, false, FORM == kLeanWide ? kLean : FORM>(ba, cu_count, waves_per_cu, max_tasks, st); \
         break;
             SWIFT_R32_CASES(SWIFT_L32)
 #undef SWIFT_L32
@@ -892,8 +894,13 @@ static hipError_t launch_rows(const BatchArgs &ba, bool int16, int rows, int cu_
 
 hipError_t launch_batch(const BatchArgs &ba, bool int16, int rows, int cu_count, int waves_per_cu,
                         int max_tasks, hipStream_t st) {
-    return ba.lean ? launch_rows<true>(ba, int16, rows, cu_count, waves_per_cu, max_tasks, st)
-                   : launch_rows<false>(ba, int16, rows, cu_count, waves_per_cu, max_tasks, st);
+    switch (ba.form) {
+    case kLean: return launch_rows<kLean>(ba, int16, rows, cu_count, waves_per_cu, max_tasks, st);
+    case kLeanWide:
+        return launch_rows<kLeanWide>(ba, int16, rows, cu_count, waves_per_cu, max_tasks, st);
+    default:
+        return launch_rows<kGeneralForm>(ba, int16, rows, cu_count, waves_per_cu, max_tasks, st);
+    }
 }
 
 hipError_t launch_walk(const BatchArgs &ba, const int32_t *order, const int32_t *first,

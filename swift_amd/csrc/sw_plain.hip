@@ -244,12 +244,12 @@ static int plain_packed_lds(int rlen_max) {
     return 4 * (kBatchG + 4 * plain_packed_stride(rlen_max) + 4);
 }
 
-template <int R>
+template <int R, int FORM>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(R <= 6 ? 5 : R <= 12 ? 4 : 3)))
 sw_plain_packed_kernel(const char *__restrict__ qseq, const char *__restrict__ rseq, int qlen,
                        int rlen_max, KeyConsts kc, int npairs, int pair0,
                        uint32_t *__restrict__ trace, int64_t wpt, int4 *__restrict__ res) {
-    using S = Lean<kBatchG, R, true>;
+    using S = Lean<kBatchG, R, true, FORM>;
     constexpr int G = kBatchG;
     extern __shared__ uint32_t lds_p[];
     const int lane = threadIdx.x, grp = lane / G, g = lane % G;
@@ -433,7 +433,8 @@ PlainPlan plain_plan(const Scoring &sc, int qlen, int rlen, int npairs) {
     }
     const bool packed = npairs >= kPlainPackedPairs && qlen <= kMaxBatchQ &&
                         rlen <= kPlainPackedCols &&
-                        qlen * sc.match < kLeanScoreLimit - 2 * sc.match;
+                        packed_form(sc, qlen) != kGeneralForm;
+    pl.form = packed_form(sc, qlen);
     pl.route = packed ? PlainPlan::kPacked : PlainPlan::kWave;
     pl.packed_rows = std::max(1, (qlen + kBatchG - 1) / kBatchG);
     pl.task_words = packed_trace_words(pl.packed_rows, rlen);
@@ -493,12 +494,18 @@ static void launch_wave(const char *q, const char *r, const PlainPlan &pl, const
                        pl.move_words, out);
 }
 
+template <int R, int FORM>
+static void launch_packed_as(const char *q, const char *r, const PlainPlan &pl, const KeyConsts &kc,
+                          int n, int pair0, uint32_t *trace, int4 *res, hipStream_t st) {
+    auto k = sw_plain_packed_kernel<R, FORM>;
+    hipLaunchKernelGGL(k, dim3((n + kSlots16 - 1) / kSlots16), dim3(64), plain_packed_lds(pl.rlen),
+                       st, q, r, pl.qlen, pl.rlen, kc, n, pair0, trace, pl.task_words, res);
+}
 template <int R>
 static void launch_packed(const char *q, const char *r, const PlainPlan &pl, const KeyConsts &kc,
                           int n, int pair0, uint32_t *trace, int4 *res, hipStream_t st) {
-    hipLaunchKernelGGL(sw_plain_packed_kernel<R>, dim3((n + kSlots16 - 1) / kSlots16), dim3(64),
-                       plain_packed_lds(pl.rlen), st, q, r, pl.qlen, pl.rlen, kc, n, pair0, trace,
-                       pl.task_words, res);
+    if (pl.form == kLean) launch_packed_as<R, kLean>(q, r, pl, kc, n, pair0, trace, res, st);
+    else launch_packed_as<R, kLeanWide>(q, r, pl, kc, n, pair0, trace, res, st);
 }
 
 #define SWIFT_PLAIN_ROWS(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(10) X(12) X(16)

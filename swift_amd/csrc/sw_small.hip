@@ -41,9 +41,9 @@ __device__ __forceinline__ WalkOut small_walk(const uint32_t *tr, int R, int W, 
                      uni(gr.row), uni(gr.col), ql, rl, mv);
 }
 
-template <int R>
+template <int R, int FORM>
 __global__ void __launch_bounds__(256) sw_small_kernel(SmallArgs a) {
-    using S = Lean<64, R, true>;
+    using S = Lean<64, R, true, FORM>;
     using S32 = Lean<64, R, false>;
     extern __shared__ uint32_t lds[];
     // every wave works alone, in its own part of the workgroup's LDS
@@ -220,16 +220,26 @@ __global__ void __launch_bounds__(256) sw_small_kernel(SmallArgs a) {
 
 int64_t small_wave_words(int maxr) { return (int64_t)((maxr + 63 + 3) & ~3) * 64; }
 
-hipError_t launch_small(const SmallArgs &a, int blocks, hipStream_t st) {
+template <int FORM>
+static hipError_t launch_small_as(const SmallArgs &a, int blocks, hipStream_t st) {
     const size_t lds = 4 * (size_t)a.wpb * small_lds_words(a.maxq, a.maxr);
     switch (std::max(1, (a.maxq + 63) / 64)) {
-#define SWIFT_S(RR) \
-    case RR: hipLaunchKernelGGL(sw_small_kernel<RR>, dim3(blocks), dim3(64 * a.wpb), lds, st, a); break;
+#define SWIFT_S(RR)                                                                          \
+    case RR: {                                                                               \
+        auto k = sw_small_kernel<RR, FORM>;                                                  \
+        hipLaunchKernelGGL(k, dim3(blocks), dim3(64 * a.wpb), lds, st, a);                   \
+        break;                                                                               \
+    }
         SWIFT_S(1) SWIFT_S(2) SWIFT_S(3) SWIFT_S(4) SWIFT_S(5)
 #undef SWIFT_S
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+hipError_t launch_small(const SmallArgs &a, int blocks, hipStream_t st) {
+    return a.form == kLean ? launch_small_as<kLean>(a, blocks, st)
+                           : launch_small_as<kLeanWide>(a, blocks, st);
 }
 
 }  // namespace swift

@@ -296,7 +296,9 @@ struct Sweep {
 //    stored 16 bytes a lane.
 // Sweep kernels before and after: 1.0M pairs of 150 x 300 (R = 10) 11.8 ->
 // 9.4 ms, 439k of 100 x 300 (R = 7) 3.89 -> 3.05 ms, 64 pairs up to 300 x 480
-// in the wide form 137 -> 79 us.
+// in the wide form 137 -> 79 us.  kLeanWide (scores of 960 to 2,016) takes 2 %
+// more cycles: a call of 100,000 pairs of 101-319 bases at 5, -4, -12, -2 with 5
+// % re-run 2.88 -> 2.51 ms.
 // No step is masked: cells left of column 1 keep H = 0; cells right of a
 // pair's last column and rows below its query never match (padding
 // selectors, bit 7 of a padding row's table), so they score strictly below
@@ -348,7 +350,7 @@ __device__ __forceinline__ uint32_t lean_selector(uint32_t cls, int half) {
     return s | 0x0C00u;
 }
 
-template <int G, int R, bool PK>
+template <int G, int R, bool PK, int FORM = kLean>
 struct Lean {
     static constexpr int KPW = PK ? 8 : 16;          // rows per trace word
     static constexpr int W = (R + KPW - 1) / KPW;     // trace words per step
@@ -420,7 +422,7 @@ struct Lean {
 #pragma unroll
             for (int b = 0; b < 4; ++b)
                 if (b * B + k < R) v[n++] = x[b * B + k] - splat<PK>(b);
-            uint32_t m = v[0];
+            uint32_t m = v[0];  // below 0x7C00 in either form
             if (n == 2) m = vmax<PK>(m, v[1]);
             if (n >= 3) m = vmax3<PK>(m, v[1], v[2]);
             if (n == 4) m = vmax<PK>(m, v[3]);
@@ -428,16 +430,27 @@ struct Lean {
             else kb[k] = (m << 3) + (uint32_t)(B - 1 - k);
         }
         uint32_t m = kb[0];
+        if constexpr (PK && FORM == kLeanWide) {
 #pragma unroll
-        for (int k = 1; k + 1 < B; k += 2) m = vmax3<PK>(m, kb[k], kb[k + 1]);
-        if constexpr (B % 2 == 0) m = vmax<PK>(m, kb[B - 1]);
-        if constexpr (PK) {
-            const uint32_t up = as_u(as_s(vsub<true>(best, m)) >> as_s(c_sign));
+            for (int k = 1; k < B; ++k)
+                m = as_u(__builtin_elementwise_max(as_us(m), as_us(kb[k])));
+            // all-ones where m > best: the saturated difference is not 0
+            const uint32_t d = as_u(__builtin_elementwise_sub_sat(as_us(m), as_us(best)));
+            const uint32_t up = vsub<true>(0u, vmin1<true>(d));
             tbest = (up & tcode) | (~up & tbest);
-            best = vmax<true>(best, m);
+            best = as_u(__builtin_elementwise_max(as_us(best), as_us(m)));
         } else {
-            tbest = m > best ? tcode : tbest;
-            best = max(best, m);
+#pragma unroll
+            for (int k = 1; k + 1 < B; k += 2) m = vmax3<PK>(m, kb[k], kb[k + 1]);
+            if constexpr (B % 2 == 0) m = vmax<PK>(m, kb[B - 1]);
+            if constexpr (PK) {
+                const uint32_t up = as_u(as_s(vsub<true>(best, m)) >> as_s(c_sign));
+                tbest = (up & tcode) | (~up & tbest);
+                best = vmax<true>(best, m);
+            } else {
+                tbest = m > best ? tcode : tbest;
+                best = max(best, m);
+            }
         }
     }
 

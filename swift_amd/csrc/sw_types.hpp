@@ -60,10 +60,23 @@ inline bool lean_scoring(const Scoring &s) {
     return s.match >= 1 && s.mismatch < 0 && s.match - s.mismatch <= 31 && s.gap_open <= -1 &&
            s.gap_open >= -63 && s.gap_ext <= -1 && s.gap_ext >= -63;
 }
-// ... and the packed ones' best-cell keys 32*H + row code must stay below the
-// half-precision infinity's bit pattern, 0x7C00 (their maxima are taken as
-// half-precision numbers): scores below this limit
-constexpr int kLeanScoreLimit = 960;
+// Forms of a sweep.  The packed lean ones keep best-cell keys 32*H + 32*match +
+// row code in 16 bits: kLean takes their maxima three at a time as
+// half-precision numbers (keys below the infinity's bit pattern, 0x7C00: H +
+// match <= 990), kLeanWide two at a time as unsigned ones (below 65536: H +
+// match <= 2046).  A pair whose best reaches the form's limit is flagged: H
+// rises by at most match (<= 30) a cell, so a pair with any larger cell has one
+// between the limit and the exact range's end.
+enum SweepForm { kGeneralForm = 0, kLean = 1, kLeanWide = 2 };
+inline int lean_limit(int form, int match) { return (form == kLean ? 960 : 2016) - match; }
+// the packed form for queries of at most maxq bases (larger scores would be
+// re-run in 32-bit lanes)
+inline SweepForm packed_form(const Scoring &s, int maxq) {
+    if (!lean_scoring(s)) return kGeneralForm;
+    const int64_t most = (int64_t)maxq * s.match;
+    return most < lean_limit(kLean, s.match) ? kLean
+           : most < lean_limit(kLeanWide, s.match) ? kLeanWide : kGeneralForm;
+}
 
 constexpr int kColBits = 12;                   // int32 best key: H << 12 | (4095 - j)
 constexpr int kMaxCols = (1 << kColBits) - 1;  // longest reference window (plain kernel)
@@ -114,7 +127,7 @@ struct BatchArgs {
     int32_t *score_out, *start_out, *end_out, *alen_out;
     char *qcons, *rcons;
     const int64_t *coff;
-    int lean;                 // 1: the lean sweeps (lean_scoring)
+    int form;                 // SweepForm
     int walk_deferred;        // 1: record PairTrace descriptors, walk in sw_walk_kernel
     int32_t *nflagged;        // counts the pairs flagged for the int32 re-run
 };
@@ -131,6 +144,7 @@ struct SmallArgs {
     const int32_t *rlen;
     int npairs, ppw, wpb;     // pairs, pairs a wave (1 or 2), waves a workgroup (<= 4)
     int maxq, maxr;
+    int form;                 // kLean or kLeanWide
     KeyConsts kc;
     uint32_t h_limit;         // 4*H at or above this: swept again in 32-bit lanes
     uint32_t *trace;          // wave_words for each wave of the grid

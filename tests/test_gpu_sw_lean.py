@@ -51,12 +51,13 @@ def check(got, want):
 
 
 # scoring, longest query: the default; each limit of the rule (match - mismatch
-# 31, penalties of 63) and one past it; scores up to the packed keys' limit
-# (a best of 950 of the 954 allowed at match 3) and past it
+# 31, penalties of 63) and one past it; scores on both sides of the packed
+# forms' limits (960 - match, 2016 - match)
 EDGES = [((2, -1, -10, -1), 320), ((1, -30, -63, -1), 320), ((1, -31, -10, -1), 200),
          ((3, -2, -2, -63), 316), ((3, -2, -64, -2), 316), ((3, -1, -5, -2), 320),
          ((30, -1, -63, -63), 30), ((30, -1, -63, -63), 32), ((5, -4, -12, -4), 190),
-         ((5, -4, -12, -4), 200), ((1, -1, -1, -2), 100)]
+         ((5, -4, -12, -4), 200), ((1, -1, -1, -2), 100), ((6, -5, -13, -3), 320),
+         ((30, -1, -63, -63), 66), ((30, -1, -63, -63), 67), ((7, -3, -9, -2), 290)]
 
 
 @pytest.mark.parametrize("form", ["rows", "coarse", "wide", "int32"])

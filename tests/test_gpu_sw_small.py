@@ -57,3 +57,16 @@ def test_plain_routes(A, orc, n, ql, rl):
     got = A.align_sequences(qs, rs, ql, rl)
     sc, st, en, al, qc, rc = orc.sw_batch(qs, rs, nthreads=8)
     check(got, (sc.astype(np.float32), st, en, al, qc, rc))
+
+
+@pytest.mark.parametrize("sc,n,ql,rl", [((5, -4, -12, -2), 4099, 201, 260),
+                                        ((6, -5, -13, -3), 70, 320, 400),
+                                        ((3, -2, -64, -2), 4099, 60, 90)])
+def test_plain_scorings(A, orc, sc, n, ql, rl):
+    """Packed route with the wider keys, wave route past them, general route."""
+    rnd = random.Random(n + ql)
+    qs, rs = edge_pairs(rnd, n, ql, rl)
+    qs = [q.ljust(ql, b"G")[:ql] for q in qs]
+    got = A.align_sequences(qs, rs, ql, rl, A.Scoring(*sc))
+    s, st, en, al, qc, rc = orc.sw_batch(qs, rs, *sc, nthreads=8)
+    check(got, (s.astype(np.float32), st, en, al, qc, rc))
