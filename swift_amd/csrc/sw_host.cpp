@@ -545,10 +545,14 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     // one-launch form's) runs the wide form: its few tasks are each one wave,
     // and a wave's sweep is the batch's latency
     const int wide = coarse == kRBins ? 1 : 0;
+    // pairs whose best alignment provably has no gap are answered from their
+    // bytes ahead of the sweeps
+    const SweepForm form16 = packed_form(sc, io.maxq);
+    const bool screen = form16 != kGeneralForm && !force32;
     auto pass_args = [&](int pass, const PairResult *prev, int f32, BinArgs &b, TaskArgs &t) {
         b = BinArgs{io.rseq, io.roff, io.qlen, io.rlen, prev, n, f32, w.bin_of.as<int32_t>(),
                     bins + (2 * pass) * kNumBins, cnt + kCntError, io.score, io.start, io.end,
-                    io.alen, coarse};
+                    io.alen, coarse, pass == 0 && screen ? w.res.as<PairResult>() : nullptr};
         t = TaskArgs{bins + (2 * pass) * kNumBins, bins + (2 * pass + 1) * kNumBins,
                      segs + (3 * pass) * NS, segs + (3 * pass + 1) * NS,
                      segs + (3 * pass + 2) * NS, cnt + 4 * pass, cnt + 4 * pass + 1,
@@ -564,7 +568,6 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     // [2048 - pos, 2047] whose key is exact.
     uint32_t h_limit = (uint32_t)std::min(32767 - (4 * pos + 3) - 4, 4 * (2048 - pos));
     const bool lean32 = lean_scoring(sc);  // 32-bit lanes have no limit
-    const SweepForm form16 = packed_form(sc, io.maxq);
     if (form16 != kGeneralForm) h_limit = 4u * (uint32_t)lean_limit(form16, sc.match);
 
     // a small call in one launch, unless row classes are asked for (coarse
@@ -596,6 +599,12 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
         SWIFT_HIP_TRY(launch_zero(z, st));
     }
     SWIFT_HIP_TRY(mark(0, st, w.timed));
+    if (screen)
+        SWIFT_HIP_TRY(launch_screen(
+            ScreenArgs{io.qseq, io.qoff, io.qlen, io.rseq, io.roff, io.rlen, n, 1, io.score,
+                       io.start, io.end, io.alen, io.qcons, io.rcons, io.cons_off,
+                       w.res.as<PairResult>()},
+            sc, st));
     // ---- pass 1: bin every pair
     BinArgs b1;
     TaskArgs t1;

@@ -485,6 +485,7 @@ __device__ __forceinline__ int classify_pair(const BinArgs &a, int p) {
         }
         return -1;
     }
+    if (a.screened && (a.screened[p].flags & kScreenedFlag)) return -1;
     int cls;
     if (a.prev) {
         if (!(a.prev[p].flags & 1)) return -1;

@@ -158,6 +158,24 @@ struct SmallArgs {
 int64_t small_wave_words(int maxr);
 hipError_t launch_small(const SmallArgs &a, int blocks, hipStream_t st);
 
+// The screen ahead of the batched path's binning (sw_screen.hip).  A pair it
+// answers has kScreenedFlag in its result's flags.
+constexpr int32_t kScreenedFlag = 2;
+struct ScreenArgs {
+    const char *qseq;
+    const int64_t *qoff;
+    const int32_t *qlen;
+    const char *rseq;
+    const int64_t *roff;
+    const int32_t *rlen;
+    int npairs, per;          // pairs; pairs a wave (set by the launch)
+    int32_t *score_out, *start_out, *end_out, *alen_out;
+    char *qcons, *rcons;
+    const int64_t *coff;
+    PairResult *res;
+};
+hipError_t launch_screen(const ScreenArgs &a, const Scoring &s, hipStream_t st);
+
 // outputs of the plain (alignSequences) kernel: reference layout
 struct PlainOut {
     float *score;
@@ -185,6 +203,7 @@ struct BinArgs {
     // or kCoarseRowsSmall for the smallest batches: at most kRBins / coarse
     // classes; exact, the extra rows are padding); 0: every R its own class
     int coarse;
+    const PairResult *screened;  // null, or results in which kScreenedFlag leaves a pair out
 };
 
 constexpr int kCoarseRows = 5;
