@@ -397,6 +397,7 @@ constexpr int kCntError = 8;
 constexpr int kCntFlagged = 9;
 constexpr int kCntQueues = 16;
 constexpr int kCntReruns = 200;  // never zeroed (sw_small.hip)
+constexpr int kCntLeft = 201;    // pairs the screen leaves to it
 constexpr int kQueuesPerPass = 2 * kRBins;
 // sync_sizes: the sizes of each pass are read back (synchronising); then
 // final_sync also waits for the pass's last kernels before returning
@@ -433,8 +434,8 @@ int sw_batch_check_in(Workspace *w, hipStream_t st) {
 
 // A small call as one kernel (sw_small.hip).  *done: 0 when a pair was longer
 // than the call said and the general path has to run.
-static int batch_run_small(Workspace &w, const BatchIO &io, SweepForm form, const KeyConsts &kc,
-                           uint32_t h_limit, hipStream_t st, bool final_sync, int *done) {
+static int batch_run_small(Workspace &w, const BatchIO &io, const Scoring &sc, SweepForm form,
+                           const KeyConsts &kc, uint32_t h_limit, hipStream_t st, bool final_sync, int *done) {
     const int n = io.npairs;
     SmallArgs a{};
     a.qseq = io.qseq;
@@ -467,9 +468,26 @@ static int batch_run_small(Workspace &w, const BatchIO &io, SweepForm form, cons
     a.coff = io.cons_off;
     a.flags = w.stage->small;
     a.reruns = w.counters.as<int32_t>() + kCntReruns;
+    // the screen first, and the one launch on what it leaves
+    const bool screen = !io.sparse && n >= kSmallScreen;
+    if (screen) {
+        a.list = w.order.as<int32_t>();
+        a.nlist = w.counters.as<int32_t>() + kCntLeft;
+        ZeroSpans z{};
+        z.p[0] = w.counters.as<int32_t>() + kCntLeft;
+        z.n[0] = 1;
+        z.nspans = 1;
+        SWIFT_HIP_TRY(launch_zero(z, st));
+    }
     volatile int32_t *flags = w.stage->small;
     for (int i = 0; i < kSmallFlags; ++i) flags[i] = 0;
     for (int i = 0; i < 2; ++i) SWIFT_HIP_TRY(mark(i, st, w.timed));
+    if (screen)
+        SWIFT_HIP_TRY(launch_screen(
+            ScreenArgs{io.qseq, io.qoff, io.qlen, io.rseq, io.roff, io.rlen, n, 1, io.score,
+                       io.start, io.end, io.alen, io.qcons, io.rcons, io.cons_off, nullptr,
+                       w.order.as<int32_t>(), w.counters.as<int32_t>() + kCntLeft},
+            sc, st));
     SWIFT_HIP_TRY(launch_small(a, blocks, st));
     for (int i = 2; i < 5; ++i) SWIFT_HIP_TRY(mark(i, st, w.timed));
     w.stats.ntasks16 = (n + a.ppw * a.wpb - 1) / (a.ppw * a.wpb);
@@ -575,7 +593,7 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     if (form16 != kGeneralForm && !force32 && (cmode < 0 || (cmode == 1 && n < kCoarseTinyPairs)) &&
         small_call(n, io.maxq, io.sparse)) {
         int done = 0;
-        if ((rc = batch_run_small(w, io, form16, kc16, h_limit, st, sync_sizes && final_sync,
+        if ((rc = batch_run_small(w, io, sc, form16, kc16, h_limit, st, sync_sizes && final_sync,
                                   &done)) ||
             done)
             return rc;
@@ -603,7 +621,7 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
         SWIFT_HIP_TRY(launch_screen(
             ScreenArgs{io.qseq, io.qoff, io.qlen, io.rseq, io.roff, io.rlen, n, 1, io.score,
                        io.start, io.end, io.alen, io.qcons, io.rcons, io.cons_off,
-                       w.res.as<PairResult>()},
+                       w.res.as<PairResult>(), nullptr, nullptr},
             sc, st));
     // ---- pass 1: bin every pair
     BinArgs b1;

@@ -150,20 +150,29 @@ constexpr int kWideShortPairs = 2048;
 // wave a SIMD), then two.
 constexpr int kSmallSingles = 1024;
 constexpr int kSmallWaves = 4096;   // each keeps a trace area
-// Its waves take pairs unsorted, 64 lanes of ceil(maxq / 64) rows each, against
-// the general path's binning, readback and 16-lane groups: taken up to
-// kSmallWork = pairs x rows a lane.  Queries of 50-300 and of 100 bases, us a
-// call, general -> one launch:
-//   50-300: 512 172 -> 104, 4,000 240 -> 172, 8,000 408 -> 286, 16,000 568 ->
-//   526, 20,000 618 -> 621, 24,000 637 -> 752
-//   100: 512 143 -> 55, 4,500 208 -> 100, 24,000 478 -> 391, 40,000 659 -> 623
-// A pipeline's capacity counts slots of which a half or fewer hold records, so
-// twice that: 5,000 reads of 300 bases (capacity 30,000) 1,052 -> 816 us,
-// 13,000 of 100 1,039 -> 995.
-constexpr int kSmallWork = 80000;
+// From this many pairs on the screen goes first (sw_screen.hip) and the one
+// launch takes what it leaves: two launches more, against the related pairs'
+// sweeps.  us a call without and with, queries of 50-300 bases beside their
+// places: 2,048 pairs 120, 130; 4,000 177, 142; 16,000 527, 335; of 100 bases
+// 59, 69; 78, 77; 219, 126.  Not where slots may be missing: most of a
+// pipeline's pairs are unrelated, and its small calls wait for launches.
+constexpr int kSmallScreen = 4000;
+// The one launch's waves take pairs unsorted, 64 lanes of ceil(maxq / 64) rows
+// each, against the general path's binning, readback and 16-lane groups: taken
+// up to kSmallWork = pairs x rows a lane.  us a call, general -> one launch,
+// both with the screen:
+//   50-300: 26,000 610 -> 438, 40,000 660 -> 583, 60,000 713 -> 793
+//   100: 60,000 319 -> 272
+// and of pairs the screen leaves, which sets the line below what those ask:
+//   50-300: 16,000 568 -> 526, 24,000 637 -> 752; 100: 40,000 659 -> 623
+// A pipeline's capacity counts slots of which a half or fewer hold records:
+// 5,000 reads of 300 bases (capacity 30,000) 1,052 -> 816 us, 13,000 of 100
+// 1,039 -> 995.
+constexpr int kSmallWork = 130000;
+constexpr int kSmallWorkSparse = 160000;
 inline bool small_call(int npairs, int maxq, bool sparse) {
     const int64_t rows = maxq > 64 ? (maxq + 63) / 64 : 1;
-    return npairs * rows <= (sparse ? 2 : 1) * (int64_t)kSmallWork;
+    return npairs * rows <= (sparse ? kSmallWorkSparse : kSmallWork);
 }
 Tuning &tuning();
 

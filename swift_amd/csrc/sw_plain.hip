@@ -5,8 +5,9 @@
 //
 // Four routes, by scoring and size (PlainPlan):
 //  * packed: the scorings of lean_scoring whose best score stays below the
-//    packed limit, from kPlainPackedPairs pairs on: the batched path's sweep,
-//    eight pairs a wave (sw_plain_packed_kernel), then walk and expansion.
+//    packed limit, from kPlainPackedPairs pairs on: the screen
+//    (sw_screen.hpp), then for the pairs it leaves, listed, the batched path's
+//    sweep, eight a wave (sw_plain_packed_kernel), walk and expansion.
 //    A pair whose reference holds a byte outside ACGTNacgtn is left to the
 //    wave kernel.
 //  * wave: the other calls under lean_scoring, and those pairs: one wave
@@ -105,6 +106,14 @@ sw_plain_kernel(const char *__restrict__ qseq, const char *__restrict__ rseq, in
     if (g == 0) res[p] = make_int4(gr.score, gr.row, gr.col, rlen);
 }
 
+// The i-th pair of a kernel's work: of n in a row, or of a list (null: none).
+struct PlainPairs {
+    const int32_t *list, *count;
+    int n;
+    __device__ __forceinline__ int size() const { return list ? uni(*count) : n; }
+    __device__ __forceinline__ int at(int i) const { return list ? list[i] : i; }
+};
+
 // Where a pair's trace lies: ppt pairs share a task's area of wpt words (8
 // packed pairs, two per 16-lane group; or one pair).
 struct PlainTrace {
@@ -123,12 +132,12 @@ struct PlainTrace {
 // best cell (res: score, row, col, columns; columns < 0: left to the wave
 // kernel) and stores the path as 2-bit moves plus the drop-in's score, start,
 // end and length.
-__global__ void __launch_bounds__(256) sw_plain_walk_kernel(PlainTrace tr, int qlen, int npairs,
-                                                            int pair0, const int4 *res,
+__global__ void __launch_bounds__(256) sw_plain_walk_kernel(PlainTrace tr, int qlen,
+                                                            PlainPairs pairs, int pair0, const int4 *res,
                                                             uint32_t *moves, int move_words,
                                                             PlainOut out) {
     const int p = blockIdx.x * 256 + (int)threadIdx.x;
-    if (p >= npairs) return;
+    if (p >= pairs.size()) return;
     const int4 r = res[p];
     if (r.w < 0) return;
     uint32_t *mv = moves + (int64_t)p * move_words;
@@ -142,7 +151,7 @@ __global__ void __launch_bounds__(256) sw_plain_walk_kernel(PlainTrace tr, int q
     };
     WalkOut wo = walk_cells<TraceReaderLean>(tr.trace, r.x, r.y, r.z, tr.of(p), qlen, r.w, emit);
     if (wo.len & 15) mv[wo.len >> 4] = word;
-    const int gp = pair0 + p;
+    const int gp = pair0 + pairs.at(p);
     out.score[gp] = (float)r.x;
     out.start[gp] = wo.start;
     out.end[gp] = wo.end;
@@ -153,10 +162,10 @@ __global__ void __launch_bounds__(256) sw_plain_walk_kernel(PlainTrace tr, int q
 // words per lane (a path's moves fit NMV * 64 words)
 template <int NMV>
 __global__ void __launch_bounds__(256)
-sw_plain_walk_wave_kernel(PlainTrace tr, int qlen, int npairs, int pair0, const int4 *res,
-                          uint32_t *moves, int move_words, PlainOut out) {
+sw_plain_walk_wave_kernel(PlainTrace tr, int qlen, PlainPairs pairs, int pair0,
+                          const int4 *res, uint32_t *moves, int move_words, PlainOut out) {
     const int p = uni((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-    if (p >= npairs) return;
+    if (p >= pairs.size()) return;
     const int4 r = res[p];
     const int score = uni(r.x);
     if (uni(r.w) < 0) return;
@@ -166,7 +175,7 @@ sw_plain_walk_wave_kernel(PlainTrace tr, int qlen, int npairs, int pair0, const 
                            tr.R, tr.W, (pt.half & 2) ? 3 : 4, (pt.half & 1) * 16, score, uni(r.y),
                            uni(r.z), qlen, uni(r.w), mv);
     if ((threadIdx.x & 63) == 0) {
-        const int gp = pair0 + p;
+        const int gp = pair0 + pairs.at(p);
         out.score[gp] = (float)score;
         out.start[gp] = wo.start;
         out.end[gp] = wo.end;
@@ -197,20 +206,24 @@ __device__ __forceinline__ ExpandPair plain_expand(const char *qseq, const char 
 // The consensus strings from the walks' moves, four pairs per one-wave
 // workgroup (dynamic LDS: 4 x (qw + rw) dwords).
 __global__ void __launch_bounds__(64) sw_plain_expand_kernel(const char *qseq, const char *rseq,
-                                                             int qlen, int rlen_max, int npairs,
-                                                             int pair0, const int4 *res,
+                                                             int qlen, int rlen_max,
+                                                             PlainPairs pairs, int pair0,
+                                                             const int4 *res,
                                                              const uint32_t *moves,
                                                              int move_words, int qw, int rw,
                                                              PlainOut out) {
     extern __shared__ uint32_t lds_x[];
     const int slot = threadIdx.x >> 4, sl = threadIdx.x & 15;
     const int p = blockIdx.x * 4 + slot;
+    const int npairs = pairs.size();
+    if ((int)blockIdx.x * 4 >= npairs) return;
     ExpandPair e;
     if (p < npairs) {
         const int4 r = res[p];
+        const int gp = pair0 + pairs.at(p);
         if (r.w >= 0)
-            e = plain_expand(qseq, rseq, qlen, rlen_max, pair0 + p, out.alen[pair0 + p], r.y, r.z,
-                             r.w, moves + (int64_t)p * move_words, out);
+            e = plain_expand(qseq, rseq, qlen, rlen_max, gp, out.alen[gp], r.y, r.z, r.w,
+                             moves + (int64_t)p * move_words, out);
     }
     expand_row<16>(e, lds_x + slot * (qw + rw), lds_x + slot * (qw + rw) + qw, sl);
 }
@@ -237,7 +250,8 @@ __device__ __forceinline__ int ref_columns(const char *rs, int rlen_max, int g) 
 // The packed sweep: eight pairs a wave, two per 16-lane group, R = ceil(qlen /
 // 16) rows a lane.  Against one wave per pair in 32-bit lanes (64 columns of
 // ramp instead of 16, one cell a lane and instruction instead of two):
-// 100,000 pairs of 100 x 300 3.37 -> 0.93 ms.  Dynamic LDS: plain_packed_lds().
+// 100,000 pairs of 100 x 300 3.37 -> 0.93 ms, and 0.40 where the screen takes
+// four in five.  Dynamic LDS: plain_packed_lds().
 constexpr int kPackedTail = kBatchG + 2;  // padding columns after the last
 __host__ __device__ constexpr int plain_packed_stride(int rlen_max) { return rlen_max + kPackedTail; }
 static int plain_packed_lds(int rlen_max) {
@@ -247,13 +261,15 @@ static int plain_packed_lds(int rlen_max) {
 template <int R, int FORM>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(R <= 6 ? 5 : R <= 12 ? 4 : 3)))
 sw_plain_packed_kernel(const char *__restrict__ qseq, const char *__restrict__ rseq, int qlen,
-                       int rlen_max, KeyConsts kc, int npairs, int pair0,
+                       int rlen_max, KeyConsts kc, PlainPairs pairs, int pair0,
                        uint32_t *__restrict__ trace, int64_t wpt, int4 *__restrict__ res) {
     using S = Lean<kBatchG, R, true, FORM>;
     constexpr int G = kBatchG;
     extern __shared__ uint32_t lds_p[];
     const int lane = threadIdx.x, grp = lane / G, g = lane % G;
     uint32_t *col = lds_p + G + grp * plain_packed_stride(rlen_max);
+    const int npairs = pairs.size();
+    if ((int)blockIdx.x * kSlots16 >= npairs) return;
     const int p0 = (int)blockIdx.x * kSlots16 + grp * 2;
     S sw;
     sw.init(kc);
@@ -262,7 +278,7 @@ sw_plain_packed_kernel(const char *__restrict__ qseq, const char *__restrict__ r
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         // a slot past the last pair reads that pair and is cleared
-        const int64_t gp = pair0 + min(p0 + h, npairs - 1);
+        const int64_t gp = pair0 + pairs.at(min(p0 + h, npairs - 1));
         const char *qs = qseq + gp * (qlen + 1);
         rs[h] = rseq + gp * (rlen_max + 1);
 #pragma unroll
@@ -317,8 +333,8 @@ sw_plain_packed_kernel(const char *__restrict__ qseq, const char *__restrict__ r
 // over its own trace area, the moves in LDS, the expansion.  For small calls,
 // where every launch and every kernel's tail counts, and for calls whose
 // scores pass the packed lanes' range.  Each wave takes pairs in turn; with
-// `flagged` (res of a packed sweep) only those that sweep left, `per` at a
-// time.  256 pairs of 143 x 253 81 -> 45 us.  Dynamic LDS: plain_wave_lds().
+// `flagged` (res of a packed sweep over `pairs`) only those that sweep left,
+// `per` at a time.  256 pairs of 143 x 253 81 -> 45 us.  Dynamic LDS: plain_wave_lds().
 static int plain_wave_lds(int qlen, int rlen_max, int move_words) {
     return 4 * (std::max(rlen_max + 2 * kPlainPad + 8, (qlen + 6) / 4 + (rlen_max + 6) / 4) +
                 move_words);
@@ -327,13 +343,14 @@ static int plain_wave_lds(int qlen, int rlen_max, int move_words) {
 template <int R>
 __global__ void __launch_bounds__(64)
 sw_plain_wave_kernel(const char *__restrict__ qseq, const char *__restrict__ rseq, int qlen,
-                     int rlen_max, KeyConsts kc, int npairs, int pair0, uint32_t *trace,
+                     int rlen_max, KeyConsts kc, PlainPairs pairs, int pair0, uint32_t *trace,
                      int64_t wpp, const int4 *flagged, int per, int move_words, PlainOut out) {
     using S = Lean<64, R, false>;
     extern __shared__ uint32_t lds_w[];
     const int g = threadIdx.x;
     uint32_t *mvs = lds_w, *col = lds_w + move_words;  // the columns, then the expansion's bases
     uint32_t *tr = trace + (int64_t)blockIdx.x * wpp;
+    const int npairs = pairs.size();
     auto pair = [&](int p) {
         const int gp = pair0 + p;
         const char *qs = qseq + (int64_t)gp * (qlen + 1);
@@ -382,7 +399,7 @@ sw_plain_wave_kernel(const char *__restrict__ qseq, const char *__restrict__ rse
         const int p = p0 + g;
         uint64_t left = __ballot(g < per && p < npairs && flagged[min(p, npairs - 1)].w < 0);
         while (left) {
-            pair(p0 + (int)__builtin_ctzll(left));
+            pair(uni(pairs.at(p0 + (int)__builtin_ctzll(left))));
             left &= left - 1;
         }
     }
@@ -412,8 +429,8 @@ static int64_t packed_trace_words(int R, int rlen) {
 // Waves of the wave kernel (each keeps a trace area): four to a SIMD
 constexpr int kPlainWaves = 4096;
 // Calls of at least this many pairs take the packed route, whose sixteen-lane
-// groups need eight times the pairs to fill the chip.  Packed against wave
-// route, us: 100 x 300 bases, 2,048 pairs 90 against 61, 4,096 94 against 104,
+// groups need eight times the pairs to fill the chip.  Packed (without the
+// screen) against wave route, us: 100 x 300 bases, 2,048 pairs 90 against 61, 4,096 94 against 104,
 // 8,192 98 against 208; 250 x 450, 231 against 133, 238 against 237, 256
 // against 462.
 constexpr int kPlainPackedPairs = 4096;
@@ -448,7 +465,8 @@ static int plain_waves(const PlainPlan &pl, int n, int64_t words) {
 }
 
 // Scratch of a chunk of n pairs: general [n traces][n best cells][n moves];
-// packed [tasks' traces][n best cells][n moves][waves' traces]; wave [waves'
+// packed [tasks' traces][n best cells][n moves][waves' traces][the list's
+// count, the list]; wave [waves'
 // traces].  Every part is a multiple of 4 words, so the best cells are 16-byte
 // aligned.
 int64_t plain_words(const PlainPlan &pl, int n, int waves) {
@@ -457,7 +475,7 @@ int64_t plain_words(const PlainPlan &pl, int n, int waves) {
     case PlainPlan::kGeneral: return (int64_t)n * pl.wave_words + cells;
     case PlainPlan::kPacked:
         return (int64_t)((n + kSlots16 - 1) / kSlots16) * pl.task_words + cells +
-               (int64_t)waves * pl.wave_words;
+               (int64_t)waves * pl.wave_words + 4 + ((n + 3) & ~3);
     default: return (int64_t)waves * pl.wave_words;
     }
 }
@@ -485,27 +503,29 @@ static void launch_general(const char *q, const char *r, const PlainPlan &pl, co
 
 template <int R>
 static void launch_wave(const char *q, const char *r, const PlainPlan &pl, const KeyConsts &kc,
-                        int n, int pair0, uint32_t *trace, int waves, const int4 *flagged,
-                        const PlainOut &out, hipStream_t st) {
+                        PlainPairs pairs, int pair0, uint32_t *trace, int waves,
+                        const int4 *flagged, const PlainOut &out, hipStream_t st) {
+    const int n = pairs.n;
     const int per = flagged ? std::min(64, (n + waves - 1) / waves) : 1;
     hipLaunchKernelGGL(sw_plain_wave_kernel<R>, dim3(std::min(waves, (n + per - 1) / per)),
                        dim3(64), plain_wave_lds(pl.qlen, pl.rlen, pl.move_words), st, q, r,
-                       pl.qlen, pl.rlen, kc, n, pair0, trace, pl.wave_words, flagged, per,
+                       pl.qlen, pl.rlen, kc, pairs, pair0, trace, pl.wave_words, flagged, per,
                        pl.move_words, out);
 }
 
 template <int R, int FORM>
 static void launch_packed_as(const char *q, const char *r, const PlainPlan &pl, const KeyConsts &kc,
-                          int n, int pair0, uint32_t *trace, int4 *res, hipStream_t st) {
+                          PlainPairs pairs, int pair0, uint32_t *trace, int4 *res, hipStream_t st) {
     auto k = sw_plain_packed_kernel<R, FORM>;
-    hipLaunchKernelGGL(k, dim3((n + kSlots16 - 1) / kSlots16), dim3(64), plain_packed_lds(pl.rlen),
-                       st, q, r, pl.qlen, pl.rlen, kc, n, pair0, trace, pl.task_words, res);
+    hipLaunchKernelGGL(k, dim3((pairs.n + kSlots16 - 1) / kSlots16), dim3(64),
+                       plain_packed_lds(pl.rlen), st, q, r, pl.qlen, pl.rlen, kc, pairs, pair0, trace, pl.task_words, res);
 }
 template <int R>
 static void launch_packed(const char *q, const char *r, const PlainPlan &pl, const KeyConsts &kc,
-                          int n, int pair0, uint32_t *trace, int4 *res, hipStream_t st) {
-    if (pl.form == kLean) launch_packed_as<R, kLean>(q, r, pl, kc, n, pair0, trace, res, st);
-    else launch_packed_as<R, kLeanWide>(q, r, pl, kc, n, pair0, trace, res, st);
+                          PlainPairs pairs, int pair0, uint32_t *trace, int4 *res,
+                          hipStream_t st) {
+    if (pl.form == kLean) launch_packed_as<R, kLean>(q, r, pl, kc, pairs, pair0, trace, res, st);
+    else launch_packed_as<R, kLeanWide>(q, r, pl, kc, pairs, pair0, trace, res, st);
 }
 
 #define SWIFT_PLAIN_ROWS(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(10) X(12) X(16)
@@ -517,10 +537,11 @@ hipError_t launch_plain(const PlainPlan &pl, const char *q, const char *r, const
                         hipStream_t st) {
     if (n <= 0) return hipSuccess;
     const KeyConsts kc = make_consts(sc, kBytes);
+    PlainPairs pairs{nullptr, nullptr, n};
     auto wave = [&](uint32_t *trace, const int4 *flagged) -> bool {
         switch (pl.wave_rows) {
 #define SWIFT_W(RR) \
-    case RR: launch_wave<RR>(q, r, pl, kc, n, pair0, trace, waves, flagged, out, st); return true;
+    case RR: launch_wave<RR>(q, r, pl, kc, pairs, pair0, trace, waves, flagged, out, st); return true;
             SWIFT_PLAIN_ROWS(SWIFT_W)
 #undef SWIFT_W
         default: return false;
@@ -534,11 +555,24 @@ hipError_t launch_plain(const PlainPlan &pl, const char *q, const char *r, const
     int4 *res = reinterpret_cast<int4 *>(scratch + tw);
     uint32_t *moves = scratch + tw + (int64_t)n * 4;
     PlainTrace tr{scratch, pl.wave_words, 1, pl.wave_rows, 1};
+    uint32_t *area = moves + (((int64_t)n * pl.move_words + 3) & ~(int64_t)3);
     if (packed) {
+        int32_t *count = reinterpret_cast<int32_t *>(area + waves * pl.wave_words);
+        pairs.list = count + 4;
+        pairs.count = count;
+        ZeroSpans z{};
+        z.p[0] = count;
+        z.n[0] = 1;
+        z.nspans = 1;
+        hipError_t e = launch_zero(z, st);
+        if (e == hipSuccess)
+            e = launch_screen_plain(q, r, sc, pl.qlen, pl.rlen, n, pair0, out, count + 4, count,
+                                    st);
+        if (e != hipSuccess) return e;
         tr = PlainTrace{scratch, pl.task_words, kSlots16, pl.packed_rows, (pl.packed_rows + 7) / 8};
         switch (pl.packed_rows) {
 #define SWIFT_P(RR) \
-    case RR: launch_packed<RR>(q, r, pl, kc, n, pair0, scratch, res, st); break;
+    case RR: launch_packed<RR>(q, r, pl, kc, pairs, pair0, scratch, res, st); break;
             SWIFT_PACKED_ROWS(SWIFT_P)
 #undef SWIFT_P
         default: return hipErrorInvalidValue;
@@ -559,20 +593,17 @@ hipError_t launch_plain(const PlainPlan &pl, const char *q, const char *r, const
                  : nmv == 3 ? sw_plain_walk_wave_kernel<3>
                  : nmv == 4 ? sw_plain_walk_wave_kernel<4>
                             : sw_plain_walk_wave_kernel<5>;
-        hipLaunchKernelGGL(k, dim3((n + 3) / 4), dim3(256), 0, st, tr, pl.qlen, n, pair0, res,
-                           moves, mw, out);
+        hipLaunchKernelGGL(k, dim3((n + 3) / 4), dim3(256), 0, st, tr, pl.qlen, pairs,
+                           pair0, res, moves, mw, out);
     } else {
         hipLaunchKernelGGL(sw_plain_walk_kernel, dim3((n + 255) / 256), dim3(256), 0, st, tr,
-                           pl.qlen, n, pair0, res, moves, mw, out);
+                           pl.qlen, pairs, pair0, res, moves, mw, out);
     }
     const int qw = (pl.qlen + 6) / 4, rw = (pl.rlen + 6) / 4;
     hipLaunchKernelGGL(sw_plain_expand_kernel, dim3((n + 3) / 4), dim3(64),
-                       sizeof(uint32_t) * 4 * (size_t)(qw + rw), st, q, r, pl.qlen, pl.rlen, n,
+                       sizeof(uint32_t) * 4 * (size_t)(qw + rw), st, q, r, pl.qlen, pl.rlen, pairs,
                        pair0, res, moves, mw, qw, rw, out);
-    if (packed) {  // the pairs the packed sweep left
-        uint32_t *area = moves + (((int64_t)n * mw + 3) & ~(int64_t)3);
-        if (!wave(area, res)) return hipErrorInvalidValue;
-    }
+    if (packed && !wave(area, res)) return hipErrorInvalidValue;  // the pairs the packed sweep left
     return hipGetLastError();
 }
 

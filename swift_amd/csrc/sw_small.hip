@@ -53,15 +53,17 @@ __global__ void __launch_bounds__(256) sw_small_kernel(SmallArgs a) {
     uint32_t *moves = lds + wv * small_lds_words(a.maxq, a.maxr);
     uint32_t *col = moves + 2 * mw;  // the columns, then the expansion's bases
     uint32_t *tr = a.trace + (int64_t)wave * a.wave_words;
-    const int ntask = (a.npairs + a.ppw - 1) / a.ppw;
+    const int npairs = a.nlist ? uni(*a.nlist) : a.npairs;
+    const int ntask = (npairs + a.ppw - 1) / a.ppw;
     for (int task = wave; task < ntask; task += nwaves) {
         int pid[2], ql[2], rl[2];
         const char *qs[2], *rs[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int p = task * a.ppw + h;
-            pid[h] = h < a.ppw && p < a.npairs ? p : -1;
-            const int at = min(p, a.npairs - 1);
+            const int i = task * a.ppw + h;
+            int at = min(i, npairs - 1);
+            if (a.list) at = uni(a.list[at]);
+            pid[h] = h < a.ppw && i < npairs ? at : -1;
             ql[h] = uni(a.qlen[at]);
             rl[h] = uni(a.rlen[at]);
             qs[h] = a.qseq + a.qoff[at];

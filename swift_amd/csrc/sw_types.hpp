@@ -142,6 +142,7 @@ struct SmallArgs {
     const char *rseq;
     const int64_t *roff;
     const int32_t *rlen;
+    const int32_t *list, *nlist;  // or null: the pairs to take (of npairs at most)
     int npairs, ppw, wpb;     // pairs, pairs a wave (1 or 2), waves a workgroup (<= 4)
     int maxq, maxr;
     int form;                 // kLean or kLeanWide
@@ -172,7 +173,8 @@ struct ScreenArgs {
     int32_t *score_out, *start_out, *end_out, *alen_out;
     char *qcons, *rcons;
     const int64_t *coff;
-    PairResult *res;
+    PairResult *res;          // or null
+    int32_t *list, *count;    // or null: the pairs left, counted on from *count
 };
 hipError_t launch_screen(const ScreenArgs &a, const Scoring &s, hipStream_t st);
 
@@ -183,6 +185,10 @@ struct PlainOut {
     char *qcons, *rcons;
     int64_t cstride;
 };
+// list: the pairs (from 0) the screen leaves, counted on from *count
+hipError_t launch_screen_plain(const char *q, const char *r, const Scoring &s, int qlen, int rlen,
+                               int n, int pair0, const PlainOut &out, int32_t *list,
+                               int32_t *count, hipStream_t st);
 
 
 struct BinArgs {

@@ -107,3 +107,19 @@ def test_screen_takes_reads(A, orc):
     finally:
         A.set_coarse_rows(before)
     check(got, orc.sw_batch(qs, rs, nthreads=8))
+
+
+@pytest.mark.parametrize("ql,rl", [(16, 40), (100, 300), (143, 200), (320, 480)])
+def test_screen_plain(A, orc, ql, rl):
+    """The plain path's packed route: the screen, and the sweep of its list;
+    references that end early."""
+    rnd = random.Random(ql)
+    qs, rs = screen_pairs(rnd, 4200, 320)
+    for i in range(len(qs)):
+        reg = rs[i][:rl].ljust(rl if i % 3 else 1, b"G")
+        o = rnd.randint(0, max(0, len(reg) - ql))
+        q = reg[o:o + ql].upper().ljust(ql, b"C") if i % 2 else qs[i].ljust(ql, b"T")[:ql]
+        qs[i], rs[i] = q, reg
+    got = A.align_sequences(qs, rs, ql, rl)
+    sc, st, en, al, qc, rc = orc.sw_batch(qs, rs, nthreads=8)
+    check(got, (sc.astype(np.float32), st, en, al, qc, rc))
