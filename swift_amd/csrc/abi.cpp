@@ -4,6 +4,7 @@
 #include <cstdlib>
 
 #include "../../include/swift_abi.h"
+#include "device_pool.hpp"
 #include "sw_host.hpp"
 #include "sw_types.hpp"
 
@@ -26,15 +27,15 @@ int swift_device_count(int *count) {
     return kOk;
 }
 int swift_device_alloc(void **ptr, size_t bytes) {
-    SWIFT_HIP_TRY(hipMalloc(ptr, bytes ? bytes : 1));
+    SWIFT_HIP_TRY(pool_alloc(ptr, bytes));
     return kOk;
 }
 int swift_device_free(void *ptr) {
-    SWIFT_HIP_TRY(hipFree(ptr));
+    SWIFT_HIP_TRY(pool_free(ptr));
     return kOk;
 }
 int swift_memcpy_htod(void *dst, const void *src, size_t bytes) {
-    SWIFT_HIP_TRY(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
+    SWIFT_HIP_TRY(copy_to_device(dst, src, bytes));
     return kOk;
 }
 int swift_memcpy_dtoh(void *dst, const void *src, size_t bytes) {

@@ -1,0 +1,189 @@
+// device_pool.cpp -- see device_pool.hpp.
+#include <cstring>
+#include <list>
+#include <mutex>
+#include <unordered_map>
+
+#include "device_pool.hpp"
+
+namespace swift {
+
+namespace {
+
+struct Block {
+    void *ptr;
+    size_t size;
+    int dev;
+    uint64_t freed;  // the pool's count of frees when it was kept
+};
+
+struct Pool {
+    std::mutex mu;
+    std::unordered_map<void *, Block> live;  // allocated here, in use
+    std::list<Block> kept;                   // oldest first
+    std::unordered_map<int, size_t> bytes;   // kept, by device
+    uint64_t frees = 0;
+};
+Pool &pool() {
+    static Pool *p = new Pool;  // lives until the process ends
+    return *p;
+}
+
+// sizes in steps of an eighth of their power of two, so that calls of slightly
+// different sizes share blocks
+size_t block_size(size_t bytes) {
+    size_t step = 256;
+    while (step * 16 <= bytes) step <<= 1;
+    return (bytes + step - 1) / step * step;
+}
+
+// hipFree's device is the block's own, whichever is current
+void drop(Pool &p, std::list<Block>::iterator it) {
+    p.bytes[it->dev] -= it->size;
+    (void)hipFree(it->ptr);
+    p.kept.erase(it);
+}
+
+}  // namespace
+
+static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (bytes > kPoolBlock && (e = hipMalloc(ptr, bytes)) != hipErrorOutOfMemory) return e;
+    Pool &p = pool();
+    std::lock_guard<std::mutex> lk(p.mu);
+    const size_t size = bytes > kPoolBlock ? bytes : block_size(bytes ? bytes : 1);
+    // the block kept last: the likeliest to be in the caches
+    for (auto it = p.kept.end(); it != p.kept.begin();) {
+        --it;
+        if (it->dev == dev && it->size == size) {
+            p.live[it->ptr] = *it;
+            *ptr = it->ptr;
+            p.bytes[dev] -= size;
+            p.kept.erase(it);
+            return hipSuccess;
+        }
+    }
+    if (bytes <= kPoolBlock) e = hipMalloc(ptr, size);
+    if (e == hipErrorOutOfMemory) {  // give back what this device keeps
+        (void)hipGetLastError();
+        for (auto it = p.kept.begin(); it != p.kept.end();) {
+            auto at = it++;
+            if (at->dev == dev) drop(p, at);
+        }
+        e = hipMalloc(ptr, size);
+    }
+    if (e == hipSuccess && size <= kPoolBlock) {
+        try {
+            p.live[*ptr] = Block{*ptr, size, dev, 0};
+        } catch (...) {  // not entered: pool_free hands it to hipFree
+        }
+    }
+    return e;
+}
+
+hipError_t pool_alloc(void **ptr, size_t bytes) {
+    hipError_t e;
+    try {
+        e = alloc_from_pool(ptr, bytes);
+    } catch (...) {  // no memory for the pool's own tables
+        e = hipMalloc(ptr, bytes ? bytes : 1);
+    }
+    if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
+    return e;
+}
+
+hipError_t pool_free(void *ptr) {
+    if (!ptr) return hipSuccess;
+    Pool &p = pool();
+    Block b{};
+    {
+        std::lock_guard<std::mutex> lk(p.mu);
+        auto it = p.live.find(ptr);
+        if (it == p.live.end()) return hipFree(ptr);
+        b = it->second;
+        p.live.erase(it);
+    }
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev != b.dev || hipDeviceSynchronize() != hipSuccess) {
+        (void)hipGetLastError();
+        return hipFree(ptr);
+    }
+    std::lock_guard<std::mutex> lk(p.mu);
+    b.freed = ++p.frees;
+    try {
+        p.bytes[dev] += b.size;
+        p.kept.push_back(b);
+    } catch (...) {
+        p.bytes[dev] -= b.size;
+        return hipFree(ptr);
+    }
+    for (auto it = p.kept.begin(); it != p.kept.end();) {
+        auto at = it++;
+        if (at->freed + kPoolAge < p.frees || (at->dev == dev && p.bytes[dev] > kPoolBytes))
+            drop(p, at);
+    }
+    return hipSuccess;
+}
+
+// ---------------------------------------------------------------------------
+namespace {
+
+constexpr size_t kStageBytes = (size_t)1 << 20;
+constexpr int kStages = 2;
+
+// One a process: a second thread's copy meanwhile takes hipMemcpy.
+struct Stage {
+    std::mutex mu;
+    int dev = -1;  // whose stream and events these are
+    void *buf[kStages] = {};
+    hipStream_t st = nullptr;
+    hipEvent_t done[kStages] = {};
+
+    hipError_t ready(int d) {
+        if (dev == d) return hipSuccess;
+        if (dev != -1) return hipErrorInvalidDevice;
+        hipError_t e = hipSuccess;
+        for (int i = 0; i < kStages && e == hipSuccess; ++i) {
+            if (!buf[i]) e = hipHostMalloc(&buf[i], kStageBytes, hipHostMallocDefault);
+            if (e == hipSuccess && !done[i])
+                e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
+        }
+        if (e == hipSuccess && !st) e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+        if (e == hipSuccess) dev = d;
+        return e;
+    }
+};
+Stage &stage() {
+    static Stage *s = new Stage;  // lives until the process ends
+    return *s;
+}
+
+}  // namespace
+
+hipError_t copy_to_device(void *dst, const void *src, size_t bytes) {
+    Stage &s = stage();
+    int dev = 0;
+    std::unique_lock<std::mutex> lk(s.mu, std::defer_lock);
+    if (bytes < kStageMin || !dst || !src || hipGetDevice(&dev) != hipSuccess || !lk.try_lock())
+        return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+    if (s.ready(dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+    }
+    hipError_t e = hipStreamSynchronize(nullptr);
+    int i = 0;
+    for (size_t at = 0; at < bytes && e == hipSuccess; at += kStageBytes, i ^= 1) {
+        const size_t n = bytes - at < kStageBytes ? bytes - at : kStageBytes;
+        if (at >= kStages * kStageBytes) e = hipEventSynchronize(s.done[i]);
+        if (e != hipSuccess) break;
+        std::memcpy(s.buf[i], (const char *)src + at, n);
+        e = hipMemcpyAsync((char *)dst + at, s.buf[i], n, hipMemcpyHostToDevice, s.st);
+        if (e == hipSuccess) e = hipEventRecord(s.done[i], s.st);
+    }
+    const hipError_t end = hipStreamSynchronize(s.st);  // the buffers are free again
+    return e != hipSuccess ? e : end;
+}
+
+}  // namespace swift

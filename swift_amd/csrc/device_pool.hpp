@@ -1,0 +1,29 @@
+// device_pool.hpp -- device memory kept between owners, and host-to-device
+// copies through pinned staging.
+#pragma once
+
+#include "swift_common.hpp"
+
+namespace swift {
+
+// hipMalloc maps memory and hipFree unmaps it behind a device synchronisation:
+// 20-60 us and up to 0.7 ms a call, 3 ms of the 6.8 that indexing 50 Mbp and
+// aligning 20,000 reads took.  Freed blocks are kept instead (at most
+// kPoolBytes a device, none above kPoolBlock, none left unused for kPoolAge
+// frees) and given back when an allocation fails.  A block is kept once the
+// device is idle, as hipFree would leave it, so its next owner may use it on
+// any stream.  Safe from any thread.
+constexpr size_t kPoolBytes = (size_t)1 << 30;
+constexpr size_t kPoolBlock = (size_t)256 << 20;
+constexpr uint64_t kPoolAge = 256;
+hipError_t pool_alloc(void **ptr, size_t bytes);
+hipError_t pool_free(void *ptr);  // null, or what pool_alloc or hipMalloc returned
+
+// hipMemcpy from pageable memory.  The runtime stages 1 MiB at a time, host copy
+// and transfer in turn (20 GB/s); from kStageMin bytes on the host copies one
+// pinned buffer while the other is on its way.  Ordered as hipMemcpy: after the
+// null stream's earlier work, done on return.
+constexpr size_t kStageMin = (size_t)4 << 20;
+hipError_t copy_to_device(void *dst, const void *src, size_t bytes);
+
+}  // namespace swift

@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "../../include/swift_abi.h"
+#include "device_pool.hpp"
 #include "phase1.hpp"
 #include "sw_host.hpp"
 
@@ -17,12 +18,12 @@ struct DevArr {
     size_t bytes = 0;
     int alloc(size_t b) {
         release();
-        SWIFT_HIP_TRY(hipMalloc(&ptr, b ? b : 1));
+        SWIFT_HIP_TRY(pool_alloc(&ptr, b));
         bytes = b;
         return kOk;
     }
     void release() {
-        if (ptr) (void)hipFree(ptr);
+        (void)pool_free(ptr);
         ptr = nullptr;
         bytes = 0;
     }
