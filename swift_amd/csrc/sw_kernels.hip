@@ -162,7 +162,7 @@ __device__ __forceinline__ void run_task(const BatchArgs &a, const Task &tk, uin
         // 256: a row past the query (no match anywhere)
         auto conv = [&](uint32_t c) -> uint32_t {
             if constexpr (LEAN)
-                return PK ? lean_table(c, c > 255u, (uint32_t)a.kc.pm) : rail_query(c & 255u, c > 255u);
+                return PK ? lean_table(c, c > 255u, (uint32_t)a.kc.ppm) : rail_query(c & 255u, c > 255u);
             else
                 return c > 255u ? 0u : PK ? query_table(query_mask_bf((unsigned char)c))
                                           : byte_qcode((unsigned char)c);

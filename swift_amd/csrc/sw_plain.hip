@@ -4,7 +4,7 @@
 // reference at refSeq + p*(rlen+1), columns stopping at its first NUL.
 //
 // Four routes, by scoring and size (PlainPlan):
-//  * packed: the scorings of lean_scoring whose best score stays below the
+//  * packed: the scorings of lean_packed_scoring whose best score stays below the
 //    packed limit, from kPlainPackedPairs pairs on: the screen
 //    (sw_screen.hpp), then for the pairs it leaves, listed, the batched path's
 //    sweep, eight a wave (sw_plain_packed_kernel), walk and expansion.
@@ -285,7 +285,7 @@ sw_plain_packed_kernel(const char *__restrict__ qseq, const char *__restrict__ r
         for (int r = 0; r < R; ++r) {
             const int row = g * R + r;
             const uint32_t c = row < qlen ? (unsigned char)qs[row] : 0u;
-            const uint32_t tb = lean_table(c, row >= qlen, (uint32_t)kc.pm);
+            const uint32_t tb = lean_table(c, row >= qlen, (uint32_t)kc.ppm);
             if (h) sw.q2[r] = tb;
             else sw.q[r] = tb;
         }

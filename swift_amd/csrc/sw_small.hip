@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(256) sw_small_kernel(SmallArgs a) {
                 for (int r = 0; r < R; ++r) {
                     const int row = g * R + r;
                     const uint32_t c = row < ql[h] ? (unsigned char)qs[h][row] : 0u;
-                    const uint32_t tb = lean_table(c, row >= ql[h], (uint32_t)a.kc.pm);
+                    const uint32_t tb = lean_table(c, row >= ql[h], (uint32_t)a.kc.ppm);
                     if (h) sw.q2[r] = tb;
                     else sw.q[r] = tb;
                 }

@@ -269,24 +269,28 @@ struct Sweep {
 };
 
 // ---------------------------------------------------------------------------
-// The lean sweep, for the scorings of lean_scoring: the same staggered
-// recurrence, keys and trace codes as Sweep in fewer and cheaper
-// instructions.
+// The lean sweep, for the scorings of lean_scoring (packed lanes:
+// lean_packed_scoring): the same staggered recurrence and trace codes as Sweep in
+// fewer instructions.
 //
-// What bounds a sweep is VALU issue.  Measured issue cost a wave (cycles per
-// SIMD): and/or/xor/add/sub and mov 2.3-2.5, everything else used here (packed
-// 16-bit, 3-operand, v_perm, shifts, max) 4.2-4.5.  A row of two packed cells
-// costs Sweep 15 instructions and about 57 cycles, this one 12.3 and 47:
+// What bounds a sweep is VALU issue, about 4 SIMD cycles an instruction
+// whichever it is (a form with 32-bit subtracts for the packed ones, 2.3 cycles
+// alone, and one more maximum a row took 7 % more).  A step of 10 rows of two
+// packed cells takes 125 instructions here, 166 in Sweep:
 //  * A cell's key is one v_pk_maximum3_f16 (v_max3_u32 in 32-bit lanes) of its
 //    three candidates.  Every candidate is kept >= 0 by saturating subtracts,
 //    which makes the zero candidate implicit, and non-negative keys below
 //    0x7C00 order as half-precision bit patterns exactly as integers do.
 //  * Exits are key - penalty[direction], the penalty a byte picked by
 //    v_perm_b32 with the direction code itself as selector: the selector's
-//    zero bytes pick entry 0, which is 0 (a start's key is 0, so what is
-//    subtracted from it does not matter).
+//    high bytes pick a 0.  A start's key and penalty are 0.
+//  * Packed keys are 8H + direction, and c = 4 + (3 - direction), one v_bitop3,
+//    is both that selector (the table in the perm's upper word) and, as key ^ c
+//    is 8H + 7, all it takes to make x in one v_xad: an instruction a row less
+//    than keys of 4H, whose bits are masked and added to.  The trace word sums
+//    the rows' c and is put right once a step.
 //  * The match test's v_perm_b32 yields the mismatch penalty (0 or pm), so the
-//    diagonal candidate is one saturating subtract from x = 4H + 4*match + 3.
+//    diagonal candidate is one saturating subtract from x.
 //  * The best cell is kept per lane, not per row: each step's maximum over
 //    the rows of 32H + row code (smaller rows larger codes), and the first
 //    step at which it rose.  That is the lane's first maximum in row-major
@@ -294,15 +298,17 @@ struct Sweep {
 //    larger classes onto a SIMD.
 //  * Four steps a loop turn: their columns read together, their trace words
 //    stored 16 bytes a lane.
-// Sweep kernels before and after: 1.0M pairs of 150 x 300 (R = 10) 11.8 ->
-// 9.4 ms, 439k of 100 x 300 (R = 7) 3.89 -> 3.05 ms, 64 pairs up to 300 x 480
-// in the wide form 137 -> 79 us.  kLeanWide (scores of 960 to 2,016) takes 2 %
-// more cycles: a call of 100,000 pairs of 101-319 bases at 5, -4, -12, -2 with 5
-// % re-run 2.88 -> 2.51 ms.
+// Sweep kernels, Sweep -> keys of 4H -> 8H: 1.0M pairs of 150 x 300 (R = 10) 11.8
+// -> 9.4 ms, 768,000 of them 7.05 -> 6.65; 323,000 of 100 x 300 (R = 7) 2.35 ->
+// 2.29; 64 pairs up to 300 x 480 in the wide form 137 -> 79 us.  kLeanWide (scores
+// of 960 to 2,016) takes 2 % more cycles: a call of 100,000 pairs of 101-319 bases
+// at 5, -4, -12, -2 with 5 % re-run 2.88 -> 2.51 ms.
 // No step is masked: cells left of column 1 keep H = 0; cells right of a
 // pair's last column and rows below its query never match (padding
 // selectors, bit 7 of a padding row's table), so they score strictly below
-// the pair's best cell.
+// the pair's best cell.  (A packed padding cell's diagonal loses 255, which
+// leaves its key 4 past a multiple of 8: half a score, which stays among padding
+// cells, as none leads back into the matrix.)
 // ---------------------------------------------------------------------------
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
@@ -356,24 +362,30 @@ struct Lean {
     static constexpr int W = (R + KPW - 1) / KPW;     // trace words per step
     static constexpr uint32_t CMASK = PK ? 0x00030003u : 3u;
     static constexpr int CTRL = G == 16 ? kRowShr1 : kWaveShr1;
-    // row r = block * B + k: codes 3 - block (2 bits), B - 1 - k (3 bits)
-    static constexpr int B = (R + 3) / 4;
-    static_assert(B <= 8, "row codes");
+    // row r = block * B + k, coded so that smaller rows are larger: NB blocks,
+    // below the key's H; B - 1 - k, KB bits
+    static constexpr int NB = PK ? 8 : 4, KB = PK ? 2 : 3;
+    static constexpr int B = (R + NB - 1) / NB;
+    static_assert(B <= 1 << KB, "row codes");
 
     uint32_t q[R];             // PK: match tables of half 0; else dual-rail bytes
     uint32_t q2[PK ? R : 1];   // PK: match tables of half 1
-    uint32_t x[R];             // 4H + 4*match + 3 of (row, j-1)
+    uint32_t x[R];             // u(H + match) + 3 of (row, j-1); u = 8 packed, else 4
     uint32_t el[R];            // left exit of (row, j-1)
     uint32_t x_top, eu_last;
     uint32_t best, tbest;      // best key and the step of its first cell
-    uint32_t c_x, c_sign, tab_u, tab_l, pm;
+    uint32_t c_x, c_sign, tab_u, tab_l, pm, c_add, c_four;
 
     __device__ __forceinline__ void init(const KeyConsts &k) {
-        c_x = splat<PK>(k.x);
+        c_x = splat<PK>(PK ? k.px : k.x);
         c_sign = splat<PK>(k.sign);
-        tab_u = k.tab_u;
-        tab_l = k.tab_l;
+        tab_u = PK ? k.ptab_u : k.tab_u;
+        tab_l = PK ? k.ptab_l : k.tab_l;
         pm = (uint32_t)k.pm;
+        if constexpr (PK) {
+            c_add = c_x - splat<true>(7);
+            c_four = opaque(splat<true>(4));  // kept a multiplier: one v_pk_mad per key
+        }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             x[r] = c_x;  // column 0: H = 0, start
@@ -381,19 +393,27 @@ struct Lean {
         }
         x_top = c_x;
         eu_last = 0;
-        best = 8u * (c_x - splat<PK>(3)) + splat<PK>(31);  // H = 0 at any row
+        best = first_key() + splat<PK>(31);  // H = 0 at any row
         tbest = 0;
+    }
+
+    // the key of H = 0 at the last row code
+    __device__ __forceinline__ uint32_t first_key() const {
+        return PK ? 4u * (c_x - splat<PK>(3)) : 8u * (c_x - 3u);
     }
 
     // One step on the reference code(s) rr of column t - g; tcode: t in every
     // element.
     __device__ __forceinline__ void step(uint32_t rr, uint32_t tcode, uint32_t *acc) {
-        // from the lane above (0 into a group's first lane, whose matrix row 0
-        // has H = 0: x = c_x, no up exit)
+        // from the lane above; a group's first lane sees matrix row 0 (H = 0: x =
+        // c_x, no up exit).  (No maximum with c_x: a padding cell's x may be less,
+        // and would take the other half's with it.)
         const uint32_t eu_in =
             (uint32_t)__builtin_amdgcn_update_dpp(0, (int)eu_last, CTRL, 0xF, 0xF, true);
-        const uint32_t x_in = max(
-            (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x[R - 1], CTRL, 0xF, 0xF, true), c_x);
+        const uint32_t x_in =
+            PK ? (uint32_t)__builtin_amdgcn_update_dpp((int)c_x, (int)x[R - 1], CTRL, 0xF, 0xF, false)
+               : max((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x[R - 1], CTRL, 0xF, 0xF, true),
+                     c_x);
         uint32_t diag[R];
 #pragma unroll
         for (int r = R - 1; r >= 0; --r) {
@@ -406,27 +426,47 @@ struct Lean {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const uint32_t K = vmax3<PK>(diag[r], el[r], eu);
-            const uint32_t c = K & CMASK;
-            acc[r / KPW] |= c << (2 * (r % KPW));
-            eu = vsub_sat<PK>(K, __builtin_amdgcn_perm(tab_u, tab_u, c));
-            el[r] = vsub_sat<PK>(K, __builtin_amdgcn_perm(tab_l, tab_l, c));
-            x[r] = (K & ~CMASK) + c_x;  // no half carries into the other
+            if constexpr (PK) {
+                const uint32_t c = (~K & CMASK) | c_four;  // 4 + (3 - direction)
+                acc[r / KPW] += c << (2 * (r % KPW));
+                eu = vsub_sat<true>(K, __builtin_amdgcn_perm(tab_u, 0u, c));
+                el[r] = vsub_sat<true>(K, __builtin_amdgcn_perm(tab_l, 0u, c));
+                x[r] = (K ^ c) + c_add;  // 8H + 7 + (8*match - 4)
+            } else {
+                const uint32_t c = K & CMASK;
+                acc[r / KPW] |= c << (2 * (r % KPW));
+                eu = vsub_sat<PK>(K, __builtin_amdgcn_perm(tab_u, tab_u, c));
+                el[r] = vsub_sat<PK>(K, __builtin_amdgcn_perm(tab_l, tab_l, c));
+                x[r] = (K & ~CMASK) + c_x;
+            }
+        }
+        if constexpr (PK) {
+            // the codes: what the rows' sums of 7 - direction fall short by
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                uint32_t sevens = 0;
+#pragma unroll
+                for (int k = 0; k < KPW && w * KPW + k < R; ++k) sevens += splat<true>(7) << (2 * k);
+                acc[w] = sevens - acc[w];
+            }
         }
         eu_last = eu;
         // the step's best key: rows of one k by block, then over k
         uint32_t kb[B];
 #pragma unroll
         for (int k = 0; k < B; ++k) {
-            uint32_t v[4];
+            uint32_t v[NB];
             int n = 0;
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+            for (int b = 0; b < NB; ++b)
                 if (b * B + k < R) v[n++] = x[b * B + k] - splat<PK>(b);
             uint32_t m = v[0];  // below 0x7C00 in either form
-            if (n == 2) m = vmax<PK>(m, v[1]);
-            if (n >= 3) m = vmax3<PK>(m, v[1], v[2]);
-            if (n == 4) m = vmax<PK>(m, v[3]);
-            if constexpr (PK) kb[k] = vmad<true>(m, splat<true>(8), splat<true>(B - 1 - k));
+            int i = 1;
+#pragma unroll
+            for (; i + 1 < n; i += 2) m = vmax3<PK>(m, v[i], v[i + 1]);
+            if (i < n) m = vmax<PK>(m, v[i]);
+            if constexpr (PK)
+                kb[k] = vmad<true>(m, c_four, splat<true>(16 + B - 1 - k));
             else kb[k] = (m << 3) + (uint32_t)(B - 1 - k);
         }
         uint32_t m = kb[0];
@@ -457,9 +497,9 @@ struct Lean {
     // best cell of the lane: H, its row within the lane (0-based), its step
     __device__ __forceinline__ void result(int half, uint32_t &h, int &r, int &t) const {
         const uint32_t s = 16u * (uint32_t)half, m = PK ? 0xFFFFu : ~0u;
-        const uint32_t k = ((best >> s) & m) - 8u * (((c_x >> s) & m) - 3u);
+        const uint32_t k = ((best >> s) & m) - ((first_key() >> s) & m);
         h = k >> 5;
-        r = (int)(3u - ((k >> 3) & 3u)) * B + B - 1 - (int)(k & 7u);
+        r = (int)(NB - 1 - ((k >> KB) & (NB - 1))) * B + B - 1 - (int)(k & ((1 << KB) - 1));
         t = (int)((tbest >> s) & m);
     }
 };

@@ -17,11 +17,14 @@ struct KeyConsts {
     // no sign-splat to turn a masked merge of packed halves into per-half
     // compares and selects
     int sign;
-    // lean sweeps (see Lean): the diagonal-ready addend 4*match + 3, the
-    // mismatch penalty 4*(match - mismatch), and the exits' penalties by the
-    // cell's direction code, one byte each
+    // lean sweeps (see Lean): the diagonal-ready value of H = 0, u*match + 3, the
+    // mismatch penalty u*(match - mismatch), and the exits' penalties, one byte
+    // each; u = 4 in 32-bit lanes, by the cell's direction code, and 8 in packed
+    // ones (p...), by 3 less the code
     int x, pm;
     uint32_t tab_u, tab_l;
+    int px, ppm;
+    uint32_t ptab_u, ptab_l;
 };
 
 // ONEHOT: flag = match,    dr = 4*mismatch + 3, dsub = 4*(match - mismatch)
@@ -45,11 +48,16 @@ inline KeyConsts make_consts(const Scoring &s, int policy) {
     k.pm = 4 * (s.match - s.mismatch);
     // exit = key - penalty: 4*(H + gap) + 2 (up) or + 1 (left) from 4*H + d;
     // d = 0 (a start, key 0) saturates whatever is subtracted
-    k.tab_u = k.tab_l = 0;
+    k.tab_u = k.tab_l = k.ptab_u = k.ptab_l = 0;
     for (int d = 1; d <= 3; ++d) {
-        k.tab_u |= (uint32_t)((d - 2 - 4 * (d == 2 ? s.gap_ext : s.gap_open)) & 0xFF) << (8 * d);
-        k.tab_l |= (uint32_t)((d - 1 - 4 * (d == 1 ? s.gap_ext : s.gap_open)) & 0xFF) << (8 * d);
+        const int up = d == 2 ? s.gap_ext : s.gap_open, left = d == 1 ? s.gap_ext : s.gap_open;
+        k.tab_u |= (uint32_t)((d - 2 - 4 * up) & 0xFF) << (8 * d);
+        k.tab_l |= (uint32_t)((d - 1 - 4 * left) & 0xFF) << (8 * d);
+        k.ptab_u |= (uint32_t)((d - 2 - 8 * up) & 0xFF) << (8 * (3 - d));
+        k.ptab_l |= (uint32_t)((d - 1 - 8 * left) & 0xFF) << (8 * (3 - d));
     }
+    k.px = 8 * s.match + 3;
+    k.ppm = 8 * (s.match - s.mismatch);
     return k;
 }
 
@@ -59,6 +67,10 @@ inline KeyConsts make_consts(const Scoring &s, int policy) {
 inline bool lean_scoring(const Scoring &s) {
     return s.match >= 1 && s.mismatch < 0 && s.match - s.mismatch <= 31 && s.gap_open <= -1 &&
            s.gap_open >= -63 && s.gap_ext <= -1 && s.gap_ext >= -63;
+}
+// ... of the packed ones, whose keys are 8*H + code
+inline bool lean_packed_scoring(const Scoring &s) {
+    return lean_scoring(s) && s.match - s.mismatch <= 15 && s.gap_open >= -31 && s.gap_ext >= -31;
 }
 // Forms of a sweep.  The packed lean ones keep best-cell keys 32*H + 32*match +
 // row code in 16 bits: kLean takes their maxima three at a time as
@@ -72,7 +84,7 @@ inline int lean_limit(int form, int match) { return (form == kLean ? 960 : 2016)
 // the packed form for queries of at most maxq bases (larger scores would be
 // re-run in 32-bit lanes)
 inline SweepForm packed_form(const Scoring &s, int maxq) {
-    if (!lean_scoring(s)) return kGeneralForm;
+    if (!lean_packed_scoring(s)) return kGeneralForm;
     const int64_t most = (int64_t)maxq * s.match;
     return most < lean_limit(kLean, s.match) ? kLean
            : most < lean_limit(kLeanWide, s.match) ? kLeanWide : kGeneralForm;

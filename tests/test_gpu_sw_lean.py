@@ -76,3 +76,19 @@ def test_batch_lean_edges(A, orc, sc, qmax, form):
         A.set_coarse_rows(rows)
         A.set_tuning(tune["waves_per_cu"], tune["allow_int16"], tune["walk_deferred"])
     check(got, orc.sw_batch(qs, rs, *sc, nthreads=8))
+
+
+# the packed rule's limits (match - mismatch 15, penalties of 31) and one past each
+@pytest.mark.parametrize("sc", [(14, -1, -31, -1), (1, -14, -31, -31), (1, -15, -10, -1),
+                                (1, -1, -32, -1), (2, -1, -16, -16), (2, -1, -5, -32)])
+@pytest.mark.parametrize("rows", [0, -1])
+def test_batch_packed_edges(A, orc, sc, rows):
+    rnd = random.Random(sum(sc))
+    qs, rs = edge_pairs(rnd, 1500, min(320, 900 // sc[0]), 400)
+    before = A.get_coarse_rows()
+    try:
+        A.set_coarse_rows(rows)
+        got = A.sw_batch(qs, rs, A.Scoring(*sc))
+    finally:
+        A.set_coarse_rows(before)
+    check(got, orc.sw_batch(qs, rs, *sc, nthreads=8))
