@@ -133,12 +133,13 @@ namespace {
 constexpr size_t kStageBytes = (size_t)1 << 20;
 constexpr int kStages = 2;
 
-// One a process: a second thread's copy meanwhile takes hipMemcpy.
+// One a process: a second thread's copy meanwhile takes hipMemcpy.  On the null
+// stream, as hipMemcpy: a stream of its own would hold one of the four hardware
+// queues that the batched path's streams want.
 struct Stage {
     std::mutex mu;
-    int dev = -1;  // whose stream and events these are
+    int dev = -1;  // whose events these are
     void *buf[kStages] = {};
-    hipStream_t st = nullptr;
     hipEvent_t done[kStages] = {};
 
     hipError_t ready(int d) {
@@ -150,7 +151,6 @@ struct Stage {
             if (e == hipSuccess && !done[i])
                 e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
         }
-        if (e == hipSuccess && !st) e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
         if (e == hipSuccess) dev = d;
         return e;
     }
@@ -172,17 +172,17 @@ hipError_t copy_to_device(void *dst, const void *src, size_t bytes) {
         (void)hipGetLastError();
         return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
     }
-    hipError_t e = hipStreamSynchronize(nullptr);
+    hipError_t e = hipSuccess;
     int i = 0;
     for (size_t at = 0; at < bytes && e == hipSuccess; at += kStageBytes, i ^= 1) {
         const size_t n = bytes - at < kStageBytes ? bytes - at : kStageBytes;
         if (at >= kStages * kStageBytes) e = hipEventSynchronize(s.done[i]);
         if (e != hipSuccess) break;
         std::memcpy(s.buf[i], (const char *)src + at, n);
-        e = hipMemcpyAsync((char *)dst + at, s.buf[i], n, hipMemcpyHostToDevice, s.st);
-        if (e == hipSuccess) e = hipEventRecord(s.done[i], s.st);
+        e = hipMemcpyAsync((char *)dst + at, s.buf[i], n, hipMemcpyHostToDevice, nullptr);
+        if (e == hipSuccess) e = hipEventRecord(s.done[i], nullptr);
     }
-    const hipError_t end = hipStreamSynchronize(s.st);  // the buffers are free again
+    const hipError_t end = hipStreamSynchronize(nullptr);  // the buffers are free again
     return e != hipSuccess ? e : end;
 }
 
