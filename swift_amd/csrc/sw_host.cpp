@@ -570,7 +570,9 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     auto pass_args = [&](int pass, const PairResult *prev, int f32, BinArgs &b, TaskArgs &t) {
         b = BinArgs{io.rseq, io.roff, io.qlen, io.rlen, prev, n, f32, w.bin_of.as<int32_t>(),
                     bins + (2 * pass) * kNumBins, cnt + kCntError, io.score, io.start, io.end,
-                    io.alen, coarse, pass == 0 && screen ? w.res.as<PairResult>() : nullptr};
+                    io.alen, coarse,
+                    wide ? kRBins : std::max(1, (io.maxq + kBatchG - 1) / kBatchG),
+                    pass == 0 && screen ? w.res.as<PairResult>() : nullptr};
         t = TaskArgs{bins + (2 * pass) * kNumBins, bins + (2 * pass + 1) * kNumBins,
                      segs + (3 * pass) * NS, segs + (3 * pass + 1) * NS,
                      segs + (3 * pass + 2) * NS, cnt + 4 * pass, cnt + 4 * pass + 1,

@@ -219,8 +219,10 @@ struct BinArgs {
     int32_t *score_out, *start_out, *end_out, *alen_out;
     // > 0: rows per lane rounded up to a multiple of `coarse` (kCoarseRows,
     // or kCoarseRowsSmall for the smallest batches: at most kRBins / coarse
-    // classes; exact, the extra rows are padding); 0: every R its own class
+    // classes; exact, the extra rows are padding) but not past max_rows, what
+    // the call's longest query takes; 0: every R its own class
     int coarse;
+    int max_rows;
     const PairResult *screened;  // null, or results in which kScreenedFlag leaves a pair out
 };
 

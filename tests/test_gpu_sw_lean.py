@@ -92,3 +92,19 @@ def test_batch_packed_edges(A, orc, sc, rows):
     finally:
         A.set_coarse_rows(before)
     check(got, orc.sw_batch(qs, rs, *sc, nthreads=8))
+
+
+# rows a lane capped at the longest query's, also where a call says less than that
+@pytest.mark.parametrize("qmax,said", [(100, 100), (161, 161), (177, 100), (33, 1)])
+def test_batch_coarse_cap(A, orc, qmax, said):
+    rnd = random.Random(qmax)
+    qs, rs = edge_pairs(rnd, 4300, qmax, 200)
+    before = A.get_coarse_rows()
+    try:
+        A.set_coarse_rows(1)
+        b = A.PairBatch(qs, rs)
+        b.maxq = said
+        b.run()
+    finally:
+        A.set_coarse_rows(before)
+    check(b.results(), orc.sw_batch(qs, rs, nthreads=8))
