@@ -434,6 +434,11 @@ constexpr int kPlainWaves = 4096;
 // 8,192 98 against 208; 250 x 450, 231 against 133, 238 against 237, 256
 // against 462.
 constexpr int kPlainPackedPairs = 4096;
+// Calls under this many pairs walk a wave a pair, others a lane.  Of a packed
+// call most pairs are the screen's: 40,000 of 100 x 300 275 -> 234 us, of 250 x 400
+// 811 -> 693, 100,000 of 100 x 300 388 -> 354 against the general route's line.
+constexpr int kPackedWalkPairs = 131072;
+constexpr int kGeneralWalkPairs = 16384;
 // longest references of the packed route (four groups' columns in LDS)
 constexpr int kPlainPackedCols = 1024;
 
@@ -587,7 +592,7 @@ hipError_t launch_plain(const PlainPlan &pl, const char *q, const char *r, const
         }
     }
     const int mw = pl.move_words, nmv = (mw + 63) / 64;
-    if (n < kWaveWalkPairs && nmv <= 5) {
+    if (n < (packed ? kPackedWalkPairs : kGeneralWalkPairs) && nmv <= 5) {
         auto k = nmv <= 1 ? sw_plain_walk_wave_kernel<1>
                  : nmv == 2 ? sw_plain_walk_wave_kernel<2>
                  : nmv == 3 ? sw_plain_walk_wave_kernel<3>
