@@ -35,7 +35,7 @@ int swift_device_free(void *ptr) {
     return kOk;
 }
 int swift_memcpy_htod(void *dst, const void *src, size_t bytes) {
-    SWIFT_HIP_TRY(copy_to_device(dst, src, bytes));
+    SWIFT_HIP_TRY(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
     return kOk;
 }
 int swift_memcpy_dtoh(void *dst, const void *src, size_t bytes) {

@@ -1,5 +1,4 @@
 // device_pool.cpp -- see device_pool.hpp.
-#include <cstring>
 #include <list>
 #include <mutex>
 #include <unordered_map>
@@ -125,65 +124,6 @@ hipError_t pool_free(void *ptr) {
             drop(p, at);
     }
     return hipSuccess;
-}
-
-// ---------------------------------------------------------------------------
-namespace {
-
-constexpr size_t kStageBytes = (size_t)1 << 20;
-constexpr int kStages = 2;
-
-// One a process: a second thread's copy meanwhile takes hipMemcpy.  On the null
-// stream, as hipMemcpy: a stream of its own would hold one of the four hardware
-// queues that the batched path's streams want.
-struct Stage {
-    std::mutex mu;
-    int dev = -1;  // whose events these are
-    void *buf[kStages] = {};
-    hipEvent_t done[kStages] = {};
-
-    hipError_t ready(int d) {
-        if (dev == d) return hipSuccess;
-        if (dev != -1) return hipErrorInvalidDevice;
-        hipError_t e = hipSuccess;
-        for (int i = 0; i < kStages && e == hipSuccess; ++i) {
-            if (!buf[i]) e = hipHostMalloc(&buf[i], kStageBytes, hipHostMallocDefault);
-            if (e == hipSuccess && !done[i])
-                e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
-        }
-        if (e == hipSuccess) dev = d;
-        return e;
-    }
-};
-Stage &stage() {
-    static Stage *s = new Stage;  // lives until the process ends
-    return *s;
-}
-
-}  // namespace
-
-hipError_t copy_to_device(void *dst, const void *src, size_t bytes) {
-    Stage &s = stage();
-    int dev = 0;
-    std::unique_lock<std::mutex> lk(s.mu, std::defer_lock);
-    if (bytes < kStageMin || !dst || !src || hipGetDevice(&dev) != hipSuccess || !lk.try_lock())
-        return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
-    if (s.ready(dev) != hipSuccess) {
-        (void)hipGetLastError();
-        return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
-    }
-    hipError_t e = hipSuccess;
-    int i = 0;
-    for (size_t at = 0; at < bytes && e == hipSuccess; at += kStageBytes, i ^= 1) {
-        const size_t n = bytes - at < kStageBytes ? bytes - at : kStageBytes;
-        if (at >= kStages * kStageBytes) e = hipEventSynchronize(s.done[i]);
-        if (e != hipSuccess) break;
-        std::memcpy(s.buf[i], (const char *)src + at, n);
-        e = hipMemcpyAsync((char *)dst + at, s.buf[i], n, hipMemcpyHostToDevice, nullptr);
-        if (e == hipSuccess) e = hipEventRecord(s.done[i], nullptr);
-    }
-    const hipError_t end = hipStreamSynchronize(nullptr);  // the buffers are free again
-    return e != hipSuccess ? e : end;
 }
 
 }  // namespace swift

@@ -1,5 +1,4 @@
-// device_pool.hpp -- device memory kept between owners, and host-to-device
-// copies through pinned staging.
+// device_pool.hpp -- device memory kept between owners.
 #pragma once
 
 #include "swift_common.hpp"
@@ -18,12 +17,5 @@ constexpr size_t kPoolBlock = (size_t)256 << 20;
 constexpr uint64_t kPoolAge = 256;
 hipError_t pool_alloc(void **ptr, size_t bytes);
 hipError_t pool_free(void *ptr);  // null, or what pool_alloc or hipMalloc returned
-
-// hipMemcpy from pageable memory.  The runtime stages 1 MiB at a time, host copy
-// and transfer in turn (20 GB/s); from kStageMin bytes on the host copies one
-// pinned buffer while the other is on its way.  Ordered as hipMemcpy: after the
-// null stream's earlier work, done on return.
-constexpr size_t kStageMin = (size_t)4 << 20;
-hipError_t copy_to_device(void *dst, const void *src, size_t bytes);
 
 }  // namespace swift

@@ -167,8 +167,8 @@ static int index_build(const char *bases, const int64_t *off, const int64_t *len
         int64_t n = len[s];
         while (e < nseq && off[e] == off[s] + n) n += len[e++];
         if (n > 0)
-            SWIFT_HIP_TRY(copy_to_device(ix->seq.as<char>() + ix->h_off[s], bases + off[s],
-                                         (size_t)n));
+            SWIFT_HIP_TRY(hipMemcpy(ix->seq.as<char>() + ix->h_off[s], bases + off[s], (size_t)n,
+                                    hipMemcpyHostToDevice));
         s = e;
     }
     {

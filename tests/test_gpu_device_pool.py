@@ -1,4 +1,4 @@
-"""Device memory kept between owners, and staged uploads."""
+"""Device memory kept between owners, and uploads of many sizes."""
 import ctypes as C
 import threading
 
@@ -8,7 +8,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-# below the staged size, at it, at whole and ragged staging buffers
+# below and past the sizes the runtime stages in one piece
 @pytest.mark.parametrize("n", [1, (4 << 20) - 1, 4 << 20, (5 << 20) + 1, (33 << 20) + 12345])
 def test_upload_round_trip(n):
     from swift_amd.device import DeviceBuffer
