@@ -14,6 +14,7 @@ struct Block {
     size_t size;
     int dev;
     uint64_t freed;  // the pool's count of frees when it was kept
+    bool leaving;    // in pool_free, on its way to the kept ones
 };
 
 struct Pool {
@@ -75,7 +76,7 @@ static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
     }
     if (e == hipSuccess && size <= kPoolBlock) {
         try {
-            p.live[*ptr] = Block{*ptr, size, dev, 0};
+            p.live[*ptr] = Block{*ptr, size, dev, 0, false};
         } catch (...) {  // not entered: pool_free hands it to hipFree
         }
     }
@@ -100,22 +101,38 @@ hipError_t pool_free(void *ptr) {
     {
         std::lock_guard<std::mutex> lk(p.mu);
         auto it = p.live.find(ptr);
-        if (it == p.live.end()) return hipFree(ptr);
-        b = it->second;
-        p.live.erase(it);
+        if (it == p.live.end()) {
+            // freed before: hipFree would unmap what the next owner is handed
+            for (const Block &k : p.kept)
+                if (k.ptr == ptr) return hipErrorInvalidValue;
+        } else if (it->second.leaving) {
+            return hipErrorInvalidValue;
+        } else {
+            it->second.leaving = true;
+            b = it->second;
+        }
     }
+    if (!b.ptr) return hipFree(ptr);
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev != b.dev || hipDeviceSynchronize() != hipSuccess) {
-        (void)hipGetLastError();
-        return hipFree(ptr);
-    }
-    std::lock_guard<std::mutex> lk(p.mu);
+    const bool idle = hipGetDevice(&dev) == hipSuccess && dev == b.dev &&
+                      hipDeviceSynchronize() == hipSuccess;
+    if (!idle) (void)hipGetLastError();
+    std::unique_lock<std::mutex> lk(p.mu);
+    p.live.erase(ptr);
     b.freed = ++p.frees;
-    try {
-        p.bytes[dev] += b.size;
-        p.kept.push_back(b);
-    } catch (...) {
-        p.bytes[dev] -= b.size;
+    b.leaving = false;
+    bool kept = false;
+    if (idle) {
+        try {
+            size_t &held = p.bytes[dev];
+            p.kept.push_back(b);
+            held += b.size;
+            kept = true;
+        } catch (...) {  // no memory for the pool's own tables
+        }
+    }
+    if (!kept) {
+        lk.unlock();
         return hipFree(ptr);
     }
     for (auto it = p.kept.begin(); it != p.kept.end();) {

@@ -1,0 +1,159 @@
+"""The pool of freed device memory (swift_amd/csrc/device_pool.cpp) on the CPU,
+over a HIP whose device memory is a table of addresses: what it hands out is
+mapped and has one owner, whatever is freed twice, elsewhere or too late."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "swift_amd", "csrc")
+
+HIP = r"""
+#pragma once
+#include <cstddef>
+#define __host__
+#define __device__
+#define __forceinline__ inline
+typedef int hipError_t;
+enum { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2 };
+typedef void *hipDeviceptr_t;
+typedef void *hipStream_t;
+hipError_t hipMalloc(void **p, size_t n);
+hipError_t hipFree(void *p);
+hipError_t hipGetDevice(int *d);
+hipError_t hipDeviceSynchronize();
+hipError_t hipGetLastError();
+hipError_t hipMemGetAddressRange(hipDeviceptr_t *base, size_t *size, hipDeviceptr_t p);
+const char *hipGetErrorString(hipError_t e);
+"""
+
+MEMORY = r"""
+#include <map>
+#include <mutex>
+#include "device_pool.hpp"
+static std::recursive_mutex mu;
+static std::map<char *, size_t> mapped;
+static size_t in_use, limit = ~(size_t)0;
+static int device, last;
+static void (*on_sync)();
+hipError_t hipMalloc(void **p, size_t n) {
+    std::lock_guard<std::recursive_mutex> lk(mu);
+    if (n > limit - in_use) return last = hipErrorOutOfMemory;
+    char *at = (char *)0x100000;  // the lowest gap
+    for (auto &m : mapped) {
+        if (m.first >= at + n) break;
+        at = m.first + m.second;
+    }
+    mapped[at] = n;
+    in_use += n;
+    *p = at;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p) {
+    std::lock_guard<std::recursive_mutex> lk(mu);
+    auto it = mapped.find((char *)p);
+    if (it == mapped.end()) return last = hipErrorInvalidValue;
+    in_use -= it->second;
+    mapped.erase(it);
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int *d) { *d = device; return hipSuccess; }
+hipError_t hipDeviceSynchronize() {
+    if (on_sync) { auto f = on_sync; on_sync = nullptr; f(); }
+    return hipSuccess;
+}
+hipError_t hipGetLastError() { int e = last; last = 0; return e; }
+hipError_t hipMemGetAddressRange(hipDeviceptr_t *base, size_t *size, hipDeviceptr_t p) {
+    std::lock_guard<std::recursive_mutex> lk(mu);
+    auto it = mapped.upper_bound((char *)p);
+    if (it == mapped.begin()) return last = hipErrorInvalidValue;
+    --it;
+    if ((char *)p >= it->first + it->second) return last = hipErrorInvalidValue;
+    *base = it->first;
+    *size = it->second;
+    return hipSuccess;
+}
+const char *hipGetErrorString(hipError_t) { return ""; }
+extern "C" {
+int t_alloc(void **p, size_t n) { return swift::pool_alloc(p, n); }
+int t_free(void *p) { return swift::pool_free(p); }
+int t_hip_malloc(void **p, size_t n) { return hipMalloc(p, n); }
+int t_hip_free(void *p) { return hipFree(p); }
+void t_limit(size_t n) { limit = n; }
+void t_device(int d) { device = d; }
+void t_on_sync(void (*f)()) { on_sync = f; }
+size_t t_mapped(void *p) {  // bytes mapped from p on, p the start of its block
+    auto it = mapped.find((char *)p);
+    return it == mapped.end() ? 0 : it->second;
+}
+}
+"""
+
+SYNC = C.CFUNCTYPE(None)
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    d = tmp_path_factory.mktemp("pool")
+    (d / "hip").mkdir()
+    (d / "hip" / "hip_runtime.h").write_text(HIP)
+    (d / "memory.cpp").write_text(MEMORY)
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", f"-I{d}", f"-I{CSRC}", "-o",
+                    str(d / "pool.so"), str(d / "memory.cpp"),
+                    os.path.join(CSRC, "device_pool.cpp")], check=True)
+    return d
+
+
+class Pool:
+    def __init__(self, so):
+        self.lib = C.CDLL(str(so))
+        for f in ("alloc", "hip_malloc"):
+            getattr(self.lib, "t_" + f).argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+        for f in ("free", "hip_free", "mapped"):
+            getattr(self.lib, "t_" + f).argtypes = [C.c_void_p]
+        self.lib.t_limit.argtypes = [C.c_size_t]
+        self.lib.t_mapped.restype = C.c_size_t
+
+    def alloc(self, n, how="alloc"):
+        p = C.c_void_p()
+        rc = getattr(self.lib, "t_" + how)(C.byref(p), n)
+        return p.value if rc == 0 else None
+
+    def __getattr__(self, name):
+        return getattr(self.lib, "t_" + name)
+
+
+@pytest.fixture
+def pool(library, tmp_path):
+    so = tmp_path / "pool.so"  # a library of its own: an empty pool
+    so.write_bytes((library / "pool.so").read_bytes())
+    return Pool(so)
+
+
+def test_kept_blocks_are_used_again(pool):
+    a = pool.alloc(1000)
+    assert pool.free(a) == 0 and pool.mapped(a) >= 1000
+    assert pool.alloc(1010) == a
+
+
+def test_second_free_is_refused(pool):
+    """... and unmaps nothing that the next owner is handed."""
+    a = pool.alloc(1000)
+    assert pool.free(a) == 0
+    assert pool.free(a) != 0
+    b = pool.alloc(1000)
+    assert b is not None and pool.mapped(b) >= 1000
+    assert pool.alloc(1000) != b
+
+
+def test_second_free_during_the_first(pool):
+    """The second comes while the first waits for the device."""
+    a = pool.alloc(1000)
+    got = []
+    again = SYNC(lambda: got.append(pool.free(a)))
+    pool.on_sync(again)
+    assert pool.free(a) == 0 and got and got[0] != 0
+    b = pool.alloc(1000)
+    assert pool.mapped(b) >= 1000 and pool.alloc(1000) != b
