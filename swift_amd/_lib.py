@@ -23,8 +23,8 @@ def lib() -> C.CDLL:
         L = C.CDLL(LIB_PATH)
         L.swift_last_error.restype = C.c_char_p
         L.swift_version.restype = C.c_char_p
-        for name in ("swift_device_alloc", "swift_device_free", "swift_memcpy_htod",
-                     "swift_memcpy_dtoh", "swift_memset_device", "swift_device_synchronize",
+        for name in ("swift_device_alloc", "swift_device_free", "swift_device_trim",
+                     "swift_memcpy_htod", "swift_memcpy_dtoh", "swift_memset_device", "swift_device_synchronize",
                      "swift_device_count", "swift_sw_batch", "swift_align_sequences",
                      "swift_sw_batch_stats", "swift_set_tuning", "swift_set_coarse_rows",
                      "swift_get_coarse_rows", "swift_set_map_mode", "swift_get_map_mode",

@@ -34,6 +34,10 @@ int swift_device_free(void *ptr) {
     SWIFT_HIP_TRY(pool_free(ptr));
     return kOk;
 }
+int swift_device_trim(void) {
+    SWIFT_HIP_TRY(pool_trim());
+    return kOk;
+}
 int swift_memcpy_htod(void *dst, const void *src, size_t bytes) {
     SWIFT_HIP_TRY(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
     return kOk;

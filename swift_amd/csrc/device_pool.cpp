@@ -44,6 +44,13 @@ void drop(Pool &p, std::list<Block>::iterator it) {
     p.kept.erase(it);
 }
 
+void drop_all(Pool &p, int dev) {
+    for (auto it = p.kept.begin(); it != p.kept.end();) {
+        auto at = it++;
+        if (at->dev == dev) drop(p, at);
+    }
+}
+
 }  // namespace
 
 static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
@@ -68,10 +75,7 @@ static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
     if (bytes <= kPoolBlock) e = hipMalloc(ptr, size);
     if (e == hipErrorOutOfMemory) {  // give back what this device keeps
         (void)hipGetLastError();
-        for (auto it = p.kept.begin(); it != p.kept.end();) {
-            auto at = it++;
-            if (at->dev == dev) drop(p, at);
-        }
+        drop_all(p, dev);
         e = hipMalloc(ptr, size);
     }
     if (e == hipSuccess && size <= kPoolBlock) {
@@ -90,6 +94,23 @@ hipError_t pool_alloc(void **ptr, size_t bytes) {
     } catch (...) {  // no memory for the pool's own tables
         e = hipMalloc(ptr, bytes ? bytes : 1);
     }
+    if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
+    return e;
+}
+
+hipError_t pool_trim() {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    Pool &p = pool();
+    std::lock_guard<std::mutex> lk(p.mu);
+    drop_all(p, dev);
+    return hipSuccess;
+}
+
+hipError_t device_malloc(void **ptr, size_t bytes) {
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipErrorOutOfMemory && pool_trim() == hipSuccess) e = hipMalloc(ptr, bytes);
     if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
     return e;
 }

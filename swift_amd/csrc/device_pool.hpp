@@ -9,7 +9,8 @@ namespace swift {
 // 20-60 us and up to 0.7 ms a call, 3 ms of the 6.8 that indexing 50 Mbp and
 // aligning 20,000 reads took.  Freed blocks are kept instead (at most
 // kPoolBytes a device, none above kPoolBlock, none left unused for kPoolAge
-// frees) and given back when an allocation fails.  A block is kept once the
+// frees) and given back when an allocation of this library fails, or by pool_trim
+// (swift_device_trim), which another allocator of the process may need.  A block is kept once the
 // device is idle, as hipFree would leave it, so its next owner may use it on
 // any stream.  Safe from any thread.
 constexpr size_t kPoolBytes = (size_t)1 << 30;
@@ -17,5 +18,9 @@ constexpr size_t kPoolBlock = (size_t)256 << 20;
 constexpr uint64_t kPoolAge = 256;
 hipError_t pool_alloc(void **ptr, size_t bytes);
 hipError_t pool_free(void *ptr);  // null, or what pool_alloc or hipMalloc returned
+hipError_t pool_trim();           // gives back what is kept on the current device
+// hipMalloc, for memory that the pool does not keep (workspaces): gives back
+// what the pool keeps before it fails
+hipError_t device_malloc(void **ptr, size_t bytes);
 
 }  // namespace swift

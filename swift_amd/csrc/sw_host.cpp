@@ -12,6 +12,7 @@
 #include <utility>
 #include <vector>
 
+#include "device_pool.hpp"
 #include "sw_host.hpp"
 #include "sw_types.hpp"
 
@@ -33,7 +34,7 @@ int DevBuf::ensure(size_t want) {
     ptr = nullptr;
     bytes = 0;
     size_t b = want + want / 8 + 256;
-    SWIFT_HIP_TRY(hipMalloc(&ptr, b));
+    SWIFT_HIP_TRY(device_malloc(&ptr, b));
     bytes = b;
     return kOk;
 }

@@ -9,6 +9,12 @@ import numpy as np
 from ._lib import check, lib
 
 
+def trim() -> None:
+    """Gives the freed device memory that the library keeps for its next
+    allocations back to the process."""
+    check(lib().swift_device_trim())
+
+
 class DeviceBuffer:
     """A HIP device allocation of `nbytes`."""
 

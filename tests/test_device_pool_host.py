@@ -79,6 +79,8 @@ const char *hipGetErrorString(hipError_t) { return ""; }
 extern "C" {
 int t_alloc(void **p, size_t n) { return swift::pool_alloc(p, n); }
 int t_free(void *p) { return swift::pool_free(p); }
+int t_device_malloc(void **p, size_t n) { return swift::device_malloc(p, n); }
+int t_trim() { return swift::pool_trim(); }
 int t_hip_malloc(void **p, size_t n) { return hipMalloc(p, n); }
 int t_hip_free(void *p) { return hipFree(p); }
 void t_limit(size_t n) { limit = n; }
@@ -109,7 +111,7 @@ def library(tmp_path_factory):
 class Pool:
     def __init__(self, so):
         self.lib = C.CDLL(str(so))
-        for f in ("alloc", "hip_malloc"):
+        for f in ("alloc", "hip_malloc", "device_malloc"):
             getattr(self.lib, "t_" + f).argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
         for f in ("free", "hip_free", "mapped"):
             getattr(self.lib, "t_" + f).argtypes = [C.c_void_p]
@@ -157,3 +159,38 @@ def test_second_free_during_the_first(pool):
     assert pool.free(a) == 0 and got and got[0] != 0
     b = pool.alloc(1000)
     assert pool.mapped(b) >= 1000 and pool.alloc(1000) != b
+
+
+def test_kept_memory_is_given_back(pool):
+    """To the library's own allocations, in the pool or beside it, before one
+    fails; to others by a trim, on the current device only."""
+    size = 1 << 20
+    pool.limit(4 * size)
+    blocks = [pool.alloc(size) for _ in range(4)]
+    for how in ("alloc", "device_malloc"):
+        for b in blocks:
+            assert pool.free(b) == 0
+        p = pool.alloc(3 * size, how)
+        assert p is not None
+        assert pool.alloc(2 * size, how) is None
+        assert pool.free(p) == 0 if how == "alloc" else pool.hip_free(p) == 0
+        blocks = [pool.alloc(size) for _ in range(4)]
+        assert None not in blocks
+    pool.device(1)
+    other = pool.alloc(0)
+    assert other is None  # no room: this device keeps nothing
+    pool.device(0)
+    for b in blocks:
+        assert pool.free(b) == 0
+    pool.device(1)
+    assert pool.trim() == 0 and pool.alloc(size, "hip_malloc") is None
+    pool.device(0)
+    assert pool.trim() == 0 and pool.alloc(4 * size, "hip_malloc") is not None
+
+
+def test_workspaces_ask_the_pool():
+    """No allocation of device memory in the library goes past the pool."""
+    for f in sorted(os.listdir(CSRC)):
+        text = open(os.path.join(CSRC, f)).read()
+        if not f.startswith("device_pool"):
+            assert "hipMalloc(" not in text, f
