@@ -49,7 +49,9 @@ const char *swift_version(void);
 int swift_device_count(int *count);
 int swift_device_alloc(void **ptr, size_t bytes);
 int swift_device_free(void *ptr);
-/* Freed device memory is kept for the library's next allocations (at most
+/* Memory of swift_device_alloc goes back through swift_device_free, not
+ * hipFree (swift_device_free also takes a pointer of hipMalloc, and frees it).
+ * Freed device memory is kept for the library's next allocations (at most
  * 1 GiB a GPU; given back by itself when one of them would fail).  This gives
  * it back on the current GPU now, for other allocators of the process. */
 int swift_device_trim(void);

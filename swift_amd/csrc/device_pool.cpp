@@ -37,10 +37,21 @@ size_t block_size(size_t bytes) {
     return (bytes + step - 1) / step * step;
 }
 
+// False once the caller has given the block's pointer to hipFree itself: its
+// address is then unmapped or another allocation's.
+bool mapped(const Block &b) {
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)b.ptr) == hipSuccess)
+        return base == (hipDeviceptr_t)b.ptr && size >= b.size;
+    (void)hipGetLastError();
+    return false;
+}
+
 // hipFree's device is the block's own, whichever is current
 void drop(Pool &p, std::list<Block>::iterator it) {
     p.bytes[it->dev] -= it->size;
-    (void)hipFree(it->ptr);
+    if (mapped(*it)) (void)hipFree(it->ptr);
     p.kept.erase(it);
 }
 
@@ -65,6 +76,11 @@ static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
     for (auto it = p.kept.end(); it != p.kept.begin();) {
         --it;
         if (it->dev == dev && it->size == size) {
+            if (!mapped(*it)) {
+                auto gone = it++;
+                drop(p, gone);
+                continue;
+            }
             p.live[it->ptr] = *it;
             *ptr = it->ptr;
             p.bytes[dev] -= size;
@@ -135,7 +151,7 @@ hipError_t pool_free(void *ptr) {
     }
     if (!b.ptr) return hipFree(ptr);
     int dev = 0;
-    const bool idle = hipGetDevice(&dev) == hipSuccess && dev == b.dev &&
+    const bool idle = hipGetDevice(&dev) == hipSuccess && dev == b.dev && mapped(b) &&
                       hipDeviceSynchronize() == hipSuccess;
     if (!idle) (void)hipGetLastError();
     std::unique_lock<std::mutex> lk(p.mu);

@@ -188,6 +188,27 @@ def test_kept_memory_is_given_back(pool):
     assert pool.trim() == 0 and pool.alloc(4 * size, "hip_malloc") is not None
 
 
+def test_pointers_given_to_hip_free(pool):
+    """A block the caller unmapped itself: a smaller allocation at its address
+    is not kept under the old size, and what is unmapped is not handed out."""
+    a = pool.alloc(100_000)
+    assert pool.hip_free(a) == 0
+    assert pool.free(a) != 0  # as hipFree answers
+    a = pool.alloc(100_000)
+    assert pool.hip_free(a) == 0
+    b = pool.alloc(1000, "hip_malloc")
+    assert b == a and pool.free(b) == 0
+    c = pool.alloc(100_000)
+    assert pool.mapped(c) >= 100_000
+    # freed here and there
+    assert pool.free(c) == 0 and pool.hip_free(c) == 0
+    d = pool.alloc(1000, "hip_malloc")
+    assert d == c
+    e = pool.alloc(100_000)
+    assert e != d and pool.mapped(e) >= 100_000
+    assert pool.trim() == 0 and pool.mapped(d) == 1000
+
+
 def test_workspaces_ask_the_pool():
     """No allocation of device memory in the library goes past the pool."""
     for f in sorted(os.listdir(CSRC)):
