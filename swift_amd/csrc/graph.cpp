@@ -105,9 +105,9 @@ int swift_pipeline_graph_check(swift_graph *h) {
         set_error("no graph");
         return kErrInvalid;
     }
-    int rc = map_check(h->gr.m, h->gr.last);
-    if (rc) return rc;
-    return sw_batch_check_in(h->gr.sws, h->gr.last);
+    const int swrc = sw_batch_check_in(h->gr.sws, h->gr.last);
+    const int rc = map_check(h->gr.m, h->gr.last);
+    return rc ? rc : swrc;
 }
 
 int swift_pipeline_graph_free(swift_graph *h) {

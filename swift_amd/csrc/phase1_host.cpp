@@ -535,7 +535,13 @@ int align_reads_in(MapWork &w, Workspace *sws, const IndexObj &ix, const ReadsDe
     int rc = align_prepare(w, ix, rd, max_read_len, max_hits, rec, &m, &p);
     if (rc) return rc;
     if ((rc = align_enqueue(m, p, sws, rd.nreads, max_read_len, sc, rec, st, true))) return rc;
-    return map_check(m, st);
+    int swrc = kOk;
+    if (sws) {
+        SWIFT_HIP_TRY(hipStreamSynchronize(st));
+        swrc = sw_batch_status_in(sws);
+    }
+    rc = map_check(m, st);
+    return rc ? rc : swrc;
 }
 
 // ---------------------------------------------------------------------------

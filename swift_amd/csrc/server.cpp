@@ -207,12 +207,13 @@ static int run_batch(Server &S, SrvSlot &sl, std::vector<SrvRequest *> &batch) {
         SWIFT_HIP_TRY(launch_serve_out(so, (int)cap, sl.st));
     }
     SWIFT_HIP_TRY(hipStreamSynchronize(sl.st));
+    const int swrc = sw_batch_status_in(sl.sws);
     int32_t n, mflags[2];
     int64_t packed;
     memcpy(&n, sl.pin_out.p, 4);
     memcpy(&packed, sl.pin_out.p + 8, 8);
     memcpy(mflags, sl.pin_out.p + 16, 8);
-    if ((rc = map_error(mflags[1]))) return rc;
+    if ((rc = map_error(mflags[1])) || (rc = swrc)) return rc;
     const ServeLayout lay = serve_layout(n, packed);
     const int32_t *col[kRecI32];
     for (int c = 0; c < kRecI32; ++c)

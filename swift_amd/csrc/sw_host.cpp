@@ -92,7 +92,7 @@ struct Workspace {
         int64_t steps[2 * kRBins];
         int32_t seg[2 * kRBins + 1];
         int32_t cnt[16];
-        int32_t small[kSmallFlags];  // written by the one-launch form
+        int32_t small[kSmallFlags];  // set by the one-launch form, cleared where they are read
     } *stage = nullptr;
     int32_t reruns_seen = 0;  // the one-launch form's counter after the last call that read it
     int cu_count = 0;
@@ -363,6 +363,7 @@ static int reserve_common(Workspace &w, int npairs) {
         void *p = nullptr;
         SWIFT_HIP_TRY(hipHostMalloc(&p, sizeof(Workspace::HostStage), hipHostMallocDefault));
         w.stage = static_cast<Workspace::HostStage *>(p);
+        std::memset(w.stage, 0, sizeof(*w.stage));
     }
     return kOk;
 }
@@ -422,15 +423,29 @@ int sw_batch_enqueue_in(Workspace *w, const BatchIO &io, const Scoring &sc, hipS
     return batch_run(*w, io, sc, st, false);
 }
 
+static int length_error() {
+    set_error("pair lengths beyond maxq/maxr or the batched limits (%d/%d)", kMaxBatchQ,
+              kMaxBatchR);
+    return kErrCapacity;
+}
+
+// Lengths the one-launch form has refused since this was last asked, its
+// kernels done: a pair left out has no outputs, and past a call that did not
+// wait for it there is no general path left to take it.
+int sw_batch_status_in(Workspace *w) {
+    if (!w->stage) return kOk;
+    volatile int32_t *flags = w->stage->small;
+    const bool bad = flags[kSmallError] || flags[kSmallLonger];
+    flags[kSmallError] = flags[kSmallLonger] = 0;
+    return bad ? length_error() : kOk;
+}
+
 int sw_batch_check_in(Workspace *w, hipStream_t st) {
     int32_t c[16];
     SWIFT_HIP_TRY(hipMemcpyAsync(c, w->counters.ptr, sizeof(c), hipMemcpyDeviceToHost, st));
     SWIFT_HIP_TRY(hipStreamSynchronize(st));
-    if (c[kCntError]) {
-        set_error("pair lengths beyond the batched limits (%d/%d)", kMaxBatchQ, kMaxBatchR);
-        return kErrCapacity;
-    }
-    return kOk;
+    const int rc = sw_batch_status_in(w);
+    return c[kCntError] ? length_error() : rc;
 }
 
 // A small call as one kernel (sw_small.hip).  *done: 0 when a pair was longer
@@ -481,7 +496,10 @@ static int batch_run_small(Workspace &w, const BatchIO &io, const Scoring &sc, S
         SWIFT_HIP_TRY(launch_zero(z, st));
     }
     volatile int32_t *flags = w.stage->small;
-    for (int i = 0; i < kSmallFlags; ++i) flags[i] = 0;
+    // (a call that does not wait leaves them to sw_batch_status_in: kernels of
+    // the call before may still set them)
+    if (final_sync)
+        for (int i = 0; i < kSmallFlags; ++i) flags[i] = 0;
     for (int i = 0; i < 2; ++i) SWIFT_HIP_TRY(mark(i, st, w.timed));
     if (screen)
         SWIFT_HIP_TRY(launch_screen(
@@ -496,11 +514,7 @@ static int batch_run_small(Workspace &w, const BatchIO &io, const Scoring &sc, S
     *done = 1;
     if (!final_sync) return kOk;
     SWIFT_HIP_TRY(hipStreamSynchronize(st));
-    if (flags[kSmallError]) {
-        set_error("pair lengths beyond maxq/maxr or the batched limits (%d/%d)", kMaxBatchQ,
-                  kMaxBatchR);
-        return kErrCapacity;
-    }
+    if (flags[kSmallError]) return length_error();
     if (flags[kSmallLonger]) *done = 0;
     if (flags[kSmallRerun]) {
         int32_t now = 0;
@@ -687,11 +701,7 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
                                     steps1))) {
             return rc;
         }
-        if (w.stage->cnt[kCntError]) {
-            set_error("pair lengths beyond maxq/maxr or the batched limits (%d/%d)", kMaxBatchQ,
-                      kMaxBatchR);
-            return kErrCapacity;
-        }
+        if (w.stage->cnt[kCntError]) return length_error();
         if ((rc = w.trace.ensure((size_t)words1 * 4 + 4))) return rc;
         w.stats.ntasks16 = force32 ? 0 : seg1[kRBins];
         w.stats.ntasks32 = seg1[2 * kRBins] - seg1[kRBins];

@@ -98,7 +98,9 @@ int reserve_batch(int npairs, int maxq, int maxr);
 // Private batched-SW workspaces (device buffers, side streams), so that
 // several batches can be in flight at once, each driven by its own host
 // thread on its own stream.  sw_batch_run_in sizes the trace on the device
-// (it synchronises `st`).
+// (it synchronises `st`) and reports lengths beyond the batched limits; a small
+// call does neither, and the caller asks sw_batch_status_in once it has
+// waited for `st`: an error too where a pair is longer than maxq or maxr.
 struct Workspace;
 // side_streams: row-class kernels spread over that many private streams
 // (0..3); 0 runs them one after another on the caller's stream
@@ -109,10 +111,12 @@ void workspace_free(Workspace *w);
 void workspace_set_waves(Workspace *w, int waves_per_cu);
 int64_t workspace_bytes(const Workspace *w);
 int sw_batch_run_in(Workspace *w, const BatchIO &io, const Scoring &sc, hipStream_t st);
+int sw_batch_status_in(Workspace *w);
 // Capturable form: no host synchronisation, no allocation (reserve_batch_in
 // first, for at least this npairs / maxq / maxr); every row class is launched
-// and empty ones exit at once.  sw_batch_check_in reads the length-error flag
-// afterwards (it synchronises `st`).
+// and empty ones exit at once.  sw_batch_check_in reads the length-error flags
+// afterwards (it synchronises `st`): of the last run and, of small calls, of
+// every one since the last check.
 int reserve_batch_in(Workspace *w, int npairs, int maxq, int maxr);
 int sw_batch_enqueue_in(Workspace *w, const BatchIO &io, const Scoring &sc, hipStream_t st);
 int sw_batch_check_in(Workspace *w, hipStream_t st);

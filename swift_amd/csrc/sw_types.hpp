@@ -145,7 +145,7 @@ struct BatchArgs {
 };
 
 // One-launch form of a small batched call (sw_small.hip).  flags: mapped host
-// words, zeroed by the host before the launch.
+// words, cleared by the host where it reads them.
 enum SmallFlag { kSmallError = 0, kSmallLonger = 1, kSmallRerun = 2, kSmallFlags = 3 };
 struct SmallArgs {
     const char *qseq;
