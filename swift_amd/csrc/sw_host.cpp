@@ -357,6 +357,9 @@ static int reserve_common(Workspace &w, int npairs) {
     if (!w.counters.ptr) {
         if ((rc = w.counters.ensure(256 * 4))) return rc;
         SWIFT_HIP_TRY(hipMemset(w.counters.ptr, 0, 256 * 4));
+        // done before the caller's stream, which need not wait for the null
+        // stream, counts in them
+        SWIFT_HIP_TRY(hipStreamSynchronize(nullptr));
     }
     if ((rc = w.totals.ensure((size_t)(kTotSteps + 2 * 2 * kRBins) * 8))) return rc;
     if (!w.stage) {

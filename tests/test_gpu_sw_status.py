@@ -32,19 +32,20 @@ class Path:
              "status": "_ZN5swift18sw_batch_status_inEPNS_9WorkspaceE",
              "new": "_ZN5swift13workspace_newEi", "free": "_ZN5swift14workspace_freeEPNS_9WorkspaceE"}
 
-    def __init__(self, npairs, maxq, maxr):
+    def __init__(self, npairs=0, maxq=0, maxr=0):
         from swift_amd._lib import lib
         from swift_amd.device import Stream
         self.f = {k: getattr(lib(), v) for k, v in self.NAMES.items()}
         self.f["new"].restype = C.c_void_p
         self.st = Stream()
         self.w = C.c_void_p(self.f["new"](0))
-        assert self.f["reserve"](self.w, npairs, maxq, maxr) == 0
+        if npairs:
+            assert self.f["reserve"](self.w, npairs, maxq, maxr) == 0
 
-    def call(self, how, b, sc):
+    def call(self, how, b, sc, sparse=1):
         io = BatchIO(b.q.ptr, b.qo.ptr, b.ql.ptr, b.r.ptr, b.ro.ptr, b.rl.ptr, b.n, b.maxq,
                      b.maxr, b.score.ptr, b.start.ptr, b.end.ptr, b.alen.ptr, b.qc.ptr, b.rc.ptr,
-                     b.co.ptr, 0, 1)
+                     b.co.ptr, 0, sparse)
         rc = self.f[how](self.w, C.byref(io), C.byref(Scoring(*sc)), self.st.cptr)
         if rc:
             return rc
@@ -98,3 +99,19 @@ def test_longer_than_said_is_not_passed_over(orc, how):
         check(b.results(), orc.sw_batch(qs, rs, nthreads=8))
     finally:
         p.close()
+
+
+def test_first_calls(orc):
+    """The first call of a workspace, which makes its counters, on a stream that
+    does not wait for the null stream: the screen and the kernel on its list."""
+    qs, rs = edge_pairs(random.Random(3), 4100, 100, 160)
+    want = orc.sw_batch(qs, rs, nthreads=8)
+    from swift_amd import align as A
+    b = A.PairBatch(qs, rs)
+    for _ in range(6):
+        p = Path()
+        try:
+            assert p.call("run", b, (2, -1, -10, -1), 0) == 0
+            check(b.results(), want)
+        finally:
+            p.close()
