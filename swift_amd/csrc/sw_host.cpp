@@ -452,9 +452,11 @@ int sw_batch_check_in(Workspace *w, hipStream_t st) {
 }
 
 // A small call as one kernel (sw_small.hip).  *done: 0 when a pair was longer
-// than the call said and the general path has to run.
+// than the call said, or the screen left more than kSmallLeft, and the general
+// path has to run; *screened: the screen's answers are in w.res.
 static int batch_run_small(Workspace &w, const BatchIO &io, const Scoring &sc, SweepForm form,
-                           const KeyConsts &kc, uint32_t h_limit, hipStream_t st, bool final_sync, int *done) {
+                           const KeyConsts &kc, uint32_t h_limit, hipStream_t st, bool final_sync,
+                           int *done, bool *screened) {
     const int n = io.npairs;
     SmallArgs a{};
     a.qseq = io.qseq;
@@ -489,15 +491,20 @@ static int batch_run_small(Workspace &w, const BatchIO &io, const Scoring &sc, S
     a.reruns = w.counters.as<int32_t>() + kCntReruns;
     // the screen first, and the one launch on what it leaves
     const bool screen = !io.sparse && n >= kSmallScreen;
+    a.most = n;
     if (screen) {
         a.list = w.order.as<int32_t>();
         a.nlist = w.counters.as<int32_t>() + kCntLeft;
+        if (final_sync) a.most = kSmallLeft;
         ZeroSpans z{};
         z.p[0] = w.counters.as<int32_t>() + kCntLeft;
         z.n[0] = 1;
-        z.nspans = 1;
+        z.p[1] = w.res.as<int32_t>();
+        z.n[1] = n * (int)(sizeof(PairResult) / 4);
+        z.nspans = 2;
         SWIFT_HIP_TRY(launch_zero(z, st));
     }
+    *screened = screen;
     volatile int32_t *flags = w.stage->small;
     // (a call that does not wait leaves them to sw_batch_status_in: kernels of
     // the call before may still set them)
@@ -507,8 +514,9 @@ static int batch_run_small(Workspace &w, const BatchIO &io, const Scoring &sc, S
     if (screen)
         SWIFT_HIP_TRY(launch_screen(
             ScreenArgs{io.qseq, io.qoff, io.qlen, io.rseq, io.roff, io.rlen, n, 1, io.score,
-                       io.start, io.end, io.alen, io.qcons, io.rcons, io.cons_off, nullptr,
-                       w.order.as<int32_t>(), w.counters.as<int32_t>() + kCntLeft},
+                       io.start, io.end, io.alen, io.qcons, io.rcons, io.cons_off,
+                       w.res.as<PairResult>(), w.order.as<int32_t>(),
+                       w.counters.as<int32_t>() + kCntLeft},
             sc, st));
     SWIFT_HIP_TRY(launch_small(a, blocks, st));
     for (int i = 2; i < 5; ++i) SWIFT_HIP_TRY(mark(i, st, w.timed));
@@ -518,7 +526,7 @@ static int batch_run_small(Workspace &w, const BatchIO &io, const Scoring &sc, S
     if (!final_sync) return kOk;
     SWIFT_HIP_TRY(hipStreamSynchronize(st));
     if (flags[kSmallError]) return length_error();
-    if (flags[kSmallLonger]) *done = 0;
+    if (flags[kSmallLonger] || flags[kSmallMany]) *done = 0;
     if (flags[kSmallRerun]) {
         int32_t now = 0;
         SWIFT_HIP_TRY(hipMemcpyAsync(&now, a.reruns, 4, hipMemcpyDeviceToHost, st));
@@ -608,13 +616,14 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     const bool lean32 = lean_scoring(sc);  // 32-bit lanes have no limit
     if (form16 != kGeneralForm) h_limit = 4u * (uint32_t)lean_limit(form16, sc.match);
 
+    bool screened = false;
     // a small call in one launch, unless row classes are asked for (coarse
     // ones below kCoarseTinyPairs are this form)
     if (form16 != kGeneralForm && !force32 && (cmode < 0 || (cmode == 1 && n < kCoarseTinyPairs)) &&
         small_call(n, io.maxq, io.sparse)) {
         int done = 0;
         if ((rc = batch_run_small(w, io, sc, form16, kc16, h_limit, st, sync_sizes && final_sync,
-                                  &done)) ||
+                                  &done, &screened)) ||
             done)
             return rc;
         w.stats = BatchStats{};
@@ -626,7 +635,7 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     {
         ZeroSpans z{};
         z.p[0] = w.res.as<int32_t>();
-        z.n[0] = n * (int)(sizeof(PairResult) / 4);
+        z.n[0] = screened ? 0 : n * (int)(sizeof(PairResult) / 4);
         z.p[1] = cnt + kCntError;
         z.n[1] = kCntQueues + 2 * kQueuesPerPass - kCntError;
         z.p[2] = bins;
@@ -637,7 +646,7 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
         SWIFT_HIP_TRY(launch_zero(z, st));
     }
     SWIFT_HIP_TRY(mark(0, st, w.timed));
-    if (screen)
+    if (screen && !screened)
         SWIFT_HIP_TRY(launch_screen(
             ScreenArgs{io.qseq, io.qoff, io.qlen, io.rseq, io.roff, io.rlen, n, 1, io.score,
                        io.start, io.end, io.alen, io.qcons, io.rcons, io.cons_off,

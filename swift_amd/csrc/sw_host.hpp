@@ -157,23 +157,32 @@ constexpr int kSmallWaves = 4096;   // each keeps a trace area
 // From this many pairs on the screen goes first (sw_screen.hip) and the one
 // launch takes what it leaves: two launches more, against the related pairs'
 // sweeps.  us a call without and with, queries of 50-300 bases beside their
-// places: 2,048 pairs 120, 130; 4,000 177, 142; 16,000 527, 335; of 100 bases
-// 59, 69; 78, 77; 219, 126.  Not where slots may be missing: most of a
+// places: 2,048 pairs 120, 130; 4,000 177, 133; 16,000 527, 294; of 100 bases
+// 59, 69; 78, 77; 219, 102.  Not where slots may be missing: most of a
 // pipeline's pairs are unrelated, and its small calls wait for launches.
 constexpr int kSmallScreen = 4000;
 // The one launch's waves take pairs unsorted, 64 lanes of ceil(maxq / 64) rows
 // each, against the general path's binning, readback and 16-lane groups: taken
-// up to kSmallWork = pairs x rows a lane.  us a call, general -> one launch,
-// both with the screen:
-//   50-300: 26,000 610 -> 438, 40,000 660 -> 583, 60,000 713 -> 793
-//   100: 60,000 319 -> 272
-// and of pairs the screen leaves, which sets the line below what those ask:
-//   50-300: 16,000 568 -> 526, 24,000 637 -> 752; 100: 40,000 659 -> 623
+// up to kSmallWork = pairs x rows a lane, and of those the screen leaves, which
+// only the device knows, up to kSmallLeft: with more the kernel's waves leave at
+// once and the host goes on to the general path, 30 us later than it would have.
+// us a call, general path -> one launch without that line, of pairs that are all
+// related, three in four of them unrelated, all unrelated:
+//   50-300 bases: 12,000 386 -> 256, 414 -> 397, 415 -> 433; 20,000 524 -> 323,
+//     607 -> 569, 617 -> 633; 26,000 575 -> 378, 634 -> 693, 639 -> 793
+//   100: 20,000 194 -> 115, 256 -> 250, 291 -> 287; 30,000 208 -> 142, 318 -> 356,
+//     362 -> 399; 60,000 275 -> 226, 526 -> 639, 586 -> 753
+//   150: 30,000 306 -> 241, 473 -> 485, 520 -> 536; 43,000 343 -> 314, 595 -> 645,
+//     703 -> 747
+//   300: 14,000 558 -> 407, 615 -> 519, 627 -> 604; 26,000 684 -> 621, 913 -> 870,
+//     1,002 -> 946
+// three rounds of the waves' pairs, two each, lie between the sides.
 // A pipeline's capacity counts slots of which a half or fewer hold records:
 // 5,000 reads of 300 bases (capacity 30,000) 1,052 -> 816 us, 13,000 of 100
 // 1,039 -> 995.
 constexpr int kSmallWork = 130000;
 constexpr int kSmallWorkSparse = 160000;
+constexpr int kSmallLeft = 3 * 2 * kSmallWaves;
 inline bool small_call(int npairs, int maxq, bool sparse) {
     const int64_t rows = maxq > 64 ? (maxq + 63) / 64 : 1;
     return npairs * rows <= (sparse ? kSmallWorkSparse : kSmallWork);

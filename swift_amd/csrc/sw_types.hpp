@@ -146,7 +146,7 @@ struct BatchArgs {
 
 // One-launch form of a small batched call (sw_small.hip).  flags: mapped host
 // words, cleared by the host where it reads them.
-enum SmallFlag { kSmallError = 0, kSmallLonger = 1, kSmallRerun = 2, kSmallFlags = 3 };
+enum SmallFlag { kSmallError = 0, kSmallLonger = 1, kSmallRerun = 2, kSmallMany = 3, kSmallFlags = 4 };
 struct SmallArgs {
     const char *qseq;
     const int64_t *qoff;
@@ -155,6 +155,7 @@ struct SmallArgs {
     const int64_t *roff;
     const int32_t *rlen;
     const int32_t *list, *nlist;  // or null: the pairs to take (of npairs at most)
+    int most;                 // with more than that on the list, none is taken
     int npairs, ppw, wpb;     // pairs, pairs a wave (1 or 2), waves a workgroup (<= 4)
     int maxq, maxr;
     int form;                 // kLean or kLeanWide

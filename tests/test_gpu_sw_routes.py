@@ -58,3 +58,17 @@ def test_list_of_unrelated_pairs(A, orc):
     finally:
         A.set_coarse_rows(before)
     assert took[-1] < 1.15 * took[1], took
+
+
+@pytest.mark.parametrize("related", [True, False])
+def test_one_launch_by_the_pairs_left(A, orc, related):
+    """A call within the one launch's line: taken by it where the screen answers
+    the pairs, handed on to the row classes where it leaves too many."""
+    n = 26_000
+    qs, rs = pairs(2, n, 30, 60, 60, related)
+    # one pair of three rows a lane: two pairs a workgroup
+    (qs[5],), (rs[5],) = pairs(3, 1, 170, 170, 20, False)
+    got = A.sw_batch(qs, rs)
+    tasks = A.batch_stats()["ntasks16"]
+    check(got, orc.sw_batch(qs, rs, nthreads=8))
+    assert tasks == n // 2 if related else tasks < n // 4
