@@ -82,7 +82,7 @@ int swift_align_sequences_noalloc(char *querySeq_d, char *refSeq_d, int querySeq
     bool f32;
     if ((rc = validate_scoring(sc, qlen, rlen, &f32))) return rc;
     if (npairs == 0) return kOk;
-    const PlainPlan pl = plain_plan(sc, qlen, rlen, npairs);
+    const PlainPlan pl = plain_plan(sc, qlen, rlen, npairs, kNoAllocWords);
     int chunk, waves;
     plain_chunk(pl, npairs, kNoAllocWords, &chunk, &waves);
     if (plain_words(pl, 1, 1) > kNoAllocWords) {

@@ -265,7 +265,7 @@ int align_sequences_status(char *q_d, char *r_d, int qlen, int rlen, float match
     bool f32;
     if ((rc = validate_scoring(sc, qlen, rlen, &f32))) return rc;
     Workspace &w = ws();
-    const PlainPlan pl = plain_plan(sc, qlen, rlen, npairs);
+    const PlainPlan pl = plain_plan(sc, qlen, rlen, npairs, (int64_t)g_plain_budget_words);
     int chunk, waves;
     plain_chunk(pl, npairs, (int64_t)g_plain_budget_words, &chunk, &waves);
     if (g_plain_chunk_pairs > 0) chunk = std::min(chunk, g_plain_chunk_pairs);

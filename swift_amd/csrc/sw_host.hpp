@@ -22,7 +22,8 @@ struct PlainPlan {
     int64_t task_words;           // trace of eight packed pairs
 };
 struct PlainOut;
-PlainPlan plain_plan(const Scoring &sc, int qlen, int rlen, int npairs);
+// budget: the words of scratch the call's chunks may take
+PlainPlan plain_plan(const Scoring &sc, int qlen, int rlen, int npairs, int64_t budget);
 // the largest chunk of at most npairs pairs that fits `budget` words of
 // scratch (one pair at least), with its waves of the wave kernel
 void plain_chunk(const PlainPlan &pl, int npairs, int64_t budget, int *chunk, int *waves);

@@ -430,9 +430,16 @@ static int64_t packed_trace_words(int R, int rlen) {
 constexpr int kPlainWaves = 4096;
 // Calls of at least this many pairs take the packed route, whose sixteen-lane
 // groups need eight times the pairs to fill the chip.  Packed (without the
-// screen) against wave route, us: 100 x 300 bases, 2,048 pairs 90 against 61, 4,096 94 against 104,
-// 8,192 98 against 208; 250 x 450, 231 against 133, 238 against 237, 256
-// against 462.
+// screen) against wave route, us: 100 x 300 bases, 2,048 pairs 90 against 61,
+// 4,096 94 against 104, 8,192 98 against 208; 250 x 450, 231 against 133, 238
+// against 237, 256 against 462.  Past 16 rows a lane (three trace words a step)
+// the chunks have to be as large: in a small scratch one is a task a wave on a
+// part of the chip, and lasts as long as that task.  With the screen, in 64 MiB,
+// 4,200 related (unrelated) pairs: 320 x 480, chunks of 1,048, 1,467 against 825
+// (1,495; 838); 300 x 200, 2,432, 308 against 256 (315; 254).  Of fewer rows the
+// packed route comes out even or ahead: 250 x 450, 1,664, 699 against 680 (725;
+// 672); 150 x 450, 1,664, 477 against 547 (497; 548); 120 x 1000, 1,528, 793
+// against 1,564 (802; 1,549).
 constexpr int kPlainPackedPairs = 4096;
 // Calls under this many pairs walk a wave a pair, others a lane.  Of a packed
 // call most pairs are the screen's: 40,000 of 100 x 300 275 -> 234 us, of 250 x 400
@@ -442,7 +449,7 @@ constexpr int kGeneralWalkPairs = 16384;
 // longest references of the packed route (four groups' columns in LDS)
 constexpr int kPlainPackedCols = 1024;
 
-PlainPlan plain_plan(const Scoring &sc, int qlen, int rlen, int npairs) {
+PlainPlan plain_plan(const Scoring &sc, int qlen, int rlen, int npairs, int64_t budget) {
     PlainPlan pl{};
     pl.qlen = qlen;
     pl.rlen = rlen;
@@ -460,6 +467,9 @@ PlainPlan plain_plan(const Scoring &sc, int qlen, int rlen, int npairs) {
     pl.route = packed ? PlainPlan::kPacked : PlainPlan::kWave;
     pl.packed_rows = std::max(1, (qlen + kBatchG - 1) / kBatchG);
     pl.task_words = packed_trace_words(pl.packed_rows, rlen);
+    int chunk, waves;
+    plain_chunk(pl, npairs, budget, &chunk, &waves);
+    if (packed && pl.packed_rows > 16 && chunk < kPlainPackedPairs) pl.route = PlainPlan::kWave;
     return pl;
 }
 
