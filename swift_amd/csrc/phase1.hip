@@ -1905,6 +1905,22 @@ hipError_t launch_index_build(const IndexDev &ix, int64_t ntup, const IndexBuild
     return hipGetLastError();
 }
 
+// [h0, h0 + n) of one of the per-hash arrays a caller reads back
+__global__ void __launch_bounds__(256) idx_export(IndexDev ix, IndexArray which, int64_t h0, int n,
+                                                  int32_t *out) {
+    const int i = blockIdx.x * 256 + (int)threadIdx.x;
+    if (i >= n) return;
+    const int2 b = bucket_of(ix, (uint32_t)(h0 + i));
+    out[i] = which == kIndexStart ? (b.y ? b.x : 0)
+             : which == kIndexActual || b.y ? b.y : ix.count[h0 + i];
+}
+
+hipError_t launch_index_export(const IndexDev &ix, IndexArray which, int64_t h0, int n,
+                               int32_t *out, hipStream_t st) {
+    hipLaunchKernelGGL(idx_export, dim3((n + 255) / 256), dim3(256), 0, st, ix, which, h0, n, out);
+    return hipGetLastError();
+}
+
 template <class K>
 static void launch_index_sort(const IndexDev &ix, const IndexBuildScratch &s, K *keys,
                               hipStream_t st) {

