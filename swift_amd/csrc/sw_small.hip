@@ -54,11 +54,9 @@ __global__ void __launch_bounds__(256) sw_small_kernel(SmallArgs a) {
     uint32_t *col = moves + 2 * mw;  // the columns, then the expansion's bases
     uint32_t *tr = a.trace + (int64_t)wave * a.wave_words;
     const int npairs = a.nlist ? uni(*a.nlist) : a.npairs;
-    if (npairs > a.most) {  // the host takes the general path
-        if (wave == 0 && g == 0) host_flag(a.flags + kSmallMany);
-        return;
-    }
-    const int ntask = (npairs + a.ppw - 1) / a.ppw;
+    // more than a.most: none, and the host takes the general path
+    const int ntask = npairs > a.most ? 0 : (npairs + a.ppw - 1) / a.ppw;
+    if (ntask == 0 && npairs > 0 && wave == 0 && g == 0) host_flag(a.flags + kSmallMany);
     for (int task = wave; task < ntask; task += nwaves) {
         int pid[2], ql[2], rl[2];
         const char *qs[2], *rs[2];
