@@ -7,12 +7,13 @@ namespace swift {
 
 // hipMalloc maps memory and hipFree unmaps it behind a device synchronisation:
 // 20-60 us and up to 0.7 ms a call, 3 ms of the 6.8 that indexing 50 Mbp and
-// aligning 20,000 reads took.  Freed blocks are kept instead (at most
-// kPoolBytes a device, none above kPoolBlock, none left unused for kPoolAge
-// frees) and given back when an allocation of this library fails, or by pool_trim
-// (swift_device_trim), which another allocator of the process may need.  A block is kept once the
-// device is idle, as hipFree would leave it, so its next owner may use it on
-// any stream.  Safe from any thread.
+// aligning 20,000 reads took, from a process's second run on (its first finds
+// nothing kept).  Freed blocks are kept instead (at most kPoolBytes a device,
+// none above kPoolBlock, none left unused for kPoolAge frees) and given back when
+// an allocation of this library fails, or by pool_trim (swift_device_trim), which
+// another allocator of the process may need.  A block is kept once the device is
+// idle, as hipFree would leave it, so its next owner may use it on any stream.
+// Safe from any thread.
 constexpr size_t kPoolBytes = (size_t)1 << 30;
 constexpr size_t kPoolBlock = (size_t)256 << 20;
 constexpr uint64_t kPoolAge = 256;

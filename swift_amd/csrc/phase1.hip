@@ -15,9 +15,9 @@
 //     rand() (src/mapHits6.cu:146-160); the mapper keeps the first maxHits,
 //     one member of the reference's tie set, and reports the set's size.
 //
-// Layout: the index lives in HBM as an int2 bucket table (start, kept count)
-// plus 64-bit entries (refIdx << 32 | refPos).  One wave maps one read
-// strand: lanes hash query offsets, a wave prefix sum lays the hits out, the
+// Layout: the index lives in HBM as the prefix array of the kept counts (a
+// bucket is two neighbours of it) plus 64-bit entries (refIdx << 32 | refPos).
+// In the tiers that sort, one wave maps one read strand: lanes hash query offsets, a wave prefix sum lays the hits out, the
 // wave gathers bucket entries cooperatively (one hit per lane), sorts 64-bit
 // hit keys in LDS and compacts the biggest clusters with ballots.  Strands
 // whose hits exceed LDS take the same steps in a global scratch slot with a
@@ -650,7 +650,10 @@ __global__ void __launch_bounds__(64) map_strands(MapArgs a) {
 //    is 1 every hit is its cluster.
 // The waves are persistent and load their next strand's bases during the
 // current one.  105,000 reads of 100 bases on 50 Mbp: the kernel
-// 0.90 -> 0.35 ms.
+// 0.90 -> 0.37 ms, a call 0.93 -> 0.44.  (A call took 20 us less with buckets of
+// 8 bytes in place of the prefix array's neighbours, a pair of which can lie in
+// two lines; the array is half as much to write for the index, and of a dense
+// one more stays in the last-level cache.)
 // ---------------------------------------------------------------------------
 constexpr int kFlatSlots = 512;  // at most kMapCap clusters: half full
 static_assert(kFlatSlots >= 2 * kMapCap, "every insertion finds its slot");

@@ -157,10 +157,12 @@ constexpr int kSmallSingles = 1024;
 constexpr int kSmallWaves = 4096;   // each keeps a trace area
 // From this many pairs on the screen goes first (sw_screen.hip) and the one
 // launch takes what it leaves: two launches more, against the related pairs'
-// sweeps.  us a call without and with, queries of 50-300 bases beside their
-// places: 2,048 pairs 120, 130; 4,000 177, 133; 16,000 527, 294; of 100 bases
-// 59, 69; 78, 77; 219, 102.  Not where slots may be missing: most of a
-// pipeline's pairs are unrelated, and its small calls wait for launches.
+// sweeps.  us a call without -> with, queries of 50-300 bases beside their places
+// (unrelated pairs, all left to the sweep): 2,048 114 -> 124 (111 -> 126); 4,000
+// 163 -> 133 (161 -> 185); 8,000 269 -> 198 (270 -> 301); 16,000 495 -> 294 (496 ->
+// 547); of 100 bases 2,048 59 -> 67 (58 -> 72); 4,000 77 -> 74 (76 -> 96); 16,000
+// 217 -> 115 (209 -> 261).  Not where slots may be missing: most of a pipeline's
+// pairs are unrelated, and its small calls wait for launches.
 constexpr int kSmallScreen = 4000;
 // The one launch's waves take pairs unsorted, 64 lanes of ceil(maxq / 64) rows
 // each, against the general path's binning, readback and 16-lane groups: taken

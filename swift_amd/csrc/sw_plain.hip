@@ -250,7 +250,7 @@ __device__ __forceinline__ int ref_columns(const char *rs, int rlen_max, int g) 
 // The packed sweep: eight pairs a wave, two per 16-lane group, R = ceil(qlen /
 // 16) rows a lane.  Against one wave per pair in 32-bit lanes (64 columns of
 // ramp instead of 16, one cell a lane and instruction instead of two):
-// 100,000 pairs of 100 x 300 3.37 -> 0.93 ms, and 0.40 where the screen takes
+// 100,000 pairs of 100 x 300 3.37 -> 0.93 ms, and 0.32 where the screen takes
 // four in five.  Dynamic LDS: plain_packed_lds().
 constexpr int kPackedTail = kBatchG + 2;  // padding columns after the last
 __host__ __device__ constexpr int plain_packed_stride(int rlen_max) { return rlen_max + kPackedTail; }
@@ -441,9 +441,11 @@ constexpr int kPlainWaves = 4096;
 // 672); 150 x 450, 1,664, 477 against 547 (497; 548); 120 x 1000, 1,528, 793
 // against 1,564 (802; 1,549).
 constexpr int kPlainPackedPairs = 4096;
-// Calls under this many pairs walk a wave a pair, others a lane.  Of a packed
-// call most pairs are the screen's: 40,000 of 100 x 300 275 -> 234 us, of 250 x 400
-// 811 -> 693, 100,000 of 100 x 300 388 -> 354 against the general route's line.
+// Calls under this many pairs walk a wave a pair, others a lane.  The packed
+// route's line against the general one's, us, related pairs, of which most are
+// the screen's (pairs that are all left to the sweep): 40,000 of 100 x 300 242
+// -> 202 (433 -> 396), of 250 x 400 747 -> 628 (1,041 -> 970), 100,000 of 100 x
+// 300 353 -> 322 (898, 905), 130,000 447 -> 404 (1,089, 1,110).
 constexpr int kPackedWalkPairs = 131072;
 constexpr int kGeneralWalkPairs = 16384;
 // longest references of the packed route (four groups' columns in LDS)

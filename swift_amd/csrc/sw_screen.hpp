@@ -38,10 +38,11 @@
 //
 // Cost: a wave's 64 lanes take 64 diagonals at once; their words come out of a
 // ring of shifted ones (two 64-bit shifts and two LDS reads a plane and turn),
-// then 4 instructions each.  Bound by VALU issue: 0.64 us of a SIMD a pair of
-// 150 x 300 (7 turns of 5 words), where the sweep takes 9.
-// Measured without the screen and with it, 1.0M uneven pairs of 143 x 253 on
-// average, a quarter with a gap: 10.1 -> 4.9 ms a call, 0.84 of it the screen.
+// then 4 instructions each.  Bound by issue: 0.64 us of a SIMD a pair of 150 x
+// 300 (7 turns of 5 words), where the sweep takes 9; of 143 x 253 on average 314
+// vector instructions a pair, 57 % of the SIMDs' cycles, beside 278 scalar ones.
+// Measured without the screen and with it, 1.0M such pairs of uneven lengths, a
+// quarter with a gap: 10.1 -> 4.9 ms a call, 0.92 of it the screen.
 // Where three pairs in four are of unrelated sequences (every candidate place
 // of 250,000 reads): 10.9 -> 9.1.
 #pragma once

@@ -257,8 +257,10 @@ hipError_t launch_batch_wide(const BatchArgs &ba, int cu_count, int max_tasks, h
 // kWaveWalkPairs pairs a wave walks each pair, else a lane.
 // A lane's walk waits for one granule after another, whatever the pairs beside
 // it; a class of the pairs the screen leaves is 10,000 to 40,000.  16,384 -> 40,960:
-// 1.0M uneven pairs 4.79 -> 4.66 ms, 100,000 with ambiguity codes 2.18 -> 2.08,
-// 100,000 of 130-150 bases 666 -> 603 us; 131,072 gave no more.
+// 1.0M uneven pairs 4.77 -> 4.64 ms, 100,000 with ambiguity codes 2.18 -> 2.08,
+// 100,000 of 130-150 bases 672 -> 606 us; of unrelated pairs, all of them left,
+// 1.0M 9.74 and 9.75 ms, 400,000 of 50-300 bases 5.75 -> 5.42.  131,072 gave no
+// more.
 constexpr int kWaveWalkPairs = 40960;
 hipError_t launch_walk(const BatchArgs &ba, const int32_t *order, const int32_t *first,
                        const int32_t *count, int max_pairs, uint32_t *moves, int move_words,
