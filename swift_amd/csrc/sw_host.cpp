@@ -84,6 +84,8 @@ struct Workspace {
     DevBuf bins;      // bin_count, bin_cursor (x2 passes)
     DevBuf segs;      // seg_task0 / seg_first / seg_len (x2 passes)
     DevBuf counters;  // int32 counters
+    bool counters_zero = false;
+    bool one_launch = false;  // the last call's form, which leaves the error counter alone
     DevBuf totals;    // int64 total trace words per pass
     // Mapped pinned host block the sizes are gathered into (one stream
     // synchronisation per pass instead of a copy each)
@@ -336,6 +338,8 @@ static int64_t worst_trace_words(int npairs, int maxq, int maxr) {
     return words;
 }
 
+constexpr int kCounters = 256;  // layout: kCntError and the others below
+
 // totals layout (int64): [pass] trace words, then from kTotSteps the sweep
 // steps of each (pass, segment)
 constexpr int kTotSteps = 8;
@@ -354,13 +358,7 @@ static int reserve_common(Workspace &w, int npairs) {
     if ((rc = w.scan_sums.ensure(((size_t)mt / 2048 + 2) * 8))) return rc;
     if ((rc = w.bins.ensure((size_t)4 * kNumBins * 4))) return rc;
     if ((rc = w.segs.ensure((size_t)2 * 3 * (2 * kRBins + 1) * 4))) return rc;
-    if (!w.counters.ptr) {
-        if ((rc = w.counters.ensure(256 * 4))) return rc;
-        SWIFT_HIP_TRY(hipMemset(w.counters.ptr, 0, 256 * 4));
-        // done before the caller's stream, which need not wait for the null
-        // stream, counts in them
-        SWIFT_HIP_TRY(hipStreamSynchronize(nullptr));
-    }
+    if ((rc = w.counters.ensure(kCounters * 4))) return rc;
     if ((rc = w.totals.ensure((size_t)(kTotSteps + 2 * 2 * kRBins) * 8))) return rc;
     if (!w.stage) {
         void *p = nullptr;
@@ -444,11 +442,13 @@ int sw_batch_status_in(Workspace *w) {
 }
 
 int sw_batch_check_in(Workspace *w, hipStream_t st) {
-    int32_t c[16];
-    SWIFT_HIP_TRY(hipMemcpyAsync(c, w->counters.ptr, sizeof(c), hipMemcpyDeviceToHost, st));
+    int32_t error = 0;
+    if (!w->one_launch)
+        SWIFT_HIP_TRY(hipMemcpyAsync(&error, w->counters.as<int32_t>() + kCntError, sizeof(error),
+                                     hipMemcpyDeviceToHost, st));
     SWIFT_HIP_TRY(hipStreamSynchronize(st));
     const int rc = sw_batch_status_in(w);
-    return c[kCntError] ? length_error() : rc;
+    return error ? length_error() : rc;
 }
 
 // A small call as one kernel (sw_small.hip).  *done: 0 when a pair was longer
@@ -561,6 +561,16 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
     const int n = io.npairs;
     const int mt = max_tasks_for(n);
     int32_t *cnt = w.counters.as<int32_t>();
+    // before the first kernels that count, on their stream (a captured call
+    // reads none of what it does not clear itself)
+    if (!w.counters_zero && sync_sizes) {
+        ZeroSpans z{};
+        z.p[0] = cnt;
+        z.n[0] = kCounters;
+        z.nspans = 1;
+        SWIFT_HIP_TRY(launch_zero(z, st));
+        w.counters_zero = true;
+    }
     int64_t *tot = w.totals.as<int64_t>();
     int32_t *bins = w.bins.as<int32_t>();
     int32_t *segs = w.segs.as<int32_t>();
@@ -624,10 +634,13 @@ static int batch_run(Workspace &w, const BatchIO &io, const Scoring &sc, hipStre
         int done = 0;
         if ((rc = batch_run_small(w, io, sc, form16, kc16, h_limit, st, sync_sizes && final_sync,
                                   &done, &screened)) ||
-            done)
+            done) {
+            w.one_launch = true;
             return rc;
+        }
         w.stats = BatchStats{};
     }
+    w.one_launch = false;
 
     // one launch zeroes the results (they start at "score 0": a pair no
     // kernel reaches never walks), the error flag, the flagged count, the

@@ -60,3 +60,28 @@ def test_free_waits_for_the_device(n):
     t = time.perf_counter()
     assert lib().swift_device_free(p) == 0
     assert done.query(), time.perf_counter() - t
+
+
+def test_first_batch_beside_a_capture(hip, orc):
+    """A workspace's first call, on its own stream, while another thread's stream
+    that the null stream waits for is being captured."""
+    import random
+
+    from swift_amd import align as A
+    from test_gpu_sw_lean import check, edge_pairs
+    from test_gpu_sw_status import Path
+    qs, rs = edge_pairs(random.Random(9), 300, 100, 160)
+    b, got = A.PairBatch(qs, rs), []
+    s = C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(s)) == 0
+    p = Path()
+    assert hip.hipStreamBeginCapture(s, THREAD_LOCAL) == 0
+    t = threading.Thread(target=lambda: got.append(p.call("run", b, (2, -1, -10, -1))))
+    t.start()
+    t.join()
+    graph = C.c_void_p()
+    end = hip.hipStreamEndCapture(s, C.byref(graph))
+    p.close()
+    assert got == [0] and end == 0
+    assert hip.hipStreamDestroy(s) == 0
+    check(b.results(), orc.sw_batch(qs, rs, nthreads=8))
