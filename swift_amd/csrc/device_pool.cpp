@@ -2,6 +2,7 @@
 #include <list>
 #include <mutex>
 #include <unordered_map>
+#include <utility>
 
 #include "device_pool.hpp"
 
@@ -48,11 +49,30 @@ bool mapped(const Block &b) {
     return false;
 }
 
-// hipFree's device is the block's own, whichever is current
-void drop(Pool &p, std::list<Block>::iterator it) {
-    p.bytes[it->dev] -= it->size;
-    if (mapped(*it)) (void)hipFree(it->ptr);
-    p.kept.erase(it);
+// Takes the kept blocks that `which` names out of the pool, to be given back
+// without its lock: hipFree waits for the device, and other threads allocate.
+template <class Which> std::list<Block> take(Pool &p, Which which) {
+    std::list<Block> out;
+    for (auto it = p.kept.begin(); it != p.kept.end();) {
+        auto at = it++;
+        if (!which(*at)) continue;
+        p.bytes[at->dev] -= at->size;
+        out.splice(out.end(), p.kept, at);
+    }
+    return out;
+}
+
+// (hipFree's device is the block's own, whichever is current; what it refuses,
+// in a thread that captures a stream, is kept)
+void give_back(Pool &p, std::list<Block> blocks) {
+    for (auto it = blocks.begin(); it != blocks.end();) {
+        auto at = it++;
+        if (!mapped(*at) || hipFree(at->ptr) == hipSuccess) blocks.erase(at);
+        else (void)hipGetLastError();
+    }
+    std::lock_guard<std::mutex> lk(p.mu);
+    for (const Block &b : blocks) p.bytes[b.dev] += b.size;
+    p.kept.splice(p.kept.begin(), blocks);
 }
 
 // Waits for the device as hipFree does, by a hipFree (1.3 us with the
@@ -63,13 +83,6 @@ bool wait_idle() {
     return hipMalloc(&p, 1) == hipSuccess && hipFree(p) == hipSuccess;
 }
 
-void drop_all(Pool &p, int dev) {
-    for (auto it = p.kept.begin(); it != p.kept.end();) {
-        auto at = it++;
-        if (at->dev == dev) drop(p, at);
-    }
-}
-
 }  // namespace
 
 static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
@@ -78,31 +91,29 @@ static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
     if (e != hipSuccess) return e;
     if (bytes > kPoolBlock && (e = hipMalloc(ptr, bytes)) != hipErrorOutOfMemory) return e;
     Pool &p = pool();
-    std::lock_guard<std::mutex> lk(p.mu);
     const size_t size = bytes > kPoolBlock ? bytes : block_size(bytes ? bytes : 1);
-    // the block kept last: the likeliest to be in the caches
-    for (auto it = p.kept.end(); it != p.kept.begin();) {
-        --it;
-        if (it->dev == dev && it->size == size) {
-            if (!mapped(*it)) {
-                auto gone = it++;
-                drop(p, gone);
-                continue;
-            }
-            p.live[it->ptr] = *it;
+    if (bytes <= kPoolBlock) {
+        std::lock_guard<std::mutex> lk(p.mu);
+        // the block kept last: the likeliest to be in the caches
+        for (auto it = p.kept.end(); it != p.kept.begin();) {
+            --it;
+            if (it->dev != dev || it->size != size) continue;
+            const bool use = mapped(*it);
+            if (use) p.live[it->ptr] = *it;
             *ptr = it->ptr;
             p.bytes[dev] -= size;
-            p.kept.erase(it);
-            return hipSuccess;
+            it = p.kept.erase(it);
+            if (use) return hipSuccess;
         }
+        e = hipSuccess;
     }
-    if (bytes <= kPoolBlock) e = hipMalloc(ptr, size);
-    if (e == hipErrorOutOfMemory) {  // give back what this device keeps
+    if (e == hipSuccess) e = hipMalloc(ptr, size);
+    if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        drop_all(p, dev);
-        e = hipMalloc(ptr, size);
+        if (pool_trim() == hipSuccess) e = hipMalloc(ptr, size);
     }
     if (e == hipSuccess && size <= kPoolBlock) {
+        std::lock_guard<std::mutex> lk(p.mu);
         try {
             p.live[*ptr] = Block{*ptr, size, dev, 0, false};
         } catch (...) {  // not entered: pool_free hands it to hipFree
@@ -127,8 +138,10 @@ hipError_t pool_trim() {
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     Pool &p = pool();
-    std::lock_guard<std::mutex> lk(p.mu);
-    drop_all(p, dev);
+    std::unique_lock<std::mutex> lk(p.mu);
+    std::list<Block> out = take(p, [&](const Block &b) { return b.dev == dev; });
+    lk.unlock();
+    give_back(p, std::move(out));
     return hipSuccess;
 }
 
@@ -180,11 +193,11 @@ hipError_t pool_free(void *ptr) {
         lk.unlock();
         return hipFree(ptr);
     }
-    for (auto it = p.kept.begin(); it != p.kept.end();) {
-        auto at = it++;
-        if (at->freed + kPoolAge < p.frees || (at->dev == dev && p.bytes[dev] > kPoolBytes))
-            drop(p, at);
-    }
+    std::list<Block> out = take(p, [&](const Block &k) {
+        return k.freed + kPoolAge < p.frees || (k.dev == dev && p.bytes[dev] > kPoolBytes);
+    });
+    lk.unlock();
+    if (!out.empty()) give_back(p, std::move(out));
     return hipSuccess;
 }
 

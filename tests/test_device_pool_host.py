@@ -4,6 +4,7 @@ mapped and has one owner, whatever is freed twice, elsewhere or too late."""
 import ctypes as C
 import os
 import subprocess
+import threading
 
 import pytest
 
@@ -36,7 +37,7 @@ MEMORY = r"""
 static std::recursive_mutex mu;
 static std::map<char *, size_t> mapped;
 static size_t in_use, limit = ~(size_t)0;
-static int device, last;
+static int device, last, refuse;  // frees to refuse, as in a capture
 static void (*on_sync)();
 static void wait() {
     if (on_sync) { auto f = on_sync; on_sync = nullptr; f(); }
@@ -57,6 +58,10 @@ hipError_t hipMalloc(void **p, size_t n) {
 hipError_t hipFree(void *p) {
     wait();
     std::lock_guard<std::recursive_mutex> lk(mu);
+    if (refuse > 0) {
+        --refuse;
+        return last = hipErrorInvalidValue;
+    }
     auto it = mapped.find((char *)p);
     if (it == mapped.end()) return last = hipErrorInvalidValue;
     in_use -= it->second;
@@ -79,6 +84,7 @@ hipError_t hipMemGetAddressRange(hipDeviceptr_t *base, size_t *size, hipDevicept
 const char *hipGetErrorString(hipError_t) { return ""; }
 extern "C" {
 int t_alloc(void **p, size_t n) { return swift::pool_alloc(p, n); }
+void t_refuse(int n) { refuse = n; }
 int t_free(void *p) { return swift::pool_free(p); }
 int t_device_malloc(void **p, size_t n) { return swift::device_malloc(p, n); }
 int t_trim() { return swift::pool_trim(); }
@@ -207,6 +213,43 @@ def test_pointers_given_to_hip_free(pool):
     e = pool.alloc(100_000)
     assert e != d and pool.mapped(e) >= 100_000
     assert pool.trim() == 0 and pool.mapped(d) == 1000
+
+
+def test_others_allocate_while_blocks_are_given_back(pool):
+    """hipFree waits for the device: the pool's lock is not held meanwhile."""
+    assert pool.free(pool.alloc(1000)) == 0
+    got = []
+
+    def from_another_thread():
+        t = threading.Thread(target=lambda: got.append(pool.alloc(5000)))
+        t.start()
+        t.join(5)
+        got.append(t.is_alive())
+
+    again = SYNC(from_another_thread)
+    pool.on_sync(again)
+    assert pool.trim() == 0
+    assert got[0] is not False and got[-1] is False, got
+
+
+def test_a_refused_free_loses_nothing(pool):
+    """A block that hipFree refuses, in a thread that captures a stream, stays."""
+    a = pool.alloc(1000)
+    assert pool.free(a) == 0
+    pool.refuse(1)
+    assert pool.trim() == 0 and pool.mapped(a) >= 1000
+    assert pool.alloc(1000) == a
+    assert pool.free(a) == 0 and pool.trim() == 0 and pool.mapped(a) == 0
+
+
+def test_the_oldest_go_first(pool):
+    """1 GiB at most is kept: four blocks of 208 MiB, as 200 are rounded up to."""
+    size = 200 << 20
+    blocks = [pool.alloc(size) for _ in range(7)]
+    for b in blocks:
+        assert pool.free(b) == 0
+    kept = [pool.mapped(b) > 0 for b in blocks]
+    assert kept == [False] * 3 + [True] * 4
 
 
 def test_workspaces_ask_the_pool():
