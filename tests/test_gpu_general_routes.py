@@ -78,25 +78,40 @@ def test_wide_form_limits(A, orc):
     check(got, orc.sw_batch(qs, rs, *GENERAL, nthreads=8))
 
 
-def noalloc(qs, rs, ql, rl, sc):
-    from swift_amd._lib import check as ok
-    from swift_amd._lib import lib
-    from swift_amd.device import DeviceBuffer
-    n, cl = len(qs), ql + rl + 2
+class NoAlloc:
+    """The no-allocation call over its own buffers."""
 
-    def fixed(seqs, width):
-        a = np.zeros((n, width + 1), np.uint8)
-        for i, s in enumerate(seqs):
-            a[i, :len(s)] = np.frombuffer(s, np.uint8)
-        return DeviceBuffer.from_array(a)
+    def __init__(self, n, ql, rl, sc):
+        from swift_amd.device import DeviceBuffer
+        self.n, self.ql, self.rl, self.sc, self.cl = n, ql, rl, sc, ql + rl + 2
+        self.q, self.r = DeviceBuffer(n * (ql + 1)), DeviceBuffer(n * (rl + 1))
+        self.out = ([DeviceBuffer(4 * n) for _ in range(4)]
+                    + [DeviceBuffer(self.cl * n) for _ in range(2)])
 
-    q, r = fixed(qs, ql), fixed(rs, rl)
-    b = [DeviceBuffer(4 * n) for _ in range(4)] + [DeviceBuffer(cl * n) for _ in range(2)]
-    ok(lib().swift_align_sequences_noalloc(q.cptr, r.cptr, ql, rl, *(C.c_float(x) for x in sc),
-                                           *(x.cptr for x in b), n, None))
-    ok(lib().swift_device_synchronize())
-    cols = [x.download(t, n) for x, t in zip(b, (np.float32, np.int32, np.int32, np.int32))]
-    return cols + [x.download(np.uint8, cl * n).reshape(n, cl) for x in b[4:]]
+    def load(self, qs, rs):
+        for buf, seqs, width in ((self.q, qs, self.ql), (self.r, rs, self.rl)):
+            a = np.zeros((self.n, width + 1), np.uint8)
+            for i, s in enumerate(seqs):
+                a[i, :len(s)] = np.frombuffer(s, np.uint8)
+            buf.upload(a)
+
+    def run(self, stream=None):
+        from swift_amd._lib import check as ok
+        from swift_amd._lib import lib
+        ok(lib().swift_align_sequences_noalloc(
+            self.q.cptr, self.r.cptr, self.ql, self.rl, *(C.c_float(x) for x in self.sc),
+            *(x.cptr for x in self.out), self.n, stream))
+
+    def check(self, want):
+        from swift_amd._lib import check as ok
+        from swift_amd._lib import lib
+        ok(lib().swift_device_synchronize())
+        for x, w in zip(self.out, want[:4]):
+            assert np.array_equal(x.download(np.int32 if x is not self.out[0] else np.float32,
+                                             self.n), w)
+        for x, w in zip(self.out[4:], want[4:]):
+            rows = x.download(np.uint8, self.cl * self.n).reshape(self.n, self.cl)
+            assert [s.tobytes().split(b"\0")[0] for s in rows] == list(w)
 
 
 # chunks of the 64 MiB array: two of the packed route, three of the general one,
@@ -107,12 +122,42 @@ def noalloc(qs, rs, ql, rl, sc):
 def test_noalloc_chunks(orc, n, ql, rl, sc):
     qs, rs = edge_pairs(random.Random(n), n, ql, rl)
     qs = [q.ljust(ql, b"G")[:ql] for q in qs]
-    s, st, en, al, qc, rc = orc.sw_batch(qs, rs, *sc, nthreads=8)
-    got = noalloc(qs, rs, ql, rl, sc)
-    for a, b in zip(got, (s.astype(np.float32), st, en, al)):
-        assert np.array_equal(a, b)
-    for a, want in zip(got[4:], (qc, rc)):
-        assert [x.tobytes().split(b"\0")[0] for x in a] == list(want)
+    call = NoAlloc(n, ql, rl, sc)
+    call.load(qs, rs)
+    call.run()
+    call.check(orc.sw_batch(qs, rs, *sc, nthreads=8))
+
+
+@pytest.mark.parametrize("n,ql,rl,sc", [(6000, 100, 300, (2, -1, -10, -1)),
+                                        (300, 100, 300, (2, -1, -10, -1)),
+                                        (800, 100, 300, GENERAL)])
+def test_noalloc_replays(orc, n, ql, rl, sc):
+    """Captured once; every replay is over other pairs, with eager calls between."""
+    from swift_amd._lib import lib
+    from swift_amd.device import Stream
+    lib()
+    hip = C.CDLL("libamdhip64.so")
+    sets = []
+    for seed in range(3):
+        qs, rs = edge_pairs(random.Random(seed), n, ql, rl)
+        qs = [q.ljust(ql, b"G")[:ql] for q in qs]
+        sets.append((qs, rs, orc.sw_batch(qs, rs, *sc, nthreads=8)))
+    call, other, st = NoAlloc(n, ql, rl, sc), NoAlloc(n, ql, rl, sc), Stream()
+    graph, run = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(st.cptr, 0) == 0
+    call.run(st.cptr)
+    assert hip.hipStreamEndCapture(st.cptr, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
+    for i in (0, 1, 2, 0):
+        qs, rs, want = sets[i]
+        call.load(qs, rs)
+        assert hip.hipGraphLaunch(run, st.cptr) == 0
+        st.synchronize()
+        call.check(want)
+        other.load(*sets[(i + 1) % 3][:2])
+        other.run()
+        other.check(sets[(i + 1) % 3][2])
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
 
 
 # the first calls whose walks take a lane a pair: a class of the batched path,
