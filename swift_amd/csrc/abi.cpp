@@ -27,11 +27,11 @@ int swift_device_count(int *count) {
     return kOk;
 }
 int swift_device_alloc(void **ptr, size_t bytes) {
-    SWIFT_HIP_TRY(pool_alloc(ptr, bytes));
+    SWIFT_HIP_TRY(pool_alloc(ptr, bytes, false));
     return kOk;
 }
 int swift_device_free(void *ptr) {
-    SWIFT_HIP_TRY(pool_free(ptr));
+    SWIFT_HIP_TRY(pool_free(ptr, true));
     return kOk;
 }
 int swift_device_trim(void) {

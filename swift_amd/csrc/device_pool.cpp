@@ -1,4 +1,5 @@
 // device_pool.cpp -- see device_pool.hpp.
+#include <algorithm>
 #include <list>
 #include <mutex>
 #include <unordered_map>
@@ -16,6 +17,7 @@ struct Block {
     int dev;
     uint64_t freed;  // the pool's count of frees when it was kept
     bool leaving;    // in pool_free, on its way to the kept ones
+    bool idle;       // the device was waited for after its owner let it go
 };
 
 struct Pool {
@@ -23,6 +25,8 @@ struct Pool {
     std::unordered_map<void *, Block> live;  // allocated here, in use
     std::list<Block> kept;                   // oldest first
     std::unordered_map<int, size_t> bytes;   // kept, by device
+    // by device: what was kept by this count of frees was waited for
+    std::unordered_map<int, uint64_t> waited;
     uint64_t frees = 0;
 };
 Pool &pool() {
@@ -77,15 +81,50 @@ void give_back(Pool &p, std::list<Block> blocks) {
 
 // Waits for the device as hipFree does, by a hipFree (1.3 us with the
 // allocation): hipDeviceSynchronize would end every stream capture in progress,
-// also those under which another thread may allocate and free.
-bool wait_idle() {
-    void *p = nullptr;
-    return hipMalloc(&p, 1) == hipSuccess && hipFree(p) == hipSuccess;
+// also those under which another thread may allocate and free.  What was kept
+// before is idle then.
+bool wait_idle(Pool &p, int dev) {
+    uint64_t before;
+    {
+        std::lock_guard<std::mutex> lk(p.mu);
+        before = p.frees;
+    }
+    void *one = nullptr;
+    if (hipMalloc(&one, 1) != hipSuccess || hipFree(one) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lk(p.mu);
+    try {
+        uint64_t &w = p.waited[dev];
+        w = std::max(w, before);
+    } catch (...) {  // no memory for the pool's own tables: nothing is marked
+    }
+    return true;
 }
 
 }  // namespace
 
-static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
+// The kept block of this size let go last (the likeliest to be in the caches),
+// of those known to be idle; *wait: there are only others.
+static void *from_kept(Pool &p, int dev, size_t size, bool *wait) {
+    std::lock_guard<std::mutex> lk(p.mu);
+    *wait = false;
+    for (auto it = p.kept.end(); it != p.kept.begin();) {
+        --it;
+        if (it->dev != dev || it->size != size) continue;
+        const bool there = mapped(*it);
+        if (there && !it->idle && it->freed > p.waited[dev]) {
+            *wait = true;
+            continue;
+        }
+        void *ptr = it->ptr;
+        if (there) p.live[ptr] = *it;
+        p.bytes[dev] -= size;
+        it = p.kept.erase(it);
+        if (there) return ptr;
+    }
+    return nullptr;
+}
+
+static hipError_t alloc_from_pool(void **ptr, size_t bytes, bool may_wait) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
@@ -93,18 +132,14 @@ static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
     Pool &p = pool();
     const size_t size = bytes > kPoolBlock ? bytes : block_size(bytes ? bytes : 1);
     if (bytes <= kPoolBlock) {
-        std::lock_guard<std::mutex> lk(p.mu);
-        // the block kept last: the likeliest to be in the caches
-        for (auto it = p.kept.end(); it != p.kept.begin();) {
-            --it;
-            if (it->dev != dev || it->size != size) continue;
-            const bool use = mapped(*it);
-            if (use) p.live[it->ptr] = *it;
-            *ptr = it->ptr;
-            p.bytes[dev] -= size;
-            it = p.kept.erase(it);
-            if (use) return hipSuccess;
+        bool wait;
+        void *got = from_kept(p, dev, size, &wait);
+        if (!got && wait && may_wait && wait_idle(p, dev)) got = from_kept(p, dev, size, &wait);
+        if (got) {
+            *ptr = got;
+            return hipSuccess;
         }
+        (void)hipGetLastError();
         e = hipSuccess;
     }
     if (e == hipSuccess) e = hipMalloc(ptr, size);
@@ -115,17 +150,17 @@ static hipError_t alloc_from_pool(void **ptr, size_t bytes) {
     if (e == hipSuccess && size <= kPoolBlock) {
         std::lock_guard<std::mutex> lk(p.mu);
         try {
-            p.live[*ptr] = Block{*ptr, size, dev, 0, false};
+            p.live[*ptr] = Block{*ptr, size, dev, 0, false, false};
         } catch (...) {  // not entered: pool_free hands it to hipFree
         }
     }
     return e;
 }
 
-hipError_t pool_alloc(void **ptr, size_t bytes) {
+hipError_t pool_alloc(void **ptr, size_t bytes, bool may_wait) {
     hipError_t e;
     try {
-        e = alloc_from_pool(ptr, bytes);
+        e = alloc_from_pool(ptr, bytes, may_wait);
     } catch (...) {  // no memory for the pool's own tables
         e = hipMalloc(ptr, bytes ? bytes : 1);
     }
@@ -152,7 +187,7 @@ hipError_t device_malloc(void **ptr, size_t bytes) {
     return e;
 }
 
-hipError_t pool_free(void *ptr) {
+hipError_t pool_free(void *ptr, bool wait) {
     if (!ptr) return hipSuccess;
     Pool &p = pool();
     Block b{};
@@ -172,15 +207,16 @@ hipError_t pool_free(void *ptr) {
     }
     if (!b.ptr) return hipFree(ptr);
     int dev = 0;
-    const bool idle = hipGetDevice(&dev) == hipSuccess && dev == b.dev && mapped(b) &&
-                      wait_idle();
-    if (!idle) (void)hipGetLastError();
+    const bool keep = hipGetDevice(&dev) == hipSuccess && dev == b.dev && mapped(b) &&
+                      (!wait || wait_idle(p, dev));
+    if (!keep) (void)hipGetLastError();
     std::unique_lock<std::mutex> lk(p.mu);
     p.live.erase(ptr);
     b.freed = ++p.frees;
     b.leaving = false;
+    b.idle = wait;
     bool kept = false;
-    if (idle) {
+    if (keep) {
         try {
             size_t &held = p.bytes[dev];
             p.kept.push_back(b);

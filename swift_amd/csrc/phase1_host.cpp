@@ -301,7 +301,7 @@ static MapWork &map_work() {
 }
 
 // grows by half again, so batches of varying size settle after a few calls
-// (hipFree synchronises the device)
+// (an allocation may wait for the device)
 int ensure(DevArr &a, size_t bytes) {
     return bytes <= a.bytes ? (int)kOk : a.alloc(bytes + bytes / 2 + 256);
 }

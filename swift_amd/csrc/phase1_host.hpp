@@ -18,12 +18,12 @@ struct DevArr {
     size_t bytes = 0;
     int alloc(size_t b) {
         release();
-        SWIFT_HIP_TRY(pool_alloc(&ptr, b));
+        SWIFT_HIP_TRY(pool_alloc(&ptr, b, true));
         bytes = b;
         return kOk;
     }
     void release() {
-        (void)pool_free(ptr);
+        (void)pool_free(ptr, false);
         ptr = nullptr;
         bytes = 0;
     }

@@ -37,9 +37,10 @@ MEMORY = r"""
 static std::recursive_mutex mu;
 static std::map<char *, size_t> mapped;
 static size_t in_use, limit = ~(size_t)0;
-static int device, last, refuse;  // frees to refuse, as in a capture
+static int waits, device, last, refuse;  // frees to refuse, as in a capture
 static void (*on_sync)();
 static void wait() {
+    ++waits;
     if (on_sync) { auto f = on_sync; on_sync = nullptr; f(); }
 }
 hipError_t hipMalloc(void **p, size_t n) {
@@ -83,9 +84,12 @@ hipError_t hipMemGetAddressRange(hipDeviceptr_t *base, size_t *size, hipDevicept
 }
 const char *hipGetErrorString(hipError_t) { return ""; }
 extern "C" {
-int t_alloc(void **p, size_t n) { return swift::pool_alloc(p, n); }
+int t_alloc(void **p, size_t n) { return swift::pool_alloc(p, n, false); }
+int t_array(void **p, size_t n) { return swift::pool_alloc(p, n, true); }
+int t_release(void *p) { return swift::pool_free(p, false); }
+int t_waits() { return waits; }
 void t_refuse(int n) { refuse = n; }
-int t_free(void *p) { return swift::pool_free(p); }
+int t_free(void *p) { return swift::pool_free(p, true); }
 int t_device_malloc(void **p, size_t n) { return swift::device_malloc(p, n); }
 int t_trim() { return swift::pool_trim(); }
 int t_hip_malloc(void **p, size_t n) { return hipMalloc(p, n); }
@@ -118,9 +122,9 @@ def library(tmp_path_factory):
 class Pool:
     def __init__(self, so):
         self.lib = C.CDLL(str(so))
-        for f in ("alloc", "hip_malloc", "device_malloc"):
+        for f in ("alloc", "array", "hip_malloc", "device_malloc"):
             getattr(self.lib, "t_" + f).argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
-        for f in ("free", "hip_free", "mapped"):
+        for f in ("free", "release", "hip_free", "mapped"):
             getattr(self.lib, "t_" + f).argtypes = [C.c_void_p]
         self.lib.t_limit.argtypes = [C.c_size_t]
         self.lib.t_mapped.restype = C.c_size_t
@@ -250,6 +254,34 @@ def test_the_oldest_go_first(pool):
         assert pool.free(b) == 0
     kept = [pool.mapped(b) > 0 for b in blocks]
     assert kept == [False] * 3 + [True] * 4
+
+
+def test_a_block_let_go_unwaited(pool):
+    """... is nobody's until the device has been waited for: by an allocation that
+    may, once for all that went before, or by a free."""
+    a, b = pool.alloc(1000), pool.alloc(1000)
+    c, d = pool.alloc(9000), pool.alloc(9000)
+    for p in (a, b, c):
+        assert pool.release(p) == 0
+    assert pool.alloc(1000) not in (a, b) and pool.waits() == 0
+    assert pool.alloc(1000, "array") == b and pool.waits() == 1
+    assert pool.alloc(1000, "array") == a and pool.alloc(9000) == c and pool.waits() == 1
+    # one that goes during the wait is not covered by it
+    late = SYNC(lambda: pool.release(d))
+    assert pool.release(a) == 0
+    pool.on_sync(late)
+    assert pool.alloc(1000, "array") == a and pool.waits() == 2
+    assert pool.alloc(9000) != d
+    # a free's wait covers what was let go before
+    assert pool.release(b) == 0 and pool.free(a) == 0 and pool.waits() == 3
+    assert pool.alloc(1000) == a and pool.alloc(1000) == b and pool.alloc(9000) == d
+    # a refused wait: new memory
+    assert pool.release(b) == 0
+    pool.refuse(1)
+    assert pool.alloc(1000, "array") not in (None, b)
+    # a second free of it, and giving it back
+    assert pool.free(b) != 0 and pool.release(b) != 0
+    assert pool.trim() == 0 and pool.mapped(b) == 0
 
 
 def test_workspaces_ask_the_pool():
